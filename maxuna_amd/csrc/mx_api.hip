@@ -804,7 +804,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
             ga.sel_norm = L->weights_norm;
             ga.sel_ids = ids;
             ga.sel_w = w;
-            if (!(kFuseSelect && decode_gate_up_selects(L->gate.dtype, ga))) {
+            if (!(kFuseSelect && decode_gate_up_selects(ga))) {
                 ga.sel_keys = nullptr;
                 for (int r = 0; r < rep(1); r++) MX_TRY(launch_decode_select((int)K, sel, s));
             }

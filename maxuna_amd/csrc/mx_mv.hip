@@ -317,16 +317,14 @@ constexpr int NG_MAX = MX_NG_MAX;
 // fewer activation registers per lane at the cost of idle lanes.
 // Built on the host and passed to the kernels as an argument (so no wave spends
 // scalar instructions on its divisions); lp = log2 P, lrpi = log2 RPI.
-// wide: every row takes the whole wave (P = 64, the tail groups masked), so one
-// row per iteration: rows whose RPI-row batches would not fit the DMA budget.
 template <int DT> struct Geo {
     int G, P, NG, RPI, lp, lrpi;
-    __host__ __device__ explicit Geo(int k, bool full_wave = false, bool wide = false) {
+    __host__ __device__ explicit Geo(int k, bool full_wave = false) {
         G = (k / block_size(DT)) * Q<DT>::GPB;
         int p = G & (-G);
         if (p > 64) p = 64;
         if (G / p > NG_MAX) p = 64;
-        if ((full_wave && G <= 64) || wide) p = 64;
+        if (full_wave && G <= 64) p = 64;
         P = p;
         NG = (G + p - 1) / p;
         RPI = 64 / p;
@@ -392,11 +390,7 @@ __device__ __forceinline__ void reduce_tuples(float (&v)[NB][NM], int P, int sub
 // as the aligned 16-byte chunks covering it, packed back to back.  `pre`
 // issues the activation loads before the first copies, `post` finishes filling
 // `xs`.  sink(row, sums[NM]) runs once per row with the fully reduced sums.
-// EARLY (RING == 1): a batch's weight words are read from LDS into registers
-// first, then the next batch's copy is issued into the same buffer, then the
-// batch is computed from registers -- the copy overlaps the compute without a
-// second buffer.
-template <int DT, int NG, int NIT, int NM, int RING, class XPreF, class XPostF, class Sink, bool EARLY = false>
+template <int DT, int NG, int NIT, int NM, int RING, class XPreF, class XPostF, class Sink>
 __device__ __forceinline__ void stream_rows(const uint8_t *const (&w)[NM], int64_t row_bytes, const Geo<DT> &geo,
                                             typename Q<DT>::X (&xs)[NG], int r_begin, int r_end, uint8_t *ring,
                                             int ni, XPreF &&pre, XPostF &&post, Sink &&sink) {
@@ -451,39 +445,6 @@ __device__ __forceinline__ void stream_rows(const uint8_t *const (&w)[NM], int64
         }
         const int rb32 = (int)row_bytes;
         float acc[NIT][NM];
-        if constexpr (EARLY) {
-            typename Q<DT>::Raw raw[NIT][NM][NG];
-#pragma unroll
-            for (int ib = 0; ib < NIT; ib++) {
-                const int row = min(r0 + rsub + geo.RPI * ib, r_end - 1);
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    const uint8_t *rl = ring + moff[m] + (row - r0) * rb32;
-#pragma unroll
-                    for (int jg = 0; jg < NG; jg++) {
-                        const int g = sub + geo.P * jg;
-                        raw[ib][m][jg] = Q<DT>::load(rl, g < geo.G ? g : 0);
-                    }
-                }
-            }
-            // the buffer's words are in registers: the next batch may overwrite it
-            wait_lgkmcnt0();
-            if (bi + 1 < nbatch) issue(bi + 1);
-#pragma unroll
-            for (int ib = 0; ib < NIT; ib++) {
-                const bool ok = r0 + rsub + geo.RPI * ib < r_end;
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    float a = 0.f;
-#pragma unroll
-                    for (int jg = 0; jg < NG; jg++) {
-                        const int g = sub + geo.P * jg;
-                        if (ok && g < geo.G) a += Q<DT>::dot(raw[ib][m][jg], g, xs[jg]);
-                    }
-                    acc[ib][m] = a;
-                }
-            }
-        } else
 #pragma unroll
         for (int ib = 0; ib < NIT; ib++) {
             const int row = r0 + rsub + geo.RPI * ib;
@@ -518,17 +479,6 @@ __device__ __forceinline__ void stream_rows(const uint8_t *const (&w)[NM], int64
             }
         }
     };
-    if constexpr (EARLY) {
-        static_assert(RING == 1, "EARLY re-issues into the one buffer");
-        pre();
-        if (nbatch > 0) issue(0);
-        post();
-        for (int bi = 0; bi < nbatch; bi++) {
-            wait_vmcnt(0);
-            process(bi);
-        }
-        return;
-    }
     pre();
     for (int bi = 0; bi < RING - 1 && bi < nbatch; bi++) issue(bi);
     post();
@@ -543,16 +493,15 @@ __device__ __forceinline__ void stream_rows(const uint8_t *const (&w)[NM], int64
 // Loads this lane's slices from the group-major staged copy (mx_stage.h):
 // GM_CHUNKS 16-byte loads per group, each wave instruction 1 KB of consecutive bytes.
 template <int DT, int NG>
-__device__ __forceinline__ void load_xs_gm(const uint8_t *gm, int k, const Geo<DT> &geo,
-                                           typename Q<DT>::X (&xs)[NG]) {
+__device__ __forceinline__ void load_xs_gm(const uint8_t *gm, int k, int P, typename Q<DT>::X (&xs)[NG]) {
     static_assert(DT == kQ4_K || DT == kQ5_K, "group-major staging is the 64-value group layout");
     const int G = k / 64;
     const uint4 *c = reinterpret_cast<const uint4 *>(gm);
-    const int sub = (threadIdx.x & 63) & (geo.P - 1);
+    const int sub = (threadIdx.x & 63) & (P - 1);
     auto put = [](uint32_t *d, const uint4 v) { d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w; };
 #pragma unroll
     for (int jg = 0; jg < NG; jg++) {
-        int g = sub + geo.P * jg;
+        int g = sub + P * jg;
         g = g < G ? g : 0;
         typename Q<DT>::X &x = xs[jg];
 #pragma unroll
@@ -569,16 +518,16 @@ __device__ __forceinline__ void load_xs_gm(const uint8_t *gm, int k, const Geo<D
     }
 }
 
-// Loads this lane's slices of a staged activation row (global memory or LDS).
+// Loads this lane's slices of a staged activation row (global memory or LDS);
+// G groups a row, P lanes.
 template <int DT, int NG>
-__device__ __forceinline__ void load_xs(const uint8_t *staged, int k, const Geo<DT> &geo,
-                                        typename Q<DT>::X (&xs)[NG]) {
+__device__ __forceinline__ void load_xs(const uint8_t *staged, int k, int G, int P, typename Q<DT>::X (&xs)[NG]) {
     const XView xv(staged, k);
-    const int sub = (threadIdx.x & 63) & (geo.P - 1);
+    const int sub = (threadIdx.x & 63) & (P - 1);
 #pragma unroll
     for (int jg = 0; jg < NG; jg++) {
-        const int g = sub + geo.P * jg;
-        Q<DT>::load_x(xv, g < geo.G ? g : 0, xs[jg]);
+        const int g = sub + P * jg;
+        Q<DT>::load_x(xv, g < G ? g : 0, xs[jg]);
     }
 }
 
@@ -586,16 +535,6 @@ __device__ __forceinline__ void load_xs(const uint8_t *staged, int k, const Geo<
 #define MX_WAVES 4
 #endif
 // rows per wave and LDS ring depth per kernel (tuned on MI355X for the C1 layer)
-#ifndef MX_RW_GU
-#define MX_RW_GU 1
-#endif
-#ifndef MX_RING_GU
-#define MX_RING_GU 1
-#endif
-#ifndef MX_GU_EARLY
-#define MX_GU_EARLY 0
-#endif
-constexpr bool GU_EARLY = MX_GU_EARLY != 0;
 #ifndef MX_RW_DN
 #define MX_RW_DN 16
 #endif
@@ -623,8 +562,8 @@ constexpr int WAVES_DN = MX_WAVES_DN;  // waves per block of the fused down kern
 #define MX_DN_TPB 4
 #endif
 constexpr int DN_TPB = MX_DN_TPB;  // RW_DN-row tiles per wave of k_decode_down
-constexpr int RW_MV = 16, RW_GU = MX_RW_GU, RW_DN = MX_RW_DN;
-constexpr int RING_MV = 2, RING_GU = MX_RING_GU, RING_DN = MX_RING_DN;
+constexpr int RW_MV = 16, RW_DN = MX_RW_DN;
+constexpr int RING_MV = 2, RING_DN = MX_RING_DN;
 
 // row-iterations per batch: NIT * RPI rows are copied per DMA batch
 template <int NG> struct Batch { static constexpr int NIT = NG == 1 ? MX_NIT1 : MX_NIT2; };
@@ -635,9 +574,8 @@ template <int NG> struct BatchDn { static constexpr int NIT = NG == 1 && DN_FULL
 
 // DMA instructions per batch for NM matrices of row_bytes rows at k
 template <int DT, int NG>
-static int ring_insts(int nm, int k, int64_t row_bytes, int nit = Batch<NG>::NIT, bool full_wave = false,
-                      bool wide = false) {
-    return dma_insts(nm, nit * Geo<DT>(k, full_wave, wide).RPI, row_bytes);
+static int ring_insts(int nm, int k, int64_t row_bytes, int nit = Batch<NG>::NIT, bool full_wave = false) {
+    return dma_insts(nm, nit * Geo<DT>(k, full_wave).RPI, row_bytes);
 }
 __host__ __device__ inline size_t align16(size_t v) { return (v + 15) & ~size_t(15); }
 
@@ -671,7 +609,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_mul_mv_id(MvArgs a, int ni, Geo<
         w, a.row_bytes, geo, xs, r0, min(r0 + RW_MV, a.n_out), ring, ni, [&] { stage_pre(xrow, a.k, xp); },
         [&] {
             stage_post(xrow, a.k, xp, lds);
-            load_xs<DT, NG>(lds, a.k, geo, xs);
+            load_xs<DT, NG>(lds, a.k, geo.G, geo.P, xs);
         },
         [&](int row, const float (&s)[1]) { dst[row] = s[0]; });
 }
@@ -907,21 +845,10 @@ template <int DT> static bool mv_fits_dt(int k) {
     const int ni = dma_insts(1, nit * g.RPI, row_bytes_of<DT>(k));
     return ni <= DMA_MAX_INSTS && align16(xstage_bytes(k)) + (size_t)WAVES * RING_MV * ni * 1024 <= 160 * 1024;
 }
-template <int DT> static bool gu_geo_fits(int hidden, int64_t row_bytes, bool wide) {
-    const Geo<DT> g(hidden, false, wide);
-    if (!(hidden > 0 && hidden % block_size(DT) == 0 && g.NG <= NG_MAX) || row_bytes != row_bytes_of<DT>(hidden))
-        return false;
-    const int nit = g.NG == 1 ? Batch<1>::NIT : Batch<2>::NIT;
-    const int ni = dma_insts(2, nit * g.RPI, row_bytes);
-    return ni <= DMA_MAX_INSTS && (size_t)WAVES * RING_GU * ni * 1024 <= 160 * 1024;
-}
-// the gate/up rows take the wide geometry (hidden 7168: 112 groups, 16 lanes a row
-// and 4 rows an iteration put 32 copy instructions in a gate + up batch)
-template <int DT> static bool gu_wide(int hidden, int64_t row_bytes) {
-    return !gu_geo_fits<DT>(hidden, row_bytes, false) && gu_geo_fits<DT>(hidden, row_bytes, true);
-}
+// gate/up rows: a gate and an up row of at most DMA_MAX_INSTS copies together
 template <int DT> static bool gu_fits_dt(int hidden, int64_t row_bytes) {
-    return gu_geo_fits<DT>(hidden, row_bytes, false) || gu_geo_fits<DT>(hidden, row_bytes, true);
+    return hidden > 0 && hidden % block_size(DT) == 0 && row_bytes == row_bytes_of<DT>(hidden) &&
+           dma_insts(2, 1, row_bytes) <= DMA_MAX_INSTS;
 }
 template <int DT> static bool dn_fits_dt(int ff, int64_t row_bytes) {
     if (!geo_ok<DT>(ff, DN_FULL) || row_bytes != row_bytes_of<DT>(ff)) return false;
@@ -975,23 +902,39 @@ mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s) {
 #ifndef MX_GU_WPE
 #define MX_GU_WPE 5
 #endif
-// waves per SIMD the generic gate/up kernel's registers must allow: MX_GU_WPE
-// for one activation group per lane; each further group holds its three digit
-// planes in registers (Q4_K / Q5_K: 52 VGPRs a group), so more groups get fewer
-// waves (at 5 waves per SIMD two groups spilled 200 bytes per lane to scratch,
-// eight 1.6 KB)
+constexpr int GU_SEL_E = 256;  // experts of the in-block top-k
+static_assert(64 * WAVES == SEL_THREADS, "the in-block top-k needs SEL_THREADS threads");
+// Any row width.  LPR lanes hold one row of NG groups per lane, the tail masked
+// (16, 32 or 64 lanes of one group where they suffice), so a wave pass takes PP
+// row pairs: gate and up rows of a pair side by side in the lanes (LPR < 64), or
+// the pair's two rows one after the other (LPR == 64).  A wave loads its
+// activation slices once and walks nr passes; the next pass's rows are copied
+// into the wave's LDS as soon as the current pass's words are in registers, so
+// the copy overlaps the dot products.
+// The form before it gave a wave one row pair, on the lanes of the largest power
+// of two dividing the group count: rows of 48 groups (hidden 3072) used 16 of 64
+// lanes, and wider rows loaded 26 KB of activations for 7 KB of weights.  Four
+// layers of hidden 3072, ff 1024, top-10 + shared at t = 1: 233 -> 136 us
+// (gate/up launch 35.6 us before); Q8_0 hidden 3072, ff 2048 at t = 9: 235 ->
+// 159 us; Q5_K hidden 5120 at t = 4: 177 -> 150 us.
+// What bounds it: the copies' latency and the VALU work of the dots (about 200
+// instructions per 64 groups of a row, the third digit plane among them).
 template <int DT, int NG> constexpr int gu_wpe() {
-    if (NG <= 1) return MX_GU_WPE;
-    if (DT == kQ8_0) return NG <= 2 ? 5 : NG <= 4 ? 4 : 2;
-    if (DT == kQ6_K) return NG <= 2 ? 4 : NG <= 3 ? 3 : NG <= 4 ? 2 : 1;
-    return NG <= 2 ? 3 : NG <= 4 ? 2 : 1;
+    // waves per SIMD the registers allow without spilling (the three digit planes
+    // of a group are 48 VGPRs for Q4_K / Q5_K, 24 for the others)
+    if (NG == 1) return DT == kQ5_K ? 4 : MX_GU_WPE;
+    if (DT == kQ4_K) return NG == 2 ? 3 : NG == 3 ? 2 : 1;
+    if (DT == kQ5_K) return NG == 2 ? 2 : 1;
+    if (DT == kQ6_K) return NG == 2 ? 3 : NG == 3 ? 2 : 1;
+    return NG == 2 ? 4 : NG == 3 ? 3 : 2;
 }
-template <int DT, int NG, bool GM>
+template <int DT, int NG, int LPR, int AUX>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(gu_wpe<DT, NG>())))
-k_decode_gate_up(DecodeGateUpArgs a, int ni, int slot0, Geo<DT> geo) {
+k_decode_gate_up(DecodeGateUpArgs a, int slot0, int nr, int area) {
+    constexpr int PP = LPR == 64 ? 1 : 32 / LPR;   // row pairs per pass
+    constexpr int NMP = LPR == 64 ? 2 : 1;         // rows a lane contracts per pass
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int slots = a.top_k + (a.sh_gate ? 1 : 0);
-    const int tile = blockIdx.x;
     int slot = slot0 + blockIdx.y, tok = blockIdx.z;
     int pe = -1;  // the pair's expert, from the expert-ordered launch list
     if (a.perm) {  // (all slots launched: slot0 == 0)
@@ -1000,41 +943,113 @@ k_decode_gate_up(DecodeGateUpArgs a, int ni, int slot0, Geo<DT> geo) {
         slot = (v & 0xFFFF) % slots;
         pe = v >> 16;
     }
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (scalar)
-    const int r0 = tile * (WAVES * RW_GU) + wave * RW_GU;
-    if (r0 >= a.ff) return;  // wave-uniform; no block barrier below
-    float *act = a.act + ((int64_t)tok * slots + slot) * a.ff;
-    const uint8_t *gw, *uw;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int sub = lane & (LPR - 1);
+    const int G = a.hidden / block_size(DT) * Q<DT>::GPB;
+    // pass i takes row pairs first + i * step .. + PP - 1: the grid's waves stream
+    // neighbouring rows together
+    const int first = (blockIdx.x * WAVES + wave) * PP, step = (int)gridDim.x * WAVES * PP;
+    typename Q<DT>::X xs[NG];
+    if (first < a.ff) {
+        if constexpr (DT == kQ4_K || DT == kQ5_K)
+            load_xs_gm<DT, NG>(a.xstage_gm + (int64_t)tok * xstage_gm_stride(a.hidden), a.hidden, LPR, xs);
+        else load_xs<DT, NG>(a.xstage + (int64_t)tok * xstage_stride(a.hidden), a.hidden, G, LPR, xs);
+    }
+    if (a.sel_keys && slot < a.top_k) {  // block-uniform: the whole block selects (t == 1)
+        auto &sh = *reinterpret_cast<SelSharedT<GU_SEL_E> *>(lds + WAVES * 2 * area);
+        const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
+        topk_from_keys<GU_SEL_E>(a.sel_keys, a.sel_probs, a.n_expert, a.top_k, a.sel_scale, a.sel_apply,
+                                 a.sel_norm, writer ? a.sel_ids : nullptr, a.sel_w, sh);
+        pe = __builtin_amdgcn_readfirstlane(sh.pick[slot]);
+    }
+    if (first >= a.ff) return;  // wave-uniform; no block barrier below
+    const uint8_t *w[2];
     int64_t rb;
     if (slot < a.top_k) {
         const uint32_t id = pe >= 0 ? (uint32_t)pe : a.ids[tok * a.top_k + slot];
         const int e = id < (uint32_t)a.n_expert ? (int)id : a.n_expert - 1;
-        gw = a.gate + (int64_t)e * a.gu_expert_bytes;
-        uw = a.up + (int64_t)e * a.gu_expert_bytes;
+        w[0] = a.gate + (int64_t)e * a.gu_expert_bytes;
+        w[1] = a.up + (int64_t)e * a.gu_expert_bytes;
         rb = a.gu_row_bytes;
     } else {
-        gw = a.sh_gate;
-        uw = a.sh_up;
+        w[0] = a.sh_gate;
+        w[1] = a.sh_up;
         rb = a.sh_row_bytes;
     }
-    const uint8_t *const w[2] = {gw, uw};
-    typename Q<DT>::X xs[NG];
-    const uint8_t *staged = a.xstage + (int64_t)tok * xstage_stride(a.hidden);
-    uint8_t *ring = lds + wave * (RING_GU * ni * 1024);
-    // GM: the slices come from the group-major copy (a compile-time choice: a
-    // runtime branch between the two loaders measurably delays the loads)
-    auto pre = [&] {
-        if constexpr (GM) load_xs_gm<DT, NG>(a.xstage_gm + (int64_t)tok * xstage_gm_stride(a.hidden), a.hidden, geo, xs);
-        else load_xs<DT, NG>(staged, a.hidden, geo, xs);
+    uint8_t *buf = lds + wave * (2 * area);  // the gate rows' span, then the up rows'
+    // the aligned 16-byte chunks covering pass i's rows of matrix m
+    auto issue = [&](int m, int i) {
+        const int p0 = first + i * step, p1 = min(p0 + PP, a.ff);
+        const uintptr_t S = reinterpret_cast<uintptr_t>(w[m] + (int64_t)p0 * rb);
+        const uintptr_t E = reinterpret_cast<uintptr_t>(w[m] + (int64_t)p1 * rb);
+        const uint8_t *base = reinterpret_cast<const uint8_t *>(S & ~uintptr_t(15));
+        const int nch = (int)((E + 15 - (S & ~uintptr_t(15))) >> 4);
+        for (int q = 0; 64 * q < nch; q++) {
+            const int ci = 64 * q + lane;
+            if (ci < nch) dma16<AUX>(base + (uint32_t)(16 * ci), buf + m * area + 1024 * q);
+        }
+        asm volatile("" ::: "memory");
     };
-    auto sink = [&](int row, const float (&s)[2]) {
-        const float g = s[0];
-        const float sg = g / (1.0f + expf(-g));
-        act[row] = sg * s[1];
-    };
-    auto nopost = [] {};
-    stream_rows<DT, NG, Batch<NG>::NIT, 2, RING_GU, decltype(pre) &, decltype(nopost) &, decltype(sink) &, GU_EARLY>(
-        w, rb, geo, xs, r0, min(r0 + RW_GU, a.ff), ring, ni, pre, nopost, sink);
+    issue(0, 0);
+    issue(1, 0);
+    float keep = 0.f;  // lane i * PP + p: pair p of pass i
+    for (int i = 0; i < nr; i++) {
+        const int p0 = first + i * step;
+        if (p0 >= a.ff) break;  // wave-uniform
+        const bool more = i + 1 < nr && p0 + step < a.ff;
+        wait_vmcnt(0);  // (both matrices' rows of pass i)
+        float v[NMP];
+#pragma unroll
+        for (int m = 0; m < NMP; m++) {
+            const int mat = NMP == 2 ? m : (lane / LPR) & 1, pair = NMP == 2 ? 0 : lane / (2 * LPR);
+            const uint8_t *wm = mat ? w[1] : w[0];
+            const int off = (int)(reinterpret_cast<uintptr_t>(wm + (int64_t)p0 * rb) & 15);
+            const uint8_t *rl = buf + mat * area + off + pair * (int)rb;
+            typename Q<DT>::Raw raw[NG];
+#pragma unroll
+            for (int jg = 0; jg < NG; jg++) {
+                const int g = sub + LPR * jg;
+                raw[jg] = Q<DT>::load(rl, g < G ? g : 0);
+            }
+            wait_lgkmcnt0();  // the words are in registers: their bytes may be overwritten
+            if (more) {
+                issue(NMP == 2 ? m : 0, i + 1);
+                if (NMP == 1) issue(1, i + 1);
+            }
+            v[m] = 0.f;
+#pragma unroll
+            for (int jg = 0; jg < NG; jg++) {
+                const int g = sub + LPR * jg;
+                const float d = Q<DT>::dot(raw[jg], g, xs[jg]);
+                v[m] += g < G ? d : 0.f;
+            }
+        }
+        // the rows' sums over their lanes; a pair's gate sum ends in the lower half of
+        // its lanes, its up sum in the upper half
+        float r;
+        if constexpr (LPR == 64) {
+            const bool hi = (lane & 32) != 0;
+            r = (hi ? v[NMP - 1] : v[0]) + lane_partner<32>(hi ? v[0] : v[NMP - 1]);
+            r += lane_partner<16>(r);
+        } else {
+            r = v[0];
+            if constexpr (LPR == 32) r += lane_partner<16>(r);
+        }
+        r += lane_partner<8>(r);
+        r += lane_partner<4>(r);
+        r += lane_partner<2>(r);
+        r += lane_partner<1>(r);
+#pragma unroll
+        for (int p = 0; p < PP; p++) {
+            constexpr int SPAN = 64 / PP;
+            const float g = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), p * SPAN));
+            const float u = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), p * SPAN + SPAN / 2));
+            const float act = g / (1.0f + expf(-g)) * u;
+            keep = lane == i * PP + p ? act : keep;
+        }
+    }
+    const int row = first + lane / PP * step + lane % PP;
+    if (lane < nr * PP && row < a.ff) a.act[((int64_t)tok * slots + slot) * a.ff + row] = keep;
 }
 
 // Gate/up rows of exactly 64 groups (Q4_K / Q5_K at hidden 4096, 16-byte-aligned
@@ -1061,8 +1076,6 @@ template <int DT> struct Row64 {
     static constexpr int RB = 16 * (DT == kQ4_K ? 144 : 176);  // row bytes (16 super-blocks)
     static constexpr int CH = RB / 16, NI = (CH + 63) / 64;     // 16-byte chunks, copy instructions
 };
-constexpr int GU_SEL_E = 256;  // experts of the in-block top-k
-static_assert(64 * WAVES == SEL_THREADS, "the in-block top-k needs SEL_THREADS threads");
 // TPB: row-pair tiles per workgroup (tiles blockIdx.x, blockIdx.x + gridDim.x, ...
 // of its (slot, token)); WPE: waves per SIMD the registers must allow (the verify
 // form runs at 4: C2 333 -> 324 us; t = 1 at 5); AUX: the weight copies' cache
@@ -1086,7 +1099,7 @@ k_decode_gate_up64(DecodeGateUpArgs a, int slot0, Geo<DT> geo) {
     // the workgroup walks its tiles loading the activation slices and the expert once
     const int rfirst = (blockIdx.x * WAVES + wave) * R;
     typename Q<DT>::X xs[1];
-    if (rfirst < a.ff) load_xs_gm<DT, 1>(a.xstage_gm + (int64_t)tok * xstage_gm_stride(a.hidden), a.hidden, geo, xs);
+    if (rfirst < a.ff) load_xs_gm<DT, 1>(a.xstage_gm + (int64_t)tok * xstage_gm_stride(a.hidden), a.hidden, 64, xs);
     if (a.sel_keys && slot < a.top_k) {  // block-uniform: the whole block selects (t == 1)
         auto &sh = *reinterpret_cast<SelSharedT<GU_SEL_E> *>(lds + WAVES * 2 * RB);
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
@@ -1249,18 +1262,36 @@ mx_status launch_pair_order(const uint32_t *ids, int t, int top_k, int n_expert,
     return MX_OK;
 }
 
-template <int DT, int NG>
-static mx_status launch_gu_ng(const DecodeGateUpArgs &a, int slot0, int nslot, hipStream_t s, bool wide) {
-    const unsigned tiles = (unsigned)((a.ff + WAVES * RW_GU - 1) / (WAVES * RW_GU));
-    const dim3 grid(tiles, (unsigned)nslot, (unsigned)a.t);
-    constexpr bool GM_OK = DT == kQ4_K || DT == kQ5_K;
-    const int ni = ring_insts<DT, NG>(2, a.hidden, a.gu_row_bytes, Batch<NG>::NIT, false, wide);
-    const size_t lds = (size_t)WAVES * RING_GU * ni * 1024;
-    const Geo<DT> geo(a.hidden, false, wide);
-    if (GM_OK && a.xstage_gm)
-        hipLaunchKernelGGL((k_decode_gate_up<DT, NG, GM_OK>), grid, dim3(64 * WAVES), lds, s, a, ni, slot0, geo);
-    else
-        hipLaunchKernelGGL((k_decode_gate_up<DT, NG, false>), grid, dim3(64 * WAVES), lds, s, a, ni, slot0, geo);
+// Waves a gate/up launch aims at, each walking a power of two of passes (so the
+// workgroups share the rows evenly; 9 passes where 8 fit took 167 against 154 us
+// in a Q8_0 layer of 9 tokens).  t = 1: about the resident waves (four groups of
+// 1024 with one activation group per lane, two where the registers allow fewer);
+// from t = 2 on more, the activation loads of a wave amortised over 4-16 passes.
+#ifndef MX_GU_WAVES1
+#define MX_GU_WAVES1 4096
+#endif
+#ifndef MX_GU_WAVES1_WIDE
+#define MX_GU_WAVES1_WIDE 2048
+#endif
+#ifndef MX_GU_WAVES
+#define MX_GU_WAVES 8192
+#endif
+#ifndef MX_GU_NR
+#define MX_GU_NR 16
+#endif
+template <int DT, int NG, int LPR>
+static mx_status launch_gu_rows(const DecodeGateUpArgs &a, int slot0, int nslot, hipStream_t s) {
+    constexpr int PP = LPR == 64 ? 1 : 32 / LPR;
+    const int64_t passes = (a.ff + PP - 1) / PP;  // per (token, slot)
+    const int64_t waves = a.t > 1 ? MX_GU_WAVES : NG == 1 ? MX_GU_WAVES1 : MX_GU_WAVES1_WIDE;
+    int64_t nr = 1;
+    while (2 * nr <= MX_GU_NR && 2 * nr * PP <= 64 && 3 * nr * waves < 2 * passes * nslot * a.t) nr *= 2;
+    const dim3 grid((unsigned)((passes + nr * WAVES - 1) / (nr * WAVES)), (unsigned)nslot, (unsigned)a.t);
+    // a span of PP rows from any 2-byte phase, whole chunks (+ the dword past a Q8_0 block)
+    const int area = (int)((PP * a.gu_row_bytes + 15 + 15 + 4) / 16 * 16);
+    const size_t lds = (size_t)WAVES * 2 * area + (a.sel_keys ? sizeof(SelSharedT<GU_SEL_E>) : 0);
+    if (a.t > 1) hipLaunchKernelGGL((k_decode_gate_up<DT, NG, LPR, 0>), grid, dim3(64 * WAVES), lds, s, a, slot0, (int)nr, area);
+    else hipLaunchKernelGGL((k_decode_gate_up<DT, NG, LPR, DMA_NT>), grid, dim3(64 * WAVES), lds, s, a, slot0, (int)nr, area);
     return MX_OK;
 }
 
@@ -1302,12 +1333,21 @@ static mx_status launch_gu_dt(const DecodeGateUpArgs &a, int slot0, int nslot, h
             return MX_OK;
         }
     }
-    const bool wide = gu_wide<DT>(a.hidden, a.gu_row_bytes);
-    const int ng = ng_variant(Geo<DT>(a.hidden, false, wide).NG);
-#define MX_L(N) return launch_gu_ng<DT, N>(a, slot0, nslot, s, wide)
-    MX_NG_SWITCH(ng, MX_L)
-#undef MX_L
-    return MX_OK;
+    const int G = a.hidden / block_size(DT) * Q<DT>::GPB;
+    if (G <= 16) return launch_gu_rows<DT, 1, 16>(a, slot0, nslot, s);
+    if (G <= 32) return launch_gu_rows<DT, 1, 32>(a, slot0, nslot, s);
+    if (G <= 64) return launch_gu_rows<DT, 1, 64>(a, slot0, nslot, s);
+    // (Q5_K rows of 80 groups: 83% of the lanes' groups filled against 62% at 64
+    // lanes of two; the layer at t = 4 163 -> 151 us; 96 groups of Q8_0: the same)
+    if (G <= 96) return launch_gu_rows<DT, 3, 32>(a, slot0, nslot, s);
+    if (G <= 128) return launch_gu_rows<DT, 2, 64>(a, slot0, nslot, s);
+    if (G <= 192) return launch_gu_rows<DT, 3, 64>(a, slot0, nslot, s);
+    // (gu_fits_dt: no row has more than 320 groups, none of Q5_K more than 192)
+    if constexpr (DT != kQ5_K) {
+        if (G <= 256) return launch_gu_rows<DT, 4, 64>(a, slot0, nslot, s);
+    }
+    if constexpr (DT == kQ6_K) return launch_gu_rows<DT, 5, 64>(a, slot0, nslot, s);
+    return fail(MX_ERR_SHAPE, "decode gate/up: %d activation groups per row", G);
 }
 
 mx_status launch_decode_select(int top_k, const DecodeSelArgs &sel, hipStream_t s) {
@@ -1320,9 +1360,8 @@ mx_status launch_decode_select(int top_k, const DecodeSelArgs &sel, hipStream_t 
     return MX_OK;
 }
 
-bool decode_gate_up_selects(int dtype, const DecodeGateUpArgs &a) {
-    return dtype == kQ4_K && gu64_ok<kQ4_K>(a) && a.t == 1 && a.n_expert <= GU_SEL_E && a.top_k <= SEL_MAX_K &&
-           !a.perm;
+bool decode_gate_up_selects(const DecodeGateUpArgs &a) {
+    return a.t == 1 && a.n_expert <= GU_SEL_E && a.top_k <= SEL_MAX_K && !a.perm;
 }
 
 mx_status launch_decode_gate_up(int dtype, const DecodeGateUpArgs &a, int slot0, int nslot, hipStream_t s) {
@@ -1333,8 +1372,8 @@ mx_status launch_decode_gate_up(int dtype, const DecodeGateUpArgs &a, int slot0,
         return fail(MX_ERR_SHAPE, "decode gate/up: shared expert rows must match the routed rows");
     if (a.perm && (slot0 != 0 || nslot != a.top_k + (a.sh_gate ? 1 : 0)))
         return fail(MX_ERR_SHAPE, "decode gate/up: an expert-ordered launch covers every slot");
-    if (a.sel_keys && (!decode_gate_up_selects(dtype, a) || slot0 != 0))
-        return fail(MX_ERR_SHAPE, "decode gate/up: the in-block top-k needs t == 1 and the 64-group kernel");
+    if (a.sel_keys && (!decode_gate_up_selects(a) || slot0 != 0))
+        return fail(MX_ERR_SHAPE, "decode gate/up: the in-block top-k needs t == 1 and n_expert <= %d", GU_SEL_E);
     switch (dtype) {
     case kQ4_K: MX_TRY(launch_gu_dt<kQ4_K>(a, slot0, nslot, s)); break;
     case kQ5_K: MX_TRY(launch_gu_dt<kQ5_K>(a, slot0, nslot, s)); break;
@@ -1396,7 +1435,7 @@ __global__ void __launch_bounds__(64 * WAVES_DN) __attribute__((amdgpu_waves_per
                                                      [&] { stage_pre(xrow, a.ff, xp); },
                                                      [&] {
                                                          stage_post(xrow, a.ff, xp, lds);
-                                                         load_xs<DT, NG>(lds, a.ff, geo, xs);
+                                                         load_xs<DT, NG>(lds, a.ff, geo.G, geo.P, xs);
                                                      },
                                                      [&](int row, const float (&s)[1]) { part[row] = s[0]; });
 }
@@ -1457,7 +1496,7 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_slots(DecodeD
                                                      [&] { stage_pre_t(xrow, a.ff, xp, lane, 64); },
                                                      [&] {
                                                          stage_post_t(xrow, a.ff, xp, xs_lds, lane, 64);
-                                                         load_xs<DT, NG>(xs_lds, a.ff, geo, xs);
+                                                         load_xs<DT, NG>(xs_lds, a.ff, geo.G, geo.P, xs);
                                                          wait_lgkmcnt0();  // before the ring overwrites it
                                                      },
                                                      [&](int row, const float (&v)[1]) { s_part[slot][row - r0] = v[0]; });
@@ -1543,7 +1582,7 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDow
     issue(0, b0);
     typename Q<DT>::X xs[DQ6_NG];
     stage_post_t(xrow, a.ff, xp, b1, lane, 64);
-    load_xs<DT, DQ6_NG>(b1, a.ff, geo, xs);
+    load_xs<DT, DQ6_NG>(b1, a.ff, geo.G, geo.P, xs);
     wait_lgkmcnt0();
     if (NB > 1) issue(1, b1);
     // this lane's field offsets inside a row (Q<kQ6_K>::load's, hoisted)
@@ -1670,7 +1709,7 @@ __global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArg
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     typename Q<DT>::X xs[DQ6_NG];
-    load_xs<DT, DQ6_NG>(stg, a.ff, geo, xs);
+    load_xs<DT, DQ6_NG>(stg, a.ff, geo.G, geo.P, xs);
     uint32_t oa[DQ6_NG], ohq[DQ6_NG], osc[DQ6_NG], od[DQ6_NG], sh[DQ6_NG];
 #pragma unroll
     for (int jg = 0; jg < DQ6_NG; jg++) {
