@@ -56,6 +56,9 @@ __host__ __device__ inline int dma_insts(int nm, int rows, int64_t row_bytes) {
     const int64_t chunks = (rows * row_bytes + 15) / 16 + 1;  // per matrix
     return nm * (int)((chunks + 63) / 64);
 }
+#ifndef MX_BATCH_BYTES
+#define MX_BATCH_BYTES 5120
+#endif
 constexpr int DMA_MAX_INSTS = 15;  // per batch (vmcnt budget of the waits, up to 2 batches ahead)
 
 __device__ __forceinline__ void lds_words(const int8_t *p, uint32_t *dst, int n16) {
@@ -304,191 +307,144 @@ template <> struct Q<kQ8_0> {
     }
 };
 
-// ---- lane geometry ----------------------------------------------------------------------
-// P = largest power of two <= 64 dividing the row's group count G; if that leaves
-// more than NG_MAX groups per lane, P = 64 with the tail groups masked.
-#ifndef MX_NG_MAX
-#define MX_NG_MAX 8
-#endif
-constexpr int NG_MAX = MX_NG_MAX;
+// the sum over aligned groups of P lanes (a power of two >= 8), in every lane
+template <int P> __device__ __forceinline__ float lane_sum(float v) {
+    if constexpr (P >= 64) v += lane_partner<32>(v);
+    if constexpr (P >= 32) v += lane_partner<16>(v);
+    if constexpr (P >= 16) v += lane_partner<8>(v);
+    v += lane_partner<4>(v);
+    v += lane_partner<2>(v);
+    v += lane_partner<1>(v);
+    return v;
+}
 
-// full_wave: a row whose groups fit one wave takes the whole wave (one group per
-// lane, lanes past G idle) instead of P = the largest power of two dividing G;
-// fewer activation registers per lane at the cost of idle lanes.
-// Built on the host and passed to the kernels as an argument (so no wave spends
-// scalar instructions on its divisions); lp = log2 P, lrpi = log2 RPI.
-template <int DT> struct Geo {
-    int G, P, NG, RPI, lp, lrpi;
-    __host__ __device__ explicit Geo(int k, bool full_wave = false) {
-        G = (k / block_size(DT)) * Q<DT>::GPB;
-        int p = G & (-G);
-        if (p > 64) p = 64;
-        if (G / p > NG_MAX) p = 64;
-        if (full_wave && G <= 64) p = 64;
-        P = p;
-        NG = (G + p - 1) / p;
-        RPI = 64 / p;
-        lp = 0;
-        while ((1 << lp) < P) lp++;
-        lrpi = 6 - lp;
+// ---- rows of one matrix through a wave ---------------------------------------------------
+// (mul_mv_id, and the down rows of the fused decode layer at any width.)
+// LPR lanes hold a row, NG groups each (the tail masked): a pass takes RPI =
+// 64 / LPR rows.  A wave walks `nb` batches of `br` rows (br / RPI passes): batch
+// b's rows start at r0 + b * stride, rows from `end` on do not exist.  A batch's
+// bytes are copied as the aligned 16-byte chunks that cover them; with two
+// buffers batch b + 1 is in flight while batch b is contracted, with one (rows
+// so wide that two do not fit) the next copy follows the contraction.  (The form
+// before copied one batch, waited for it, contracted it, and so on: Q8_0 hidden
+// 3072, ff 2048 layers at t = 9 159 -> 116 us, four of them at t = 1 158 -> 111;
+// four Q6_K-down layers of hidden 3072, ff 1024 at t = 1 136 -> 119.)  Bound by
+// the copies' latency at t = 1 (a wave lives for two to four batches) and by the
+// VALU work of the dots from a few tokens on.
+template <int DT, int LPR, int AUX> struct RowWalk {
+    static constexpr int RPI = 64 / LPR;
+    const uint8_t *w;  // row 0
+    int64_t rb;
+    int r0, stride, end, br, nb;
+    uint8_t *buf0, *buf1;  // buf1 == buf0: one buffer
+    __device__ __forceinline__ const uint8_t *src(int b) const { return w + (int64_t)(r0 + b * stride) * rb; }
+    __device__ __forceinline__ int rows(int b) const { return min(br, end - (r0 + b * stride)); }
+    // 16-byte chunks of batch b (at least one row)
+    __device__ __forceinline__ int chunks(int b) const {
+        const uintptr_t S = reinterpret_cast<uintptr_t>(src(b));
+        return (int)((S + (uintptr_t)(rows(b) * rb) + 15 - (S & ~uintptr_t(15))) >> 4);
+    }
+    __device__ __forceinline__ void issue(int b) const {
+        const uint8_t *base = reinterpret_cast<const uint8_t *>(reinterpret_cast<uintptr_t>(src(b)) & ~uintptr_t(15));
+        uint8_t *dst = (b & 1) ? buf1 : buf0;
+        const int nch = chunks(b), lane = threadIdx.x & 63;
+        for (int q = 0; 64 * q < nch; q++) {
+            const int ci = 64 * q + lane;
+            if (ci < nch) dma16<AUX>(base + (uint32_t)(16 * ci), dst + 1024 * q);
+        }
+        asm volatile("" ::: "memory");
+    }
+    // issues the first copies (nb >= 1)
+    __device__ __forceinline__ void start() const {
+        issue(0);
+        if (buf1 != buf0 && nb > 1) issue(1);
+    }
+    // sink(row, sum) once per row, on the row's first lane
+    template <int NG, class Sink>
+    __device__ __forceinline__ void run(const typename Q<DT>::X (&xs)[NG], int G, Sink &&sink) const {
+        const int lane = threadIdx.x & 63, sub = lane & (LPR - 1), rsub = lane / LPR;
+        const bool two = buf1 != buf0;
+        for (int b = 0; b < nb; b++) {
+            // batch b has landed once only batch b + 1's copies are outstanding
+            wait_vmcnt(two && b + 1 < nb ? (chunks(b + 1) + 63) >> 6 : 0);
+            const uint8_t *buf = ((b & 1) ? buf1 : buf0) + (reinterpret_cast<uintptr_t>(src(b)) & 15);
+            const int n = rows(b);
+            for (int p = 0; p < n; p += RPI) {
+                const uint8_t *rl = buf + (p + rsub) * (int)rb;
+                float v = 0.f;
+                if constexpr (NG > (DT == kQ6_K ? 2 : 3)) {
+                    // (a branch per group: every group's words at once would spill)
+#pragma unroll
+                    for (int jg = 0; jg < NG; jg++) {
+                        const int g = sub + LPR * jg;
+                        if (g < G) v += Q<DT>::dot(Q<DT>::load(rl, g), g, xs[jg]);
+                    }
+                } else {
+                    typename Q<DT>::Raw raw[NG];
+#pragma unroll
+                    for (int jg = 0; jg < NG; jg++) {
+                        const int g = sub + LPR * jg;
+                        raw[jg] = Q<DT>::load(rl, g < G ? g : 0);
+                    }
+#pragma unroll
+                    for (int jg = 0; jg < NG; jg++) {
+                        const int g = sub + LPR * jg;
+                        const float d = Q<DT>::dot(raw[jg], g, xs[jg]);
+                        v += g < G ? d : 0.f;
+                    }
+                }
+                v = lane_sum<LPR>(v);
+                if (sub == 0 && p + rsub < n) sink(r0 + b * stride + p + rsub, v);
+            }
+            wait_lgkmcnt0();  // every read of the buffer returned before it is overwritten
+            const int nx = b + (two ? 2 : 1);
+            if (nx < nb) issue(nx);
+        }
     }
 };
 
-// the compiled groups-per-lane variants: the smallest >= NG
-__host__ __device__ constexpr int ng_variant(int ng) {
-    return ng <= 1 ? 1 : ng <= 2 ? 2 : ng <= 3 ? 3 : ng <= 4 ? 4 : ng <= 6 ? 6 : 8;
-}
-
-// Reduces NB tuples of NM floats over the P lanes of each row group.  While the
-// tuple count allows, each exchange step (lane_partner) halves the tuples a lane
-// keeps (the lane whose offset bit is set keeps the upper half), so NB tuples cost
-// NB - 1 + log2(P / NB) shuffles per float instead of NB * log2(P).  On return
-// v[0] holds the full sums of tuple `*which` on the lanes that must publish it
-// (`*leader`).  Requires P >= NB; otherwise every tuple is reduced in place and
-// published by the lane with sub == 0.
-template <int NM, int NB>
-__device__ __forceinline__ void reduce_tuples(float (&v)[NB][NM], int P, int sub, int &which, bool &leader) {
-    which = 0;
-    if (P < NB) {
-#pragma unroll
-        for (int ib = 0; ib < NB; ib++)
-#pragma unroll
-            for (int m = 0; m < NM; m++) v[ib][m] = warp_sum_width(v[ib][m], P);
-        leader = sub == 0;
-        return;
+// The compiled (LPR, NG) pairs: the fewest padded groups, and of equal ones the
+// most rows per pass (fewer exchange steps per row).  Q4_K / Q5_K groups are 64
+// weights and 52 registers of activation digits, the others 32 weights and up to
+// 36, so the former stop at two groups a lane where they can.
+// f(integral_constant LPR, integral_constant NG)
+template <int DT, class F> static auto with_lanes(int G, F &&f) {
+#define MX_LN(L, N) return f(std::integral_constant<int, L>{}, std::integral_constant<int, N>{})
+    if constexpr (DT == kQ4_K || DT == kQ5_K) {
+        if (G <= 8) MX_LN(8, 1);
+        if (G <= 16) MX_LN(16, 1);
+        if (G <= 32) MX_LN(16, 2);
+        if (G <= 64) MX_LN(32, 2);
+    } else {
+        if (G <= 16) MX_LN(16, 1);
+        if (G <= 24) MX_LN(8, 3);
+        // (16 lanes of two: 113 registers, one workgroup of 11 slot waves per CU
+        // instead of two; hidden 3072, ff 1024 at t = 4 80 -> 76 us)
+        if (G <= 32) MX_LN(32, 1);
+        if (G <= 48) MX_LN(16, 3);
+        if (G <= 64) MX_LN(32, 2);
+        if (G <= 96) MX_LN(32, 3);
     }
-    int o = P >> 1;
-#pragma unroll
-    for (int half = NB / 2; half >= 1; half /= 2) {
-        const bool up = (sub & o) != 0;
-        at_offset(o, [&](auto c) {
-#pragma unroll
-            for (int i = 0; i < half; i++) {
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    const float keep = up ? v[half + i][m] : v[i][m];
-                    const float send = up ? v[i][m] : v[half + i][m];
-                    v[i][m] = keep + lane_partner<decltype(c)::value>(send);
-                }
-            }
-        });
-        if (up) which += half;
-        o >>= 1;
-    }
-    for_offsets_down(o, [&](auto c) {
-#pragma unroll
-        for (int m = 0; m < NM; m++) v[0][m] += lane_partner<decltype(c)::value>(v[0][m]);
-    });
-    leader = (sub & (P / NB - 1)) == 0;
+    if (G <= 128) MX_LN(64, 2);
+    if (G <= 256) MX_LN(64, 4);
+    MX_LN(64, 8);
+#undef MX_LN
 }
-
-// Streams the rows [r_begin, r_end) of NM matrices that share one activation
-// through this wave, NIT row-iterations (NIT * RPI rows) per batch, through the
-// wave's LDS ring `ring` of RING buffers of ni KB (ni = dma_insts(NM, rows per
-// batch, row_bytes)): batches i+1 .. i+RING-1 are in flight while batch i is
-// computed.  A batch's image in a buffer is the NM matrices' row spans, each
-// as the aligned 16-byte chunks covering it, packed back to back.  `pre`
-// issues the activation loads before the first copies, `post` finishes filling
-// `xs`.  sink(row, sums[NM]) runs once per row with the fully reduced sums.
-template <int DT, int NG, int NIT, int NM, int RING, class XPreF, class XPostF, class Sink>
-__device__ __forceinline__ void stream_rows(const uint8_t *const (&w)[NM], int64_t row_bytes, const Geo<DT> &geo,
-                                            typename Q<DT>::X (&xs)[NG], int r_begin, int r_end, uint8_t *ring,
-                                            int ni, XPreF &&pre, XPostF &&post, Sink &&sink) {
-    static_assert((NIT & (NIT - 1)) == 0, "NIT: a power of two");
-    constexpr int LNIT = NIT == 1 ? 0 : NIT == 2 ? 1 : NIT == 4 ? 2 : NIT == 8 ? 3 : 4;
-    const int lane = threadIdx.x & 63;
-    const int sub = lane & (geo.P - 1);
-    const int rsub = lane >> geo.lp;
-    const int step = NIT << geo.lrpi;
-    const int bstride = ni * 1024;
-    const int nbatch = (r_end - r_begin + step - 1) >> (LNIT + geo.lrpi);
-    // the chunk range [base_m, base_m + 16 * nch_m) of matrix m's span for the batch at r0
-    auto span = [&](int m, int r0, uintptr_t &base, int &nch) {
-        const int r1 = min(r0 + step, r_end);
-        const uintptr_t S = reinterpret_cast<uintptr_t>(w[m] + (int64_t)r0 * row_bytes);
-        const uintptr_t E = reinterpret_cast<uintptr_t>(w[m] + (int64_t)r1 * row_bytes);
-        base = S & ~uintptr_t(15);
-        nch = (int)((E + 15 - base) >> 4);
-    };
-    auto issue = [&](int bi) {
-        const int r0 = r_begin + bi * step;
-        uintptr_t base[NM];
-        int nch[NM];
-#pragma unroll
-        for (int m = 0; m < NM; m++) span(m, r0, base[m], nch[m]);
-        uint8_t *dst = ring + (bi % RING) * bstride;
-        const int per = ni / NM;  // instructions per matrix span
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-            const uint8_t *b = reinterpret_cast<const uint8_t *>(base[m]);
-            for (int q = 0; q < per; q++) {
-                const int ci = min(64 * q + lane, nch[m] - 1);  // spare lanes re-copy the last chunk
-                dma16(b + (uint32_t)(16 * ci), dst + 1024 * (m * per + q));
-            }
-        }
-    };
-    auto process = [&](int bi) {
-        const int r0 = r_begin + bi * step;
-        // LDS offset of each matrix's row r0 in the batch's buffer (wave-uniform);
-        // row r0 + i sits i * row_bytes after it
-        int moff[NM];
-        {
-            uintptr_t base0, base1 = 0;
-            int n0, n1 = 0;
-            span(0, r0, base0, n0);
-            moff[0] = (bi % RING) * bstride + (int)(reinterpret_cast<uintptr_t>(w[0] + (int64_t)r0 * row_bytes) - base0);
-            if (NM > 1) {
-                span(1, r0, base1, n1);
-                moff[NM - 1] = (bi % RING) * bstride + 1024 * (ni / NM) +
-                               (int)(reinterpret_cast<uintptr_t>(w[NM - 1] + (int64_t)r0 * row_bytes) - base1);
-            }
-        }
-        const int rb32 = (int)row_bytes;
-        float acc[NIT][NM];
-#pragma unroll
-        for (int ib = 0; ib < NIT; ib++) {
-            const int row = r0 + rsub + geo.RPI * ib;
-            const bool ok = row < r_end;
-#pragma unroll
-            for (int m = 0; m < NM; m++) {
-                float a = 0.f;
-                if (ok) {
-                    const uint8_t *rl = ring + moff[m] + (row - r0) * rb32;
-#pragma unroll
-                    for (int jg = 0; jg < NG; jg++) {
-                        const int g = sub + geo.P * jg;
-                        if (g < geo.G) a += Q<DT>::dot(Q<DT>::load(rl, g), g, xs[jg]);
-                    }
-                }
-                acc[ib][m] = a;
-            }
-        }
-        int which;
-        bool leader;
-        reduce_tuples<NM, NIT>(acc, geo.P, sub, which, leader);
-        if (leader) {
-            if (geo.P < NIT) {
-#pragma unroll
-                for (int ib = 0; ib < NIT; ib++) {
-                    const int row = r0 + rsub + geo.RPI * ib;
-                    if (row < r_end) sink(row, acc[ib]);
-                }
-            } else {
-                const int row = r0 + rsub + geo.RPI * which;
-                if (row < r_end) sink(row, acc[0]);
-            }
-        }
-    };
-    pre();
-    for (int bi = 0; bi < RING - 1 && bi < nbatch; bi++) issue(bi);
-    post();
-    for (int bi = 0; bi < nbatch; bi++) {
-        if (bi + RING - 1 < nbatch) issue(bi + RING - 1);
-        // batch bi has landed once at most the copies of the later batches are outstanding
-        wait_vmcnt(ni * min(RING - 1, nbatch - 1 - bi));
-        process(bi);
-    }
+constexpr int G_MAX = 512;  // groups of the widest compiled row
+template <int DT> __host__ __device__ constexpr int groups(int k) { return k / block_size(DT) * Q<DT>::GPB; }
+// waves per SIMD the registers of NG activation groups allow without spilling
+template <int DT, int NG> constexpr int rows_wpe() {
+    if (DT == kQ4_K || DT == kQ5_K) return NG == 1 ? 4 : NG == 2 ? 3 : 1;
+    return NG == 1 ? 4 : NG <= 3 ? 3 : NG == 4 ? 2 : 1;
 }
+// rows per batch: passes of rpi rows up to about 5 KB, a power of two of them
+static int batch_rows(int rpi, int64_t row_bytes, int most) {
+    int br = rpi;
+    while (2 * br <= most && 2 * br * row_bytes <= MX_BATCH_BYTES) br *= 2;
+    return br;
+}
+// LDS of a batch: whole chunks from any 2-byte phase, and the dword past a Q8_0 block
+static int batch_area(int br, int64_t row_bytes) { return (int)((br * row_bytes + 15 + 15 + 4) / 16 * 16); }
 
 // Loads this lane's slices from the group-major staged copy (mx_stage.h):
 // GM_CHUNKS 16-byte loads per group, each wave instruction 1 KB of consecutive bytes.
@@ -534,56 +490,38 @@ __device__ __forceinline__ void load_xs(const uint8_t *staged, int k, int G, int
 #ifndef MX_WAVES
 #define MX_WAVES 4
 #endif
-// rows per wave and LDS ring depth per kernel (tuned on MI355X for the C1 layer)
-#ifndef MX_RW_DN
-#define MX_RW_DN 16
-#endif
-#ifndef MX_RING_DN
-#define MX_RING_DN 1
-#endif
-#ifndef MX_NIT1
-#define MX_NIT1 1
-#endif
-#ifndef MX_NIT2
-#define MX_NIT2 1
-#endif
 #ifndef MX_WAVES_DN
 #define MX_WAVES_DN 4
 #endif
-#ifndef MX_DN_FULL
-#define MX_DN_FULL 0
-#endif
-#ifndef MX_NIT_DN
-#define MX_NIT_DN 1
-#endif
 constexpr int WAVES = MX_WAVES;
 constexpr int WAVES_DN = MX_WAVES_DN;  // waves per block of the fused down kernel
-#ifndef MX_DN_TPB
-#define MX_DN_TPB 4
-#endif
-constexpr int DN_TPB = MX_DN_TPB;  // RW_DN-row tiles per wave of k_decode_down
-constexpr int RW_MV = 16, RW_DN = MX_RW_DN;
-constexpr int RING_MV = 2, RING_DN = MX_RING_DN;
-
-// row-iterations per batch: NIT * RPI rows are copied per DMA batch
-template <int NG> struct Batch { static constexpr int NIT = NG == 1 ? MX_NIT1 : MX_NIT2; };
-
-// the down kernel's row layout (Geo full_wave) and row-iterations per batch
-constexpr bool DN_FULL = MX_DN_FULL != 0;
-template <int NG> struct BatchDn { static constexpr int NIT = NG == 1 && DN_FULL ? MX_NIT_DN : Batch<NG>::NIT; };
-
-// DMA instructions per batch for NM matrices of row_bytes rows at k
-template <int DT, int NG>
-static int ring_insts(int nm, int k, int64_t row_bytes, int nit = Batch<NG>::NIT, bool full_wave = false) {
-    return dma_insts(nm, nit * Geo<DT>(k, full_wave).RPI, row_bytes);
-}
+constexpr int RW_DN = 16;  // most rows of a slot-per-wave down tile
 __host__ __device__ inline size_t align16(size_t v) { return (v + 15) & ~size_t(15); }
 
+// the staging loads have returned: ordinary loads are not counted across LDS
+// copies, so they are waited for before the first copy is issued
+template <int NP> __device__ __forceinline__ void stage_landed(XPreT<NP> &xp) {
+    wait_vmcnt(0);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) asm volatile("" : "+v"(xp.v[i][j]));
+}
+// a block barrier after this wave's LDS writes that does not wait for the weight
+// copies in flight (__syncthreads would)
+__device__ __forceinline__ void lds_barrier() {
+    wait_lgkmcnt0();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // ---- mul_mv_id -----------------------------------------------------------------------
-// grid (row tiles, t * top_k); one (token, slot) pair per block, its activation
-// row staged into LDS by the whole block, then one LDS ring per wave.
-template <int DT, int NG>
-__global__ void __launch_bounds__(64 * WAVES) k_mul_mv_id(MvArgs a, int ni, Geo<DT> geo) {
+// grid (workgroups, t * top_k); one (token, slot) pair per block, its activation
+// row staged into LDS by the whole block.  Each wave walks nb batches of br rows,
+// strided by the grid's waves so that the grid streams neighbouring rows together.
+template <int DT, int NG, int LPR>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(rows_wpe<DT, NG>())))
+k_mul_mv_id(MvArgs a, int br, int nb, int area, int two) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int pair = blockIdx.y;  // token * top_k + slot
     const int tok = pair / a.top_k, slot = pair % a.top_k;
@@ -593,54 +531,46 @@ __global__ void __launch_bounds__(64 * WAVES) k_mul_mv_id(MvArgs a, int ni, Geo<
         e = id < (uint32_t)a.n_expert ? (int)id : a.n_expert - 1;
     }
     const float *xrow = a.x + ((int64_t)tok * a.x_per_row + (a.x_per_row == 1 ? 0 : slot)) * a.k;
-    const uint8_t *const w[1] = {a.w + (int64_t)e * a.expert_bytes};
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (scalar)
-    const int r0 = blockIdx.x * (WAVES * RW_MV) + wave * RW_MV;
-    typename Q<DT>::X xs[NG];
+    const int NW = (int)gridDim.x * WAVES, r0 = (blockIdx.x * WAVES + wave) * br;
+    uint8_t *ring = lds + align16(xstage_bytes(a.k)) + wave * ((two ? 2 : 1) * area);
+    RowWalk<DT, LPR, 0> rw{a.w + (int64_t)e * a.expert_bytes, a.row_bytes, r0, NW * br, a.n_out, br, 0, ring,
+                           ring + (two ? area : 0)};
+    rw.nb = r0 < a.n_out ? min(nb, (a.n_out - r0 + NW * br - 1) / (NW * br)) : 0;
     XPre xp;
-    uint8_t *ring = lds + align16(xstage_bytes(a.k)) + wave * (RING_MV * ni * 1024);
-    if (r0 >= a.n_out) {  // wave-uniform: take part in the staging, then leave
-        stage_pre(xrow, a.k, xp);
-        stage_post(xrow, a.k, xp, lds);
-        return;
-    }
+    stage_pre(xrow, a.k, xp);
+    stage_landed(xp);
+    if (rw.nb > 0) rw.start();
+    stage_post_t(xrow, a.k, xp, lds, (int)threadIdx.x, (int)blockDim.x);
+    lds_barrier();
+    if (rw.nb == 0) return;  // wave-uniform; no block barrier below
+    typename Q<DT>::X xs[NG];
+    load_xs<DT, NG>(lds, a.k, groups<DT>(a.k), LPR, xs);
     float *dst = a.dst + (int64_t)pair * a.n_out;
-    stream_rows<DT, NG, Batch<NG>::NIT, 1, RING_MV>(
-        w, a.row_bytes, geo, xs, r0, min(r0 + RW_MV, a.n_out), ring, ni, [&] { stage_pre(xrow, a.k, xp); },
-        [&] {
-            stage_post(xrow, a.k, xp, lds);
-            load_xs<DT, NG>(lds, a.k, geo.G, geo.P, xs);
-        },
-        [&](int row, const float (&s)[1]) { dst[row] = s[0]; });
+    rw.run(xs, groups<DT>(a.k), [&](int row, float v) { dst[row] = v; });
 }
 
-#define MX_NG_SWITCH(ng, MACRO) \
-    switch (ng) {               \
-    case 1: MACRO(1); break;    \
-    case 2: MACRO(2); break;    \
-    case 3: MACRO(3); break;    \
-    case 4: MACRO(4); break;    \
-    case 6: MACRO(6); break;    \
-    default: MACRO(8); break;   \
-    }
-
-template <int DT, int NG>
-static mx_status launch_mv_ng(const MvArgs &a, dim3 grid, hipStream_t s) {
-    const int ni = ring_insts<DT, NG>(1, a.k, a.row_bytes);
-    if (ni > DMA_MAX_INSTS) return fail(MX_ERR_SHAPE, "mul_mv_id: rows of %lld bytes are too long", (long long)a.row_bytes);
-    const size_t lds = align16(xstage_bytes(a.k)) + (size_t)WAVES * RING_MV * ni * 1024;
-    if (lds > 160 * 1024) return fail(MX_ERR_SHAPE, "mul_mv_id: k = %d needs %zu bytes of LDS", a.k, lds);
-    hipLaunchKernelGGL((k_mul_mv_id<DT, NG>), grid, dim3(64 * WAVES), lds, s, a, ni, Geo<DT>(a.k));
-    return MX_OK;
-}
-
-template <int DT>
-static mx_status launch_mv_dt(const MvArgs &a, dim3 grid, hipStream_t s) {
-    const int ng = ng_variant(Geo<DT>(a.k).NG);
-#define MX_L(N) return launch_mv_ng<DT, N>(a, grid, s)
-    MX_NG_SWITCH(ng, MX_L)
-#undef MX_L
-    return MX_OK;
+// waves a launch aims at (8 per CU), at least two batches each
+#ifndef MX_MV_WAVES
+#define MX_MV_WAVES 4096
+#endif
+template <int DT> static mx_status launch_mv_dt(const MvArgs &a, hipStream_t s) {
+    return with_lanes<DT>(groups<DT>(a.k), [&](auto lpr, auto ng) -> mx_status {
+        constexpr int LPR = decltype(lpr)::value, NG = decltype(ng)::value;
+        const int br = batch_rows(64 / LPR, a.row_bytes, 16), area = batch_area(br, a.row_bytes);
+        const int64_t pairs = (int64_t)a.t * a.top_k, batches = (a.n_out + br - 1) / br;
+        int64_t nb = batches * pairs / MX_MV_WAVES;
+        nb = nb < 2 ? 2 : nb;
+        const unsigned gx = (unsigned)((batches + nb * WAVES - 1) / (nb * WAVES));
+        // (the waves' batches interleave over the launched grid: round nb up to cover it)
+        nb = (batches + (int64_t)gx * WAVES - 1) / ((int64_t)gx * WAVES);
+        const size_t stg = align16(xstage_bytes(a.k));
+        const int two = stg + (size_t)WAVES * 2 * area <= 160 * 1024;
+        const size_t lds = stg + (size_t)WAVES * (two ? 2 : 1) * area;
+        hipLaunchKernelGGL((k_mul_mv_id<DT, NG, LPR>), dim3(gx, (unsigned)pairs), dim3(64 * WAVES), lds, s, a, br,
+                           (int)nb, area, two);
+        return MX_OK;
+    });
 }
 
 // ---- compile-time Q6_K mat-vec (plain mul_mv and mul_mv_id, e.g. the lm_head) ----------
@@ -653,7 +583,7 @@ static mx_status launch_mv_dt(const MvArgs &a, dim3 grid, hipStream_t s) {
 // MVQ6_RPW rows of one (token, slot) pair in batches through two LDS buffers of
 // its own (batch b + 1 in flight while b is contracted); the workgroup stages the
 // pair's activation row once.  Same per-row arithmetic and 32-lane sum as
-// k_mul_mv_id (Q<kQ6_K>::dot, reduce_tuples).  The rows per wave (nb batches) are
+// k_mul_mv_id (Q<kQ6_K>::dot, lane_sum).  The rows per wave (nb batches) are
 // chosen at launch so that the grid is one round of resident workgroups: with a
 // fixed 16 rows the lm_head's 1568 workgroups ran as 2.04 rounds of 768, the last
 // round almost empty.
@@ -744,7 +674,6 @@ __global__ void __launch_bounds__(64 * WAVES) k_mv_q6(MvArgs a, int nb) {
     auto batch = [&](int bi, uint8_t *buf) {
         wait_vmcnt(NI);  // batch bi has landed (bi + 1 is in flight)
         const uint8_t *rl = buf + rsub * RB;
-        float acc[1][1];
         // the batch's fields into registers, then the copy of batch bi + 2 into the
         // same buffer, then the dots: the copy is in flight while they run (175
         // VGPRs, 2 waves/SIMD; forced to 3 it spills and takes 64 us instead of 54)
@@ -763,12 +692,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_mv_q6(MvArgs a, int nb) {
         float v = 0.f;
 #pragma unroll
         for (int jg = 0; jg < NG; jg++) v += Q<DT>::dot(r[jg], sub + P * jg, xs[jg]);
-        acc[0][0] = v;
-        int which;
-        bool leader;
-        reduce_tuples<1, 1>(acc, P, sub, which, leader);
+        v = lane_sum<P>(v);
         const int b = gw + bi * NW;
-        if (leader && b < nbt) dst[b * RPI + rsub] = acc[0][0];
+        if (sub == 0 && b < nbt) dst[b * RPI + rsub] = v;
     };
 #pragma unroll 1
     for (int bi = 0; bi < nb; bi += 2) {
@@ -835,15 +761,10 @@ static mx_status launch_mv_q6(const MvArgs &a, int ng, int p, hipStream_t s) {
 // Each kernel holds NG <= NG_MAX activation groups per lane, copies a batch of rows
 // with at most DMA_MAX_INSTS wave instructions per matrix set, and needs its LDS.
 template <int DT> static int64_t row_bytes_of(int k) { return (int64_t)(k / block_size(DT)) * type_size(DT); }
-template <int DT> static bool geo_ok(int k, bool full_wave = false) {
-    return k > 0 && k % block_size(DT) == 0 && Geo<DT>(k, full_wave).NG <= NG_MAX;
-}
 template <int DT> static bool mv_fits_dt(int k) {
-    if (!geo_ok<DT>(k)) return false;
-    const Geo<DT> g(k);
-    const int nit = g.NG == 1 ? Batch<1>::NIT : Batch<2>::NIT;
-    const int ni = dma_insts(1, nit * g.RPI, row_bytes_of<DT>(k));
-    return ni <= DMA_MAX_INSTS && align16(xstage_bytes(k)) + (size_t)WAVES * RING_MV * ni * 1024 <= 160 * 1024;
+    if (k <= 0 || k % block_size(DT) || groups<DT>(k) > G_MAX) return false;
+    return dma_insts(1, 1, row_bytes_of<DT>(k)) <= DMA_MAX_INSTS &&
+           align16(xstage_bytes(k)) + (size_t)WAVES * batch_area(1, row_bytes_of<DT>(k)) <= 160 * 1024;
 }
 // gate/up rows: a gate and an up row of at most DMA_MAX_INSTS copies together
 template <int DT> static bool gu_fits_dt(int hidden, int64_t row_bytes) {
@@ -851,11 +772,7 @@ template <int DT> static bool gu_fits_dt(int hidden, int64_t row_bytes) {
            dma_insts(2, 1, row_bytes) <= DMA_MAX_INSTS;
 }
 template <int DT> static bool dn_fits_dt(int ff, int64_t row_bytes) {
-    if (!geo_ok<DT>(ff, DN_FULL) || row_bytes != row_bytes_of<DT>(ff)) return false;
-    const Geo<DT> g(ff, DN_FULL);
-    const int nit = g.NG == 1 ? BatchDn<1>::NIT : BatchDn<2>::NIT;
-    const int ni = dma_insts(1, nit * g.RPI, row_bytes);
-    return ni <= DMA_MAX_INSTS && align16(xstage_bytes(ff)) + (size_t)WAVES_DN * RING_DN * ni * 1024 <= 160 * 1024;
+    return mv_fits_dt<DT>(ff) && row_bytes == row_bytes_of<DT>(ff);
 }
 #define MX_DT_SWITCH(dtype, EXPR)                       \
     switch (dtype) {                                    \
@@ -871,8 +788,7 @@ bool decode_down_fits(int dtype, int ff, int64_t row_bytes) { MX_DT_SWITCH(dtype
 #undef MX_DT_SWITCH
 
 mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.n_out + WAVES * RW_MV - 1) / (WAVES * RW_MV)), (unsigned)(a.t * a.top_k));
-    if (grid.y == 0 || grid.x == 0) return MX_OK;
+    if (a.n_out == 0 || (int64_t)a.t * a.top_k == 0) return MX_OK;
     if (!mv_ring_fits(dtype, a.k)) {  // any other row width: the f32 mat-vec
         const MvfArgs f{a.w, a.expert_bytes, a.row_bytes, a.n_expert, a.n_out, a.k, a.x, a.x_per_row,
                         a.ids, a.t, a.top_k, a.dst, a.top_k, 0};
@@ -881,10 +797,10 @@ mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s) {
     int ng = 0, p = 0;
     if (dtype == kQ6_K && MX_MV_Q6 && mv_q6_pick(a, ng, p)) return launch_mv_q6(a, ng, p, s);
     switch (dtype) {
-    case kQ4_K: MX_TRY(launch_mv_dt<kQ4_K>(a, grid, s)); break;
-    case kQ5_K: MX_TRY(launch_mv_dt<kQ5_K>(a, grid, s)); break;
-    case kQ6_K: MX_TRY(launch_mv_dt<kQ6_K>(a, grid, s)); break;
-    default: MX_TRY(launch_mv_dt<kQ8_0>(a, grid, s)); break;
+    case kQ4_K: MX_TRY(launch_mv_dt<kQ4_K>(a, s)); break;
+    case kQ5_K: MX_TRY(launch_mv_dt<kQ5_K>(a, s)); break;
+    case kQ6_K: MX_TRY(launch_mv_dt<kQ6_K>(a, s)); break;
+    default: MX_TRY(launch_mv_dt<kQ8_0>(a, s)); break;
     }
     MX_LAUNCH("k_mul_mv_id");
     return MX_OK;
@@ -1082,7 +998,7 @@ template <int DT> struct Row64 {
 // policy (DMA_NT at t = 1).
 template <int DT, int R, int TPB, int WPE, int AUX>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_decode_gate_up64(DecodeGateUpArgs a, int slot0, Geo<DT> geo) {
+k_decode_gate_up64(DecodeGateUpArgs a, int slot0) {
     constexpr int RB = Row64<DT>::RB, CH = Row64<DT>::CH, NI = Row64<DT>::NI;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int slots = a.top_k + (a.sh_gate ? 1 : 0);
@@ -1304,7 +1220,7 @@ static bool gu64_ok(const DecodeGateUpArgs &a) {
         return false;
     } else {
         auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-        return GU64_R > 0 && Geo<DT>(a.hidden).G == 64 && a.gu_row_bytes == Row64<DT>::RB &&
+        return GU64_R > 0 && groups<DT>(a.hidden) == 64 && a.gu_row_bytes == Row64<DT>::RB &&
                a.gu_expert_bytes % 16 == 0 && al(a.gate) && al(a.up) && a.xstage_gm &&
                (!a.sh_gate || (al(a.sh_gate) && al(a.sh_up)));
     }
@@ -1313,7 +1229,10 @@ static bool gu64_ok(const DecodeGateUpArgs &a) {
 template <int DT>
 static mx_status launch_gu_dt(const DecodeGateUpArgs &a, int slot0, int nslot, hipStream_t s) {
     if constexpr (DT == kQ4_K) {  // (gu64_ok holds for Q4_K only)
-        if (gu64_ok<DT>(a)) {
+        // (at 2-4 tokens its 8 tiles a workgroup leave too few workgroups: C1-shaped
+        // layer at t = 2 79 us against 70 us of the kernel for any width, 3: 102 / 98,
+        // 4: 116 / 114, 6: 155 / 159; t = 1: 37 / 39)
+        if (gu64_ok<DT>(a) && (a.t == 1 || a.t >= 5)) {
             const unsigned tiles = (unsigned)((a.ff + WAVES * GU64_R - 1) / (WAVES * GU64_R));
             // verify blocks (t > 1): GU64_TPB tiles per workgroup, the activation
             // slices and per-wave setup amortised over more rows (C2: 8 tiles
@@ -1325,11 +1244,10 @@ static mx_status launch_gu_dt(const DecodeGateUpArgs &a, int slot0, int nslot, h
             const size_t lds = (size_t)WAVES * 2 * Row64<DT>::RB + (a.sel_keys ? sizeof(SelSharedT<GU_SEL_E>) : 0);
             constexpr int R = GU64_R > 0 ? GU64_R : 1;
             if (verify)
-                hipLaunchKernelGGL((k_decode_gate_up64<DT, R, GU64_TPB, 4, 0>), grid, dim3(64 * WAVES), lds, s, a, slot0,
-                                   Geo<DT>(a.hidden));
+                hipLaunchKernelGGL((k_decode_gate_up64<DT, R, GU64_TPB, 4, 0>), grid, dim3(64 * WAVES), lds, s, a, slot0);
             else
                 hipLaunchKernelGGL((k_decode_gate_up64<DT, R, GU64_TPB1, MX_GU_WPE, DMA_NT>), grid, dim3(64 * WAVES), lds,
-                                   s, a, slot0, Geo<DT>(a.hidden));
+                                   s, a, slot0);
             return MX_OK;
         }
     }
@@ -1385,18 +1303,15 @@ mx_status launch_decode_gate_up(int dtype, const DecodeGateUpArgs &a, int slot0,
 }
 
 // ---- fused decode: down (one slot per block), then the combine kernel ---------------------
-// grid (hidden / (WAVES_DN * rpw), slots, t), rpw = RW_DN * DN_TPB rows per wave (C2:
-// 4 tiles per wave 362 -> 334 us, the act row staged once per workgroup for 4x the
-// rows; 2 and 8 measured 343).  Each block writes its slot's down rows to part[tok, slot, :]; the
-// combine kernel that follows on the stream (the kernel boundary orders the two)
-// forms out[c] = residual[c] + ( sum_k w[k] * part[k][c] + shared[c] )
+// grid (hidden / (WAVES_DN * rpw), slots, t), rpw rows per wave.  Each block
+// stages its slot's act row and writes its slot's down rows to part[tok, slot, :];
+// the combine kernel that follows on the stream (the kernel boundary orders the
+// two) forms out[c] = residual[c] + ( sum_k w[k] * part[k][c] + shared[c] )
 // (combine.metal:70-97, moe.rs:73-78, model.rs:351).  The shared expert is
 // part's last slot when it has the routed quant types, else a.shared_out.
-#ifndef MX_DN_WPE
-#define MX_DN_WPE 1
-#endif
-template <int DT, int NG>
-__global__ void __launch_bounds__(64 * WAVES_DN) __attribute__((amdgpu_waves_per_eu(MX_DN_WPE))) k_decode_down(DecodeDownArgs a, int ni, int rpw, Geo<DT> geo) {
+template <int DT, int NG, int LPR>
+__global__ void __launch_bounds__(64 * WAVES_DN) __attribute__((amdgpu_waves_per_eu(rows_wpe<DT, NG>())))
+k_decode_down(DecodeDownArgs a, int rpw, int br, int area, int two) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int slots = a.top_k + (a.sh_down ? 1 : 0);
     const int tile = blockIdx.x;  // grid (row tiles, slots, t)
@@ -1410,96 +1325,77 @@ __global__ void __launch_bounds__(64 * WAVES_DN) __attribute__((amdgpu_waves_per
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform (scalar)
     const int r0 = (tile * WAVES_DN + wave) * rpw;  // rpw rows per wave, the act row staged once
     const float *xrow = a.act + ((int64_t)tok * slots + slot) * a.ff;
-    uint8_t *ring = lds + align16(xstage_bytes(a.ff)) + wave * (RING_DN * ni * 1024);
-    XPre xp;
-    if (r0 >= a.hidden) {  // wave-uniform; every wave takes part in the staging barrier
-        stage_pre(xrow, a.ff, xp);
-        stage_post(xrow, a.ff, xp, lds);
-        return;
-    }
-    const uint8_t *wp;
-    int64_t rb;
+    uint8_t *ring = lds + align16(xstage_bytes(a.ff)) + wave * ((two ? 2 : 1) * area);
+    RowWalk<DT, LPR, 0> rw{nullptr, a.d_row_bytes, r0, br, min(r0 + rpw, a.hidden), br, 0, ring,
+                           ring + (two ? area : 0)};
     if (slot < a.top_k) {
         const uint32_t id = pe >= 0 ? (uint32_t)pe : a.ids[tok * a.top_k + slot];
         const int e = id < (uint32_t)a.n_expert ? (int)id : a.n_expert - 1;
-        wp = a.down + (int64_t)e * a.d_expert_bytes;
-        rb = a.d_row_bytes;
+        rw.w = a.down + (int64_t)e * a.d_expert_bytes;
     } else {
-        wp = a.sh_down;
-        rb = a.sh_row_bytes;
+        rw.w = a.sh_down;
+        rw.rb = a.sh_row_bytes;
     }
-    const uint8_t *const w[1] = {wp};
+    rw.nb = r0 < a.hidden ? (rw.end - r0 + br - 1) / br : 0;
+    XPre xp;
+    stage_pre(xrow, a.ff, xp);
+    stage_landed(xp);
+    if (rw.nb > 0) rw.start();
+    stage_post_t(xrow, a.ff, xp, lds, (int)threadIdx.x, (int)blockDim.x);
+    lds_barrier();
+    if (rw.nb == 0) return;  // wave-uniform; no block barrier below
     typename Q<DT>::X xs[NG];
+    load_xs<DT, NG>(lds, a.ff, groups<DT>(a.ff), LPR, xs);
     float *part = a.part + ((int64_t)tok * slots + slot) * a.hidden;
-    stream_rows<DT, NG, BatchDn<NG>::NIT, 1, RING_DN>(w, rb, geo, xs, r0, min(r0 + rpw, a.hidden), ring, ni,
-                                                     [&] { stage_pre(xrow, a.ff, xp); },
-                                                     [&] {
-                                                         stage_post(xrow, a.ff, xp, lds);
-                                                         load_xs<DT, NG>(lds, a.ff, geo.G, geo.P, xs);
-                                                     },
-                                                     [&](int row, const float (&s)[1]) { part[row] = s[0]; });
+    rw.run(xs, groups<DT>(a.ff), [&](int row, float v) { part[row] = v; });
 }
 
 // ---- fused decode down, one workgroup per (token, row tile) holding every slot ---------
-// grid (hidden / RW_DN, t), 64 * slots threads: wave s stages slot s's act row into
-// its own LDS area and streams the slot's RW_DN down rows; the partial rows meet in
-// LDS and threads 0 .. RW_DN - 1 combine them in slot order, with the arithmetic of
+// grid (hidden / rows, t), 64 * slots threads: wave s stages slot s's act row into
+// its own LDS area and streams the slot's `rows` down rows; the partial rows meet in
+// LDS and threads 0 .. rows - 1 combine them in slot order, with the arithmetic of
 // k_decode_down's combine (combine.metal:70-97).  No partial rows in global
 // memory, no arrival counters, no cross-block tail.
-#ifndef MX_DN_SLOTS
-#define MX_DN_SLOTS 1
-#endif
+// above this, more and smaller blocks (k_decode_down) keep the CUs fuller (Q5_K /
+// Q6_K hidden 5120 at t = 4: layer 151 -> 136 us; Q6_K / Q4_K hidden 6144, ff 2816
+// at t = 3: 183 -> 139; hidden 4096 at t = 3: the same)
 #ifndef MX_DN_SLOTS_MAX_T
-#define MX_DN_SLOTS_MAX_T 4  // above this, more and smaller blocks (k_decode_down) keep the CUs fuller
+#define MX_DN_SLOTS_MAX_T 2
 #endif
 constexpr int DN_SLOTS_MAX = 12;  // 3 waves per SIMD: 168 VGPRs
-// row-iterations per DMA batch (NG > 1): 2 -> 8-row batches of Q6_K at ff = 1536
-#ifndef MX_NIT_DNS
-#define MX_NIT_DNS 2
-#endif
-template <int NG> struct BatchDnSlots { static constexpr int NIT = NG == 1 ? BatchDn<1>::NIT : MX_NIT_DNS; };
-// LDS per slot (wave): the staged act row, then the wave's ring in the same bytes
-static_assert(RING_DN == 1, "k_decode_down_slots overlays its ring on the staged row: one batch in flight");
-__host__ __device__ inline size_t dn_slot_area(int ff, int ni) {
-    const size_t xs = align16(xstage_bytes(ff)), ring = (size_t)ni * 1024;
-    return xs > ring ? xs : ring;
-}
 constexpr int XPRE_W = 4;  // act quarters per lane held in registers before the weight copies
-template <int DT, int NG>
-__global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_slots(DecodeDownArgs a, int ni, Geo<DT> geo) {
+template <int DT, int NG, int LPR, int AUX>
+__global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_slots(DecodeDownArgs a, int rows, int br, int area,
+                                                                         int area1) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ float s_part[DN_SLOTS_MAX][RW_DN];
     const int slots = a.top_k + (a.sh_down ? 1 : 0);
     const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int tok = blockIdx.y;
-    const int r0 = blockIdx.x * RW_DN, r1 = min(r0 + RW_DN, a.hidden);
-    // the slot's staged row is read into registers before the first weight copy,
-    // so the ring reuses its LDS (dn_slot_area)
-    uint8_t *xs_lds = lds + (size_t)slot * dn_slot_area(a.ff, ni);
-    uint8_t *ring = xs_lds;
+    const int r0 = blockIdx.x * rows, r1 = min(r0 + rows, a.hidden);
+    // the staged row is built in the second buffer while the first batch's copy
+    // runs, and read into registers before that buffer's first copy
+    uint8_t *b0 = lds + (size_t)slot * (area + area1), *b1 = b0 + area;
     const float *xrow = a.act + ((int64_t)tok * slots + slot) * a.ff;
-    XPreT<XPRE_W> xp;
-    const uint8_t *wp;
-    int64_t rb;
+    RowWalk<DT, LPR, AUX> rw{nullptr, a.d_row_bytes, r0, br, r1, br, (r1 - r0 + br - 1) / br, b0, b1};
     if (slot < a.top_k) {
         const uint32_t id = a.ids[tok * a.top_k + slot];
         const int e = id < (uint32_t)a.n_expert ? (int)id : a.n_expert - 1;
-        wp = a.down + (int64_t)e * a.d_expert_bytes;
-        rb = a.d_row_bytes;
+        rw.w = a.down + (int64_t)e * a.d_expert_bytes;
     } else {
-        wp = a.sh_down;
-        rb = a.sh_row_bytes;
+        rw.w = a.sh_down;
+        rw.rb = a.sh_row_bytes;
     }
-    const uint8_t *const w[1] = {wp};
+    XPreT<XPRE_W> xp;
+    stage_pre_t(xrow, a.ff, xp, lane, 64);
+    stage_landed(xp);
+    rw.issue(0);
+    stage_post_t(xrow, a.ff, xp, b1, lane, 64);
     typename Q<DT>::X xs[NG];
-    stream_rows<DT, NG, BatchDnSlots<NG>::NIT, 1, RING_DN>(w, rb, geo, xs, r0, r1, ring, ni,
-                                                     [&] { stage_pre_t(xrow, a.ff, xp, lane, 64); },
-                                                     [&] {
-                                                         stage_post_t(xrow, a.ff, xp, xs_lds, lane, 64);
-                                                         load_xs<DT, NG>(xs_lds, a.ff, geo.G, geo.P, xs);
-                                                         wait_lgkmcnt0();  // before the ring overwrites it
-                                                     },
-                                                     [&](int row, const float (&v)[1]) { s_part[slot][row - r0] = v[0]; });
+    load_xs<DT, NG>(b1, a.ff, groups<DT>(a.ff), LPR, xs);
+    wait_lgkmcnt0();  // before the second buffer's copy overwrites the staged row
+    if (rw.nb > 1) rw.issue(1);
+    rw.run(xs, groups<DT>(a.ff), [&](int row, float v) { s_part[slot][row - r0] = v; });
     __syncthreads();
     const int r = threadIdx.x;
     if (r >= r1 - r0) return;
@@ -1534,7 +1430,7 @@ constexpr int DQ6_FF = 1536, DQ6_RB = 1260, DQ6_P = 16, DQ6_NG = 3, DQ6_RPI = 64
 constexpr int DQ6R_BROWS = 4, DQ6R_CH = DQ6R_BROWS * DQ6_RB / 16, DQ6R_NI = (DQ6R_CH + 63) / 64;
 static_assert(DQ6R_BROWS == DQ6_RPI, "one row per lane group per batch");
 template <int AUX>  // cache policy of the weight copies (DMA_NT at t = 1)
-__global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDownArgs a, Geo<kQ6_K> geo) {
+__global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDownArgs a) {
     constexpr int DT = kQ6_K, NB = RW_DN / DQ6R_BROWS;
     // two separate LDS objects, so the compiler can tell a copy into one buffer
     // from the reads of the other
@@ -1582,7 +1478,7 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDow
     issue(0, b0);
     typename Q<DT>::X xs[DQ6_NG];
     stage_post_t(xrow, a.ff, xp, b1, lane, 64);
-    load_xs<DT, DQ6_NG>(b1, a.ff, geo.G, geo.P, xs);
+    load_xs<DT, DQ6_NG>(b1, a.ff, DQ6_P * DQ6_NG, DQ6_P, xs);
     wait_lgkmcnt0();
     if (NB > 1) issue(1, b1);
     // this lane's field offsets inside a row (Q<kQ6_K>::load's, hoisted)
@@ -1602,26 +1498,20 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDow
         uint8_t *const buf = (bi & 1) ? b1 : b0;
         wait_vmcnt(bi + 1 < NB ? DQ6R_NI : 0);  // batch bi has landed (bi + 1 may be in flight)
         const uint8_t *rl = buf + rsub * DQ6_RB;
-        float acc[1][1];
-        {
-            float v = 0.f;
+        float v = 0.f;
 #pragma unroll
-            for (int jg = 0; jg < DQ6_NG; jg++) {
-                typename Q<DT>::Raw r;
-                Q<DT>::ld3(rl + oa[jg], r.a);
-                Q<DT>::ld3(rl + oa[jg] + 32, r.b);
-                Q<DT>::ld3(rl + ohq[jg], r.hq);
-                Q<DT>::ld3(rl + osc[jg], r.sc);
-                r.d = ld_u16(rl + od[jg]);
-                r.sh = sh[jg];
-                v += Q<DT>::dot(r, sub + DQ6_P * jg, xs[jg]);
-            }
-            acc[0][0] = v;
+        for (int jg = 0; jg < DQ6_NG; jg++) {
+            typename Q<DT>::Raw r;
+            Q<DT>::ld3(rl + oa[jg], r.a);
+            Q<DT>::ld3(rl + oa[jg] + 32, r.b);
+            Q<DT>::ld3(rl + ohq[jg], r.hq);
+            Q<DT>::ld3(rl + osc[jg], r.sc);
+            r.d = ld_u16(rl + od[jg]);
+            r.sh = sh[jg];
+            v += Q<DT>::dot(r, sub + DQ6_P * jg, xs[jg]);
         }
-        int which;
-        bool leader;
-        reduce_tuples<1, 1>(acc, DQ6_P, sub, which, leader);
-        if (leader) s_part[slot][bi * DQ6R_BROWS + rsub] = acc[0][0];
+        v = lane_sum<DQ6_P>(v);
+        if (sub == 0) s_part[slot][bi * DQ6R_BROWS + rsub] = v;
         if (bi + 2 < NB) {
             wait_lgkmcnt0();  // every read of the buffer returned before it is overwritten
             issue(bi + 2, buf);
@@ -1652,7 +1542,7 @@ constexpr int DQ6V_RPW = 64;
 #ifndef MX_DN_Q6V
 #define MX_DN_Q6V 1
 #endif
-__global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArgs a, Geo<kQ6_K> geo) {
+__global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArgs a) {
     constexpr int DT = kQ6_K, NB = DQ6V_RPW / DQ6R_BROWS;
     __shared__ __attribute__((aligned(16))) uint8_t ring0[WAVES_DN][DQ6R_NI * 1024];
     __shared__ __attribute__((aligned(16))) uint8_t ring1[WAVES_DN][DQ6R_NI * 1024];
@@ -1709,7 +1599,7 @@ __global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArg
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     typename Q<DT>::X xs[DQ6_NG];
-    load_xs<DT, DQ6_NG>(stg, a.ff, geo.G, geo.P, xs);
+    load_xs<DT, DQ6_NG>(stg, a.ff, DQ6_P * DQ6_NG, DQ6_P, xs);
     uint32_t oa[DQ6_NG], ohq[DQ6_NG], osc[DQ6_NG], od[DQ6_NG], sh[DQ6_NG];
 #pragma unroll
     for (int jg = 0; jg < DQ6_NG; jg++) {
@@ -1725,7 +1615,6 @@ __global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArg
     auto batch = [&](int bi, uint8_t *buf) {
         wait_vmcnt(DQ6R_NI);  // batch bi has landed (the next copy is in flight)
         const uint8_t *rl = buf + rsub * DQ6_RB;
-        float acc[1][1];
         float v = 0.f;
 #pragma unroll
         for (int jg = 0; jg < DQ6_NG; jg++) {
@@ -1738,11 +1627,8 @@ __global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArg
             r.sh = sh[jg];
             v += Q<DT>::dot(r, sub + DQ6_P * jg, xs[jg]);
         }
-        acc[0][0] = v;
-        int which;
-        bool leader;
-        reduce_tuples<1, 1>(acc, DQ6_P, sub, which, leader);
-        if (leader) part[bi * DQ6R_BROWS + rsub] = acc[0][0];
+        v = lane_sum<DQ6_P>(v);
+        if (sub == 0) part[bi * DQ6R_BROWS + rsub] = v;
         wait_lgkmcnt0();  // every read of the buffer returned before it is overwritten
         issue(bi + 2, buf);
     };
@@ -1757,53 +1643,39 @@ __global__ void __launch_bounds__(64 * WAVES_DN) k_decode_down_q6v(DecodeDownArg
 static bool dn_q6_ok(const DecodeDownArgs &a) {
     if (MX_DN_Q6 == 0) return false;
     auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const Geo<kQ6_K> g(DQ6_FF, DN_FULL);
-    return a.ff == DQ6_FF && a.d_row_bytes == DQ6_RB && g.P == DQ6_P && g.NG == DQ6_NG && g.G == DQ6_P * DQ6_NG &&
+    return a.ff == DQ6_FF && a.d_row_bytes == DQ6_RB &&
            a.hidden % RW_DN == 0 && (size_t)xstage_bytes(DQ6_FF) <= (size_t)DQ6R_NI * 1024 &&
            a.d_expert_bytes % 16 == 0 && al(a.down) && (!a.sh_down || (a.sh_row_bytes == DQ6_RB && al(a.sh_down)));
 }
 
 // the slot waves (3 per SIMD: 168 VGPRs) hold this many activation groups without
 // spilling to scratch; wider rows take k_decode_down and the combine
-template <int DT> constexpr int dn_slots_max_ng() { return DT == kQ8_0 ? 4 : DT == kQ6_K ? 3 : 2; }
-template <int DT, int NG>
-static mx_status launch_dn_slots_ng(const DecodeDownArgs &a, hipStream_t s) {
-    if constexpr (NG > dn_slots_max_ng<DT>()) {  // (not instantiated: dn_slots_fit refuses these)
-        (void)a;
-        (void)s;
-        return fail(MX_ERR_SHAPE, "decode down: %d activation groups per lane exceed the slot kernel", NG);
-    } else {
-        const int ni = ring_insts<DT, NG>(1, a.ff, a.d_row_bytes, BatchDnSlots<NG>::NIT, DN_FULL);
-        if (ni > DMA_MAX_INSTS) return fail(MX_ERR_SHAPE, "decode down: rows too long for the LDS ring");
-        const int slots = a.top_k + (a.sh_down ? 1 : 0);
-        const size_t lds = (size_t)slots * dn_slot_area(a.ff, ni);
-        const dim3 grid((unsigned)((a.hidden + RW_DN - 1) / RW_DN), (unsigned)a.t);
-        hipLaunchKernelGGL((k_decode_down_slots<DT, NG>), grid, dim3(64 * slots), lds, s, a, ni, Geo<DT>(a.ff, DN_FULL));
-        return MX_OK;
+template <int DT> constexpr int dn_slots_max_ng() { return DT == kQ4_K || DT == kQ5_K ? 2 : 3; }
+// rows per tile, rows per batch and the two LDS areas of a slot wave
+#ifndef MX_DN_TILES
+#define MX_DN_TILES 160
+#endif
+struct DnSlots {
+    int rows, br, area, area1;
+    size_t lds;
+    DnSlots(const DecodeDownArgs &a, int rpi) {
+        // (fewer rows per tile where 16 leave many CUs without one: hidden 2048 down
+        // 10.0 -> 8.1 us; at hidden 3072, 192 tiles, 16 rows take 13.8 us and 8 rows 14.6)
+        rows = (int64_t)((a.hidden + RW_DN - 1) / RW_DN) * a.t >= MX_DN_TILES || RW_DN / 2 < rpi ? RW_DN : RW_DN / 2;
+        br = batch_rows(rpi, a.d_row_bytes, rows / 2 < rpi ? rpi : rows / 2);
+        area = batch_area(br, a.d_row_bytes);
+        const int stg = (int)align16(xstage_bytes(a.ff));
+        area1 = area > stg ? area : stg;
+        lds = (size_t)(a.top_k + (a.sh_down ? 1 : 0)) * (area + area1);
     }
-}
-// LDS bytes of the slot-per-wave kernel (SIZE_MAX: its DMA batch does not fit)
-template <int DT, int NG>
-static size_t dn_slots_lds(const DecodeDownArgs &a) {
-    const int ni = ring_insts<DT, NG>(1, a.ff, a.d_row_bytes, BatchDnSlots<NG>::NIT, DN_FULL);
-    if (ni > DMA_MAX_INSTS) return SIZE_MAX;
-    const int slots = a.top_k + (a.sh_down ? 1 : 0);
-    return (size_t)slots * dn_slot_area(a.ff, ni);
-}
+};
 // true when the slot-per-wave kernel takes this launch
-template <int DT>
-static bool dn_slots_fit(const DecodeDownArgs &a) {
-    if (!MX_DN_SLOTS || a.t > MX_DN_SLOTS_MAX_T) return false;
-    if (a.top_k + (a.sh_down ? 1 : 0) > DN_SLOTS_MAX) return false;
-    const int ng = ng_variant(Geo<DT>(a.ff, DN_FULL).NG);
-    if (ng > dn_slots_max_ng<DT>()) return false;
-    size_t lds = SIZE_MAX;
-    [&] {
-#define MX_L(N) { lds = dn_slots_lds<DT, N>(a); return; }
-        MX_NG_SWITCH(ng, MX_L)
-#undef MX_L
-    }();
-    return lds <= 160 * 1024 - sizeof(float) * DN_SLOTS_MAX * RW_DN;
+template <int DT> static bool dn_slots_fit(const DecodeDownArgs &a) {
+    if (a.t > MX_DN_SLOTS_MAX_T || a.top_k + (a.sh_down ? 1 : 0) > DN_SLOTS_MAX) return false;
+    return with_lanes<DT>(groups<DT>(a.ff), [&](auto lpr, auto ng) {
+        return decltype(ng)::value <= dn_slots_max_ng<DT>() &&
+               DnSlots(a, 64 / decltype(lpr)::value).lds <= 160 * 1024 - sizeof(float) * DN_SLOTS_MAX * RW_DN;
+    });
 }
 template <int DT>
 static mx_status launch_dn_slots_dt(const DecodeDownArgs &a, hipStream_t s) {
@@ -1812,40 +1684,51 @@ static mx_status launch_dn_slots_dt(const DecodeDownArgs &a, hipStream_t s) {
             const int slots = a.top_k + (a.sh_down ? 1 : 0);
             const dim3 grid((unsigned)(a.hidden / RW_DN), (unsigned)a.t);
             if (a.t == 1)
-                hipLaunchKernelGGL(k_decode_down_q6r<DMA_NT>, grid, dim3(64 * slots), 0, s, a,
-                                   Geo<kQ6_K>(DQ6_FF, DN_FULL));
+                hipLaunchKernelGGL(k_decode_down_q6r<DMA_NT>, grid, dim3(64 * slots), 0, s, a);
             else
-                hipLaunchKernelGGL(k_decode_down_q6r<0>, grid, dim3(64 * slots), 0, s, a, Geo<kQ6_K>(DQ6_FF, DN_FULL));
+                hipLaunchKernelGGL(k_decode_down_q6r<0>, grid, dim3(64 * slots), 0, s, a);
             return MX_OK;
         }
     }
-    const int ng = ng_variant(Geo<DT>(a.ff, DN_FULL).NG);
-#define MX_L(N) return launch_dn_slots_ng<DT, N>(a, s)
-    MX_NG_SWITCH(ng, MX_L)
-#undef MX_L
-    return MX_OK;
+    return with_lanes<DT>(groups<DT>(a.ff), [&](auto lpr, auto ng) -> mx_status {
+        constexpr int LPR = decltype(lpr)::value, NG = decltype(ng)::value;
+        if constexpr (NG > dn_slots_max_ng<DT>()) {  // (dn_slots_fit refuses these)
+            return fail(MX_ERR_SHAPE, "decode down: %d activation groups per lane exceed the slot kernel", NG);
+        } else {
+            const DnSlots d(a, 64 / LPR);
+            const int slots = a.top_k + (a.sh_down ? 1 : 0);
+            const dim3 grid((unsigned)((a.hidden + d.rows - 1) / d.rows), (unsigned)a.t);
+            if (a.t == 1)
+                hipLaunchKernelGGL((k_decode_down_slots<DT, NG, LPR, DMA_NT>), grid, dim3(64 * slots), d.lds, s, a,
+                                   d.rows, d.br, d.area, d.area1);
+            else
+                hipLaunchKernelGGL((k_decode_down_slots<DT, NG, LPR, 0>), grid, dim3(64 * slots), d.lds, s, a, d.rows,
+                                   d.br, d.area, d.area1);
+            return MX_OK;
+        }
+    });
 }
 
-template <int DT, int NG>
-static mx_status launch_dn_ng(const DecodeDownArgs &a, dim3 grid, hipStream_t s) {
-    const int ni = ring_insts<DT, NG>(1, a.ff, a.d_row_bytes, BatchDn<NG>::NIT, DN_FULL);
-    if (ni > DMA_MAX_INSTS) return fail(MX_ERR_SHAPE, "decode down: rows too long for the LDS ring");
-    const size_t lds = align16(xstage_bytes(a.ff)) + (size_t)WAVES_DN * RING_DN * ni * 1024;
-    if (lds > 160 * 1024) return fail(MX_ERR_SHAPE, "decode down: expert_ff = %d needs %zu bytes of LDS", a.ff, lds);
-    // RW_DN * DN_TPB rows per wave: each workgroup stages its act row once for that many
-    const int rpw = RW_DN * DN_TPB;
-    const dim3 g((unsigned)((a.hidden + WAVES_DN * rpw - 1) / (WAVES_DN * rpw)), grid.y, grid.z);
-    hipLaunchKernelGGL((k_decode_down<DT, NG>), g, dim3(64 * WAVES_DN), lds, s, a, ni, rpw, Geo<DT>(a.ff, DN_FULL));
-    return MX_OK;
-}
-
+// waves a down launch aims at; 16 to 64 rows each (the act row is staged once per
+// workgroup)
+#ifndef MX_DN_WAVES
+#define MX_DN_WAVES 6144
+#endif
 template <int DT>
-static mx_status launch_dn_dt(const DecodeDownArgs &a, dim3 grid, hipStream_t s) {
-    const int ng = ng_variant(Geo<DT>(a.ff, DN_FULL).NG);
-#define MX_L(N) return launch_dn_ng<DT, N>(a, grid, s)
-    MX_NG_SWITCH(ng, MX_L)
-#undef MX_L
-    return MX_OK;
+static mx_status launch_dn_dt(const DecodeDownArgs &a, hipStream_t s) {
+    const int slots = a.top_k + (a.sh_down ? 1 : 0);
+    return with_lanes<DT>(groups<DT>(a.ff), [&](auto lpr, auto ng) -> mx_status {
+        constexpr int LPR = decltype(lpr)::value, NG = decltype(ng)::value;
+        int rpw = 16;
+        while (rpw < 64 && (int64_t)a.hidden * slots * a.t >= (int64_t)3 * rpw * MX_DN_WAVES / 2) rpw *= 2;
+        const int br = batch_rows(64 / LPR, a.d_row_bytes, rpw), area = batch_area(br, a.d_row_bytes);
+        const size_t stg = align16(xstage_bytes(a.ff));
+        const int two = stg + (size_t)WAVES_DN * 2 * area <= 160 * 1024;
+        const size_t lds = stg + (size_t)WAVES_DN * (two ? 2 : 1) * area;
+        const dim3 g((unsigned)((a.hidden + WAVES_DN * rpw - 1) / (WAVES_DN * rpw)), (unsigned)slots, (unsigned)a.t);
+        hipLaunchKernelGGL((k_decode_down<DT, NG, LPR>), g, dim3(64 * WAVES_DN), lds, s, a, rpw, br, area, two);
+        return MX_OK;
+    });
 }
 
 mx_status launch_decode_down(int dtype, const DecodeDownArgs &a, hipStream_t s) {
@@ -1875,16 +1758,16 @@ mx_status launch_decode_down(int dtype, const DecodeDownArgs &a, hipStream_t s) 
     }
     if (dtype == kQ6_K && MX_DN_Q6V && dn_q6_ok(a) && a.hidden % (WAVES_DN * DQ6V_RPW) == 0) {
         const dim3 g((unsigned)(a.hidden / (WAVES_DN * DQ6V_RPW)), grid.y, grid.z);
-        hipLaunchKernelGGL(k_decode_down_q6v, g, dim3(64 * WAVES_DN), 0, s, a, Geo<kQ6_K>(DQ6_FF, DN_FULL));
+        hipLaunchKernelGGL(k_decode_down_q6v, g, dim3(64 * WAVES_DN), 0, s, a);
         MX_LAUNCH("k_decode_down_q6v");
         return launch_combine_prefill(a.part, a.w, a.residual, a.t, a.top_k, a.sh_down ? 1 : 0, a.hidden, a.out, s,
                                       a.shared_out);
     }
     switch (dtype) {
-    case kQ4_K: MX_TRY(launch_dn_dt<kQ4_K>(a, grid, s)); break;
-    case kQ5_K: MX_TRY(launch_dn_dt<kQ5_K>(a, grid, s)); break;
-    case kQ6_K: MX_TRY(launch_dn_dt<kQ6_K>(a, grid, s)); break;
-    default: MX_TRY(launch_dn_dt<kQ8_0>(a, grid, s)); break;
+    case kQ4_K: MX_TRY(launch_dn_dt<kQ4_K>(a, s)); break;
+    case kQ5_K: MX_TRY(launch_dn_dt<kQ5_K>(a, s)); break;
+    case kQ6_K: MX_TRY(launch_dn_dt<kQ6_K>(a, s)); break;
+    default: MX_TRY(launch_dn_dt<kQ8_0>(a, s)); break;
     }
     MX_LAUNCH("k_decode_down");
     return launch_combine_prefill(a.part, a.w, a.residual, a.t, a.top_k, a.sh_down ? 1 : 0, a.hidden, a.out, s,
