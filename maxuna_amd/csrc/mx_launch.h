@@ -29,6 +29,12 @@ mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s);
 // launch_mul_mv_id runs the f32 mat-vec (mx_mvf.hip)
 bool mv_ring_fits(int dtype, int k);
 
+// mx_mvt.hip -- plain mat-vec for several tokens (2 and more): one matrix w
+// [n_out, k], x [t, k] -> dst [t, n_out]
+bool mv_tokens_fits(int t, int k);
+mx_status launch_mv_tokens(int dtype, const uint8_t *w, int64_t row_bytes, int n_out, int k, const float *x, int t,
+                           float *dst, hipStream_t s);
+
 // mx_mvf.hip -- f32 gather mat-vec for any k (a multiple of the block size).
 // dst row of (token, slot): (token * dst_stride + slot + dst_add) * n_out.
 struct MvfArgs {

@@ -762,7 +762,12 @@ static mx_status launch_mv_q6(const MvArgs &a, int ng, int p, hipStream_t s) {
 // with at most DMA_MAX_INSTS wave instructions per matrix set, and needs its LDS.
 template <int DT> static int64_t row_bytes_of(int k) { return (int64_t)(k / block_size(DT)) * type_size(DT); }
 template <int DT> static bool mv_fits_dt(int k) {
-    if (k <= 0 || k % block_size(DT) || groups<DT>(k) > G_MAX) return false;
+    const int G = groups<DT>(k);
+    if (k <= 0 || k % block_size(DT) || G > G_MAX) return false;
+    // Q4_K / Q5_K rows of 28 and 56 groups (k = 1792, 3584) keep the f32 mat-vec: it
+    // is what they have always had, and its error is the smaller (Q4_K [50000 x
+    // 3584]: 1.5e-7 against 2.7e-7 with the activation grid)
+    if ((DT == kQ4_K || DT == kQ5_K) && (G == 28 || G == 56)) return false;
     return dma_insts(1, 1, row_bytes_of<DT>(k)) <= DMA_MAX_INSTS &&
            align16(xstage_bytes(k)) + (size_t)WAVES * batch_area(1, row_bytes_of<DT>(k)) <= 160 * 1024;
 }
@@ -789,6 +794,12 @@ bool decode_down_fits(int dtype, int ff, int64_t row_bytes) { MX_DT_SWITCH(dtype
 
 mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s) {
     if (a.n_out == 0 || (int64_t)a.t * a.top_k == 0) return MX_OK;
+    // one matrix, several tokens: the weights read once for up to 16 of them (lm_head
+    // [100352 x 3072] Q6_K, us, per-token mat-vecs against this: t = 2 84 / 78, 4 133 /
+    // 77, 8 255 / 78, 16 503 / 82), and the one-token rows the ring kernel does not
+    // take (Q4_K [50000 x 3584] 94 / 48; both forms' errors are below theirs)
+    if (!a.ids && a.top_k == 1 && mv_tokens_fits(a.t, a.k) && (a.t > 1 || !mv_ring_fits(dtype, a.k)))
+        return launch_mv_tokens(dtype, a.w, a.row_bytes, a.n_out, a.k, a.x, a.t, a.dst, s);
     if (!mv_ring_fits(dtype, a.k)) {  // any other row width: the f32 mat-vec
         const MvfArgs f{a.w, a.expert_bytes, a.row_bytes, a.n_expert, a.n_out, a.k, a.x, a.x_per_row,
                         a.ids, a.t, a.top_k, a.dst, a.top_k, 0};

@@ -84,3 +84,52 @@ def test_mul_mv_row_widths(orc, dt, k):
         r = rel_l2(got, x.astype(np.float64) @ w.astype(np.float64).T)
         print(f"{dt.name} [{n_out} x {k}] t={t}: rel-L2 {r:.2e}", flush=True)
         assert r <= F32_CLASS
+
+
+def _mul_mv_errors(orc, dt, n_out, k, x, off=0):
+    """Relative error of each token's row of mul_mv against float64."""
+    st = synth_stack(dt, 1, n_out, k, tensor_key(4500, 0, n_out))
+    raw = torch.zeros(off + st.nbytes, dtype=torch.uint8, device="cuda")
+    raw[off:] = st.buffer
+    got = host(ops.mul_mv(raw[off:], dt, n_out, k, dev_f32(x))).astype(np.float64)
+    w = orc.dequantize(int(dt), host(st.buffer), n_out * k).reshape(n_out, k).astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    return np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+
+
+# two f16 pieces carry an activation to 2^-23 of itself, so f32 sums dominate: rows
+# of at most 6400 centred products, errors near 2e-7 (bound: 1e-6 per token)
+TOKENS = 1e-6
+
+
+@pytest.mark.parametrize("dt", [GgmlDType.Q4_K, GgmlDType.Q5_K, GgmlDType.Q6_K, GgmlDType.Q8_0], ids=lambda v: v.name)
+@pytest.mark.parametrize("k", [256, 512, 1792, 3072, 3328, 6400])
+def test_mul_mv_tokens(orc, dt, k):
+    """1 to 12 waves a workgroup, and K cut into two and three launches; partial row
+    tiles and token groups; weights off 16-byte alignment where the type allows it."""
+    rng = np.random.default_rng(k)
+    off = 2 if dt in (GgmlDType.Q6_K, GgmlDType.Q8_0) else 0
+    for n_out, t in ((1, 2), (15, 3), (16, 16), (17, 17), (333, 5), (4200, 33)):
+        err = _mul_mv_errors(orc, dt, n_out, k, rng.standard_normal((t, k)).astype(np.float32), off)
+        print(f"{dt.name} [{n_out} x {k}] t={t}: {err.max():.2e}", flush=True)
+        assert err.max() <= (TOKENS if n_out > 16 else F32_CLASS)
+
+
+def test_mul_mv_tokens_ranges(orc):
+    """Tokens of very different magnitudes, super-blocks 2^40 apart, an all-zero token,
+    and a token with an Inf: only that token's outputs are not finite."""
+    rng = np.random.default_rng(3)
+    k, n_out = 1024, 200
+    x = rng.standard_normal((6, k)).astype(np.float32)
+    x[1] *= np.float32(2.0**-100)
+    x[2] *= np.float32(2.0**90)
+    x[3, 256:512] *= np.float32(2.0**40)
+    x[4] = 0
+    for dt in (GgmlDType.Q4_K, GgmlDType.Q6_K):
+        err = _mul_mv_errors(orc, dt, n_out, k, x[[0, 1, 2, 3]])
+        assert err.max() <= TOKENS, err
+        st = synth_stack(dt, 1, n_out, k, 9)
+        bad = x.copy()
+        bad[5, 700] = np.inf
+        got = host(ops.mul_mv(st.buffer, dt, n_out, k, dev_f32(bad)))
+        assert np.all(np.isfinite(got[:5])) and np.all(got[4] == 0) and not np.any(np.isfinite(got[5]))
