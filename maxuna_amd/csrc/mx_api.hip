@@ -41,6 +41,11 @@ mx_status hip_check(hipError_t e, const char *what) {
 #endif
 constexpr int64_t kVmmMaxPairs = MX_VMM_MAX_PAIRS;
 static_assert(kVmmMaxPairs <= PAIR_ORDER_MAX, "the pair order covers the tiles' range");
+// ... and where the stationary-activation matmuls (mx_gst.hip) take the shape: C1-shaped
+// layers (11 slots), µs, tiles vs those: t = 32: 324 vs 371, 64: 414 vs 438, 128:
+// 541 vs 501, 200: 671 vs 581, 232: 730 vs 610; hidden 3072, ff 1024: t = 64: 251 vs
+// 256, 128: 328 vs 301, 200: 378 vs 339
+constexpr int64_t kVmmGstPairs = 1024;
 
 static bool supported(int dt) { return dt == kQ4_K || dt == kQ5_K || dt == kQ6_K || dt == kQ8_0; }
 static bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
@@ -232,11 +237,24 @@ size_t mm_tiles_order_bytes(int64_t pairs) { return (((size_t)pairs + 2 * ((size
 size_t mm_tiles_bytes(int64_t t, int64_t top_k, int64_t x_per_row, int64_t k) {
     return mm_tiles_order_bytes(t * top_k) + mm_x16_bytes(t, x_per_row, k);
 }
+// a projection's operands as the grouped kernels take them (A operand left out)
+GemmArgs mm_args(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64_t top_k) {
+    GemmArgs a{};
+    a.w[0] = g.w;
+    a.expert_bytes = g.expert_bytes; a.row_bytes = g.row_bytes; a.sh_row_bytes = g.row_bytes;
+    a.n_expert = (int)st->n_expert; a.n_out = (int)st->n_out; a.k = (int)st->k;
+    a.t = (int)t; a.top_k = (int)top_k; a.n_map_expert = (int)st->n_expert;
+    a.out_stride = (int)top_k;
+    return a;
+}
+bool mm_on_gst(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64_t top_k) {
+    return gst_fits(st->dtype, mm_args(st, g, t, top_k), false);
+}
 // A few pairs per expert: the 16-pair MFMA tiles of the verify blocks (each
 // touched expert's weights streamed once) instead of 128-pair GEMM m-tiles
 bool mm_on_tiles(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64_t top_k) {
     return (st->dtype == kQ4_K || st->dtype == kQ6_K) && st->k % 512 == 0 && st->n_out % 32 == 0 &&
-           t * top_k <= kVmmMaxPairs && st->n_expert <= 1024 && (st->dtype != kQ4_K || g.row_bytes % 16 == 0) &&
+           t * top_k <= (mm_on_gst(st, g, t, top_k) ? kVmmGstPairs : kVmmMaxPairs) && st->n_expert <= 1024 && (st->dtype != kQ4_K || g.row_bytes % 16 == 0) &&
            st->n_out * g.row_bytes < ((int64_t)1 << 31) && st->k * 2 < ((int64_t)1 << 31);
 }
 // pair order, x -> scaled f16 rows (the Q4_K tiles' K order), the plain tiles;
@@ -289,18 +307,18 @@ mx_status mm_gemm(const mx_expert_stack *st, const StackGeom &g, const float *x,
     // one per token: the token's row, shared by its slots
     const MapLayout L((int)st->n_expert, (int)t, (int)top_k);
     const bool by_pair = x_per_row != 1;
-    if (by_pair)
-        MX_TRY(launch_to_f16_rows(x, t * top_k, k, map + L.off + st->n_expert, x16, x16s, s, false, map + L.list));
-    else
-        MX_TRY(launch_to_f16_rows(x, t, k, nullptr, x16, x16s, s));
-    GemmArgs a{};
-    a.w[0] = g.w;
-    a.expert_bytes = g.expert_bytes; a.row_bytes = g.row_bytes; a.sh_row_bytes = g.row_bytes;
-    a.n_expert = (int)st->n_expert; a.n_out = (int)st->n_out; a.k = k;
+    GemmArgs a = mm_args(st, g, t, top_k);
     a.a = x16; a.a_scale = x16s;
     a.a_div = by_pair ? 0 : (int)top_k;  // bucket position / token of the pair
-    a.t = (int)t; a.top_k = (int)top_k; a.n_map_expert = (int)st->n_expert; a.map = map;
-    a.out = dst; a.out_stride = (int)top_k; a.out_add = 0;
+    a.map = map;
+    a.out = dst;
+    const bool gst = mm_on_gst(st, g, t, top_k);
+    const bool perm = gst && st->dtype == kQ4_K;
+    if (by_pair)
+        MX_TRY(launch_to_f16_rows(x, t * top_k, k, map + L.off + st->n_expert, x16, x16s, s, perm, map + L.list));
+    else
+        MX_TRY(launch_to_f16_rows(x, t, k, nullptr, x16, x16s, s, perm));
+    if (gst) return launch_gst(st->dtype, false, a, s);
     return launch_gemm(st->dtype, false, a, s);
 }
 }  // namespace
@@ -474,6 +492,7 @@ struct Plan {
                             // router + f32 gather mat-vecs + SwiGLU + combine
     bool shared_in_decode;  // shared expert rides in the fused decode kernels (same quant types)
     bool vmm;               // verify block on the 16-pair MFMA tiles (after the fused router)
+    bool gst_gu, gst_d;     // grouped path: gate/up, down on the stationary-activation matmuls
     int64_t min_seq;
 };
 
@@ -481,9 +500,35 @@ int64_t stack_row_bytes(const mx_expert_stack &st) {
     return supported(st.dtype) ? st.k / block_size(st.dtype) * type_size(st.dtype) : 0;
 }
 
+// The grouped path's gate/up and down matmuls, whether mx_gst.hip takes them: one
+// bucket map (a shared expert of the routed quant types joins it), few pairs per
+// expert, aligned matrices.
+void plan_gst(const mx_moe_layer *L, int64_t t, Plan &p) {
+    p.gst_gu = p.gst_d = false;
+    if (p.has_shared && !p.shared_in_decode) return;
+    auto ptr = [](const mx_expert_stack &st) { return static_cast<const uint8_t *>(st.data) + st.base_off; };
+    const int64_t S = p.has_shared ? 1 : 0;
+    GemmArgs a{};
+    a.t = (int)t; a.top_k = (int)(L->top_k + S); a.n_expert = (int)L->gate.n_expert; a.n_map_expert = a.n_expert + (int)S;
+    auto set = [&](const mx_expert_stack &st, const mx_expert_stack &sh, int m) {
+        a.w[m] = ptr(st);
+        a.w_sh[m] = S ? ptr(sh) : nullptr;
+        a.row_bytes = stack_row_bytes(st);
+        a.sh_row_bytes = S ? stack_row_bytes(sh) : 0;
+        a.n_out = (int)st.n_out; a.k = (int)st.k;
+        a.expert_bytes = st.n_out * a.row_bytes;
+    };
+    set(L->up, L->shared_up, 1);
+    set(L->gate, L->shared_gate, 0);
+    p.gst_gu = gst_fits(L->gate.dtype, a, true);
+    set(L->down, L->shared_down, 0);
+    p.gst_d = gst_fits(L->down.dtype, a, false);
+}
+
 // Chooses the kernels of a forward; every shape limit of the chosen kernels is
 // checked here, so a validated call never fails after its first launch.
-Plan plan_for(const mx_moe_layer *L, int64_t t) {
+// small_ws: of two plans the one with the smaller workspace (the no-alloc forward)
+Plan plan_for(const mx_moe_layer *L, int64_t t, bool small_ws = false) {
     Plan p;
     p.min_seq = L->mm_min_seq > 0 ? L->mm_min_seq : kDefaultMmMinSeq;
     // < 0: never (LAGUNA_NO_MM_ID).  The MFMA GEMM needs K % 256 == 0 for every
@@ -500,6 +545,7 @@ Plan plan_for(const mx_moe_layer *L, int64_t t) {
     p.has_shared = L->shared_gate.data != nullptr;
     p.shared_in_decode = p.has_shared && L->shared_gate.dtype == L->gate.dtype &&
                          L->shared_down.dtype == L->down.dtype;
+    plan_gst(L, t, p);
     const bool decode_fits = decode_gate_up_fits(L->gate.dtype, (int)L->hidden, stack_row_bytes(L->gate)) &&
                              decode_down_fits(L->down.dtype, (int)L->expert_ff, stack_row_bytes(L->down));
     const int64_t slots = L->top_k + (p.shared_in_decode ? 1 : 0);
@@ -510,7 +556,7 @@ Plan plan_for(const mx_moe_layer *L, int64_t t) {
     // LAGUNA_NO_MM_ID (mm_min_seq < 0) keeps every t on the mat-vec kernels
     const bool vmm_ok =
         L->mm_min_seq >= 0 && decode_fits && t >= kVmmMinT && (!p.has_shared || p.shared_in_decode) &&
-        t * slots <= kVmmMaxPairs && L->gate.n_expert <= 1024 &&
+        t * slots <= (p.gst_gu && p.gst_d && shapes && t >= p.min_seq && !small_ws ? kVmmGstPairs : kVmmMaxPairs) && L->gate.n_expert <= 1024 &&
         vmm_supported(L->gate.dtype, L->down.dtype, (int)L->hidden, (int)L->expert_ff, gu_rb, d_rb) &&
         L->expert_ff * gu_rb < ((int64_t)1 << 31) && L->hidden * d_rb < ((int64_t)1 << 31) &&
         (!p.has_shared || (stack_row_bytes(L->shared_gate) == gu_rb && stack_row_bytes(L->shared_down) == d_rb));
@@ -694,7 +740,7 @@ struct Repeat {
 
 mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, const float *residual, float *out,
                            uint32_t *ids_out, float *w_out, void *workspace, size_t workspace_bytes,
-                           hipStream_t s, StageTimer *tm, Repeat rep = Repeat()) {
+                           hipStream_t s, StageTimer *tm, Repeat rep = Repeat(), bool small_ws = false) {
     StackGeom gg, gu, gd, sg{}, su{}, sd{};
     MX_TRY(check_layer(L, t, gg, gu, gd, sg, su, sd));
     if (t == 0) return MX_OK;
@@ -702,7 +748,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
     MX_TRY(check_f32(out, "out"));
     if (residual) MX_TRY(check_f32(residual, "residual"));
     if (!workspace) return fail(MX_ERR_NULL, "moe: workspace is NULL");
-    const Plan p = plan_for(L, t);
+    const Plan p = plan_for(L, t, small_ws);
     const Layout o = carve(L, t, p, workspace);
     if (workspace_bytes < o.bytes)
         return fail(MX_ERR_SCRATCH, "moe: workspace of %zu bytes, need %zu", workspace_bytes, o.bytes);
@@ -888,7 +934,9 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         }
     }
     MX_STAGE();
-    MX_TRY(launch_to_f16_rows(xin, t, (int)H, nullptr, o.x16, o.x16s, s));
+    // (the stationary-activation Q4_K matmuls read A in the verify tiles' K order)
+    const bool gst_gu = p.gst_gu, gst_d = p.gst_d;
+    MX_TRY(launch_to_f16_rows(xin, t, (int)H, nullptr, o.x16, o.x16s, s, gst_gu && L->gate.dtype == kQ4_K));
     MX_STAGE();
     // one bucket map's gate+up (SwiGLU, act rows at its bucket positions from act_row0 on)
     // and down (rows token * KK + slot + out_add)
@@ -906,10 +954,10 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         ga.a = o.x16; ga.a_scale = o.x16s; ga.a_div = top_k;
         ga.t = (int)t; ga.top_k = top_k; ga.n_map_expert = n_map_expert; ga.map = map;
         ga.out = o.act + act_row0 * FF;
-        MX_TRY(launch_gemm(dt_gu, true, ga, s));
+        MX_TRY(gst_gu ? launch_gst(dt_gu, true, ga, s) : launch_gemm(dt_gu, true, ga, s));
         MX_STAGE();
         MX_TRY(launch_to_f16_rows(ga.out, t * top_k, (int)FF, map + LM.off + n_map_expert,
-                                  o.act16 + act_row0 * FF, o.act16s + act_row0, s));
+                                  o.act16 + act_row0 * FF, o.act16s + act_row0, s, gst_d && dt_d == kQ4_K));
         MX_STAGE();
         GemmArgs da = ga;
         da.w[0] = wd; da.w[1] = nullptr;
@@ -918,7 +966,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         da.n_out = (int)H; da.k = (int)FF;
         da.a = o.act16 + act_row0 * FF; da.a_scale = o.act16s + act_row0; da.a_div = 0;
         da.out = o.down; da.out_stride = KK; da.out_add = out_add;
-        MX_TRY(launch_gemm(dt_d, false, da, s));
+        MX_TRY(gst_d ? launch_gst(dt_d, false, da, s) : launch_gemm(dt_d, false, da, s));
         MX_STAGE();
         return MX_OK;
     };
@@ -1026,7 +1074,11 @@ mx_status mx_moe_forward_noalloc(const mx_moe_layer *L, const float *x, int64_t 
                                  uint32_t *ids_out, float *w_out, mx_stream_t stream) {
     StackGeom gg, gu, gd, sg{}, su{}, sd{};
     MX_TRY(check_layer(L, t, gg, gu, gd, sg, su, sd));
-    const size_t need = mx_moe_workspace_bytes(L, t);
+    size_t need = mx_moe_workspace_bytes(L, t);
+    // (the verify tiles' workspace is the smaller one: they keep the sizes whose grouped
+    // path does not fit)
+    const bool small_ws = need > kNoAllocScratchBytes;
+    if (small_ws) need = carve(L, t, plan_for(L, t, true), nullptr).bytes;
     if (need > kNoAllocScratchBytes)
         return fail(MX_ERR_SCRATCH,
                     "no-alloc forward: t = %lld needs %zu bytes of workspace, its scratch holds %zu "
@@ -1036,7 +1088,7 @@ mx_status mx_moe_forward_noalloc(const mx_moe_layer *L, const float *x, int64_t 
     void *ws = nullptr;
     MX_TRY(scratch_for_current_device(&ws));
     return moe_forward_impl(L, x, t, residual, out, ids_out, w_out, ws, kNoAllocScratchBytes, (hipStream_t)stream,
-                            nullptr);
+                            nullptr, Repeat(), small_ws);
 }
 
 uint64_t mx_tensor_key(uint64_t seed, uint32_t layer, uint32_t tensor_id) {

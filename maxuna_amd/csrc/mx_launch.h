@@ -29,6 +29,9 @@ mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s);
 // launch_mul_mv_id runs the f32 mat-vec (mx_mvf.hip)
 bool mv_ring_fits(int dtype, int k);
 
+// compute units of the current device (mx_vmm.hip)
+int device_cus();
+
 // mx_mvt.hip -- plain mat-vec for several tokens (2 and more): one matrix w
 // [n_out, k], x [t, k] -> dst [t, n_out]
 bool mv_tokens_fits(int t, int k);
@@ -256,6 +259,10 @@ bool gemm_supported(int dtype, int k);
 bool gemm_fits(int t, int hidden, int ff, int64_t gu_row_bytes, int64_t d_row_bytes);
 // the same for one plain GEMM over a_rows A rows addressed by pair (a_div > 0)
 bool gemm_plain_fits(int64_t a_rows, int k, int n_out, int64_t row_bytes);
+// mx_gst.hip -- the same contraction for a few dozen pairs per expert (activations
+// stationary).  Q4_K: A rows in the verify tiles' K order (launch_to_f16_rows perm).
+bool gst_fits(int dtype, const GemmArgs &a, bool swiglu);
+mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 mx_status launch_gemm(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 // rows of x (f32, [rows, k], k % 4 == 0) -> f16 times a per-row power of two;
 // rows at or beyond *count (when count != NULL) are skipped.  perm: each group of

@@ -411,17 +411,6 @@ __global__ void __launch_bounds__(64 * MT_WAVES) k_mv_tokens(MtArgs a) {
 }
 
 namespace {
-int mt_cus() {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cus[dev]) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-        cus[dev] = v;
-    }
-    return cus[dev];
-}
 template <int DT> void mt_launch(MtArgs a, hipStream_t s) {
     const int nsb = a.k / 256, parts = (nsb + MT_WAVES - 1) / MT_WAVES, per = (nsb + parts - 1) / parts;
     for (a.sb = 0; a.sb < nsb; a.sb += per) {
@@ -429,7 +418,7 @@ template <int DT> void mt_launch(MtArgs a, hipStream_t s) {
         // resident workgroups: 12 waves per CU by registers, and by LDS
         const int by_lds = 160 * 1024 / (MtLds<DT>::bytes(W) + MtLds<DT>::FIXED), by_waves = MT_WAVES / W;
         const int per_cu = by_lds < by_waves ? by_lds : by_waves;
-        const int tiles = (a.n_out + MT_ROWS - 1) / MT_ROWS, most = per_cu * mt_cus();
+        const int tiles = (a.n_out + MT_ROWS - 1) / MT_ROWS, most = per_cu * device_cus();
         const dim3 grid((unsigned)(tiles < most ? tiles : most), (unsigned)((a.t + MT_TOK - 1) / MT_TOK));
         if (a.sb) hipLaunchKernelGGL((k_mv_tokens<DT, true>), grid, dim3(64 * W), MtLds<DT>::bytes(W), s, a);
         else hipLaunchKernelGGL((k_mv_tokens<DT, false>), grid, dim3(64 * W), MtLds<DT>::bytes(W), s, a);

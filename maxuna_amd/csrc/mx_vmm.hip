@@ -42,6 +42,7 @@
 #include "mx_launch.h"
 #include "mx_dma.h"
 #include "mx_wb.h"
+#include "mx_vmq.h"
 
 namespace mx {
 
@@ -71,71 +72,6 @@ template <int DT, bool SWIGLU, int COLS> struct VmGeo {
     static constexpr int NI = (POS + 63) / 64;  // copy instructions per stage
     static constexpr int BUF = NI * 1024;       // bytes per stage buffer (spare lanes land past POS)
     static constexpr bool kBuf = DT == kQ6_K;   // copies through a buffer resource
-};
-
-// Q6_K half super-block `par` of the lane's row from its stage slot (the whole
-// block, from the 16-byte-aligned address below it; m1 = the block's phase):
-// the registers WB<kQ6_K>::load_lds fills from the prefill GEMM's per-half slots.
-__device__ __forceinline__ void vm_load(WB<kQ6_K> &w, const uint8_t *slot, int kh, uint32_t m1, int par) {
-    w.lo = lds16_a2(slot, m1 + 64 * par + 16 * kh);       // ql[64 par + 16 kh, +16)
-    w.hi = lds16_a2(slot, m1 + 64 * par + 32 + 16 * kh);  // ql[64 par + 32 + 16 kh, +16)
-    w.qh = lds16_a2(slot, m1 + 128 + 32 * par + 16 * kh); // qh[32 par + 16 kh, +16)
-    const uint32_t so = m1 + 192 + 8 * par;               // scales[8 par, +8)
-    const uint32_t *p = reinterpret_cast<const uint32_t *>(slot + (so & ~3u));
-    const uint32_t sh = (so & 2u) * 8u;
-    const uint32_t a0 = p[0], a1 = p[1], a2 = p[2];
-    w.s0 = __builtin_amdgcn_alignbit(a1, a0, sh);
-    w.s1 = __builtin_amdgcn_alignbit(a2, a1, sh);
-    w.dbits = *reinterpret_cast<const uint16_t *>(slot + m1 + 208);
-}
-
-// Q4_K half super-block `PAR` of the lane's row for the sub-block-per-lane
-// order: sub-block j = 4 PAR + q (32 values, one 6-bit scale and min).  Word i of
-// its 32 quant bytes holds values 4 i .. 4 i + 3 in the lane's nibble (low for
-// even q, high for odd q).  One and-or against the f16 exponent 0x6400 turns a
-// word into the f16 pair 1024 + q of values 4 i and 4 i + 2 (the word shifted by
-// a byte: 4 i + 1 and 4 i + 3), so step P gives values 8 P + {0, 2, 1, 3, 4, 6,
-// 5, 7}: the A rows are stored in that order (launch_to_f16_rows with perm).  A
-// high nibble reads as 1024 + 16 q, so odd sub-blocks take d1 / 16 (exact); each
-// value is the f32 fma (1024 + q) d1 + c rounded to f16 once, as in WB<kQ4_K>.
-struct VmQ4 {
-    uint32_t w[8];  // the quant bytes of values 4 i .. 4 i + 3 in word i
-    uint32_t m;     // the lane's nibble of bytes 0 and 2: 0x000F000F or 0x00F000F0
-    float d1, c1;   // d * sc (/ 16 for a high nibble) and -dmin * m - 1024 * d1
-    template <int PAR> __device__ __forceinline__ void load(const uint8_t *slot, int q) {
-        const uint4 h = *reinterpret_cast<const uint4 *>(slot);  // d, dmin | scales[12]
-        const uint8_t *qs = slot + 16 + 64 * PAR + 32 * (q >> 1); // the sub-block pair's 32 bytes
-        const uint4 a = *reinterpret_cast<const uint4 *>(qs);
-        const uint4 b = *reinterpret_cast<const uint4 *>(qs + 16);
-        w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
-        w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
-        m = (q & 1) ? 0x00F000F0u : 0x000F000Fu;
-        // get_scale_min_k4 of sub-block j (q4k_scale_min) with j = 4 PAR + q
-        const uint32_t o = 8u * (uint32_t)q;
-        uint32_t sc, mn;
-        if constexpr (PAR == 0) {
-            sc = __builtin_amdgcn_ubfe(h.y, o, 6);
-            mn = __builtin_amdgcn_ubfe(h.z, o, 6);
-        } else {
-            const uint32_t b8 = __builtin_amdgcn_ubfe(h.w, o, 8);
-            sc = (b8 & 0xFu) | (__builtin_amdgcn_ubfe(h.y, o + 6, 2) << 4);
-            mn = (b8 >> 4) | (__builtin_amdgcn_ubfe(h.z, o + 6, 2) << 4);
-        }
-        const float d = h2f((uint16_t)(h.x & 0xFFFFu)), dmin = h2f((uint16_t)(h.x >> 16));
-        d1 = d * (float)sc * ((q & 1) ? 0.0625f : 1.0f);
-        c1 = __builtin_fmaf(-1024.0f, d1, -(dmin * (float)mn));
-    }
-    __device__ __forceinline__ half8_t step(int P) const {
-        const uint32_t r0 = w[2 * P], r1 = w[2 * P + 1];
-        const half2_t x[4] = {__builtin_bit_cast(half2_t, (r0 & m) | 0x64006400u),
-                              __builtin_bit_cast(half2_t, ((r0 >> 8) & m) | 0x64006400u),
-                              __builtin_bit_cast(half2_t, (r1 & m) | 0x64006400u),
-                              __builtin_bit_cast(half2_t, ((r1 >> 8) & m) | 0x64006400u)};
-        half2_t y[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) y[i] = mix2(x[i], d1, c1);
-        return pk_join(y);
-    }
 };
 
 // One work item, as a wave sees it.  Uniform: the matrices and the run; per
@@ -373,8 +309,7 @@ k_vmm(VmmArgs a, const int32_t *__restrict__ perm, const int32_t *__restrict__ r
     wait_vmcnt(0);  // the clamped re-copy has landed before the wave's LDS can be reused
 }
 
-namespace {
-int vm_cus() {
+int device_cus() {
     static int cus[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -385,7 +320,7 @@ int vm_cus() {
     }
     return cus[dev];
 }
-}  // namespace
+
 
 bool vmm_supported(int gate_dtype, int down_dtype, int hidden, int ff, int64_t gu_row_bytes, int64_t d_row_bytes) {
     // both contractions need an even number of super-blocks and 32-column
@@ -418,7 +353,7 @@ void vm_launch(const VmmArgs &a, int max_runs, hipStream_t s) {
     const int64_t want = (items + VM_WAVES - 1) / VM_WAVES;
     // resident workgroups per CU: WPE by registers (4 waves each), and by LDS
     const int by_lds = (160 * 1024) / (2 * VM_WAVES * G::BUF);
-    const int64_t cap = (int64_t)(WPE < by_lds ? WPE : by_lds) * vm_cus();
+    const int64_t cap = (int64_t)(WPE < by_lds ? WPE : by_lds) * device_cus();
     const unsigned grid = (unsigned)(want < cap ? want : cap);
     hipLaunchKernelGGL((k_vmm<DT, SWIGLU, COLS, WPE>), dim3(grid), dim3(64 * VM_WAVES), 0, s, a, a.perm, a.runs,
                        a.a_scale);

@@ -65,6 +65,14 @@ __device__ __forceinline__ half8_t pk_join(const half2_t (&y)[4]) {
     }
     return r;
 }
+// four words from LDS as a vector of words (not through the uint4 struct, whose
+// type-based alias class covers everything: the compiler then waits for every LDS
+// copy in flight before the read)
+typedef uint32_t word4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 ld_w4(const uint8_t *p) {
+    const word4_t v = *reinterpret_cast<const word4_t *>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 // d1 = d * sc, c = -dmin * m - 1024 * d1 (f32)
 __device__ __forceinline__ half8_t dq8_kmin(uint32_t w0, uint32_t w1, float d1, float c) {
     half2_t x[4], y[4];

@@ -8,10 +8,10 @@ import pytest
 import torch
 
 from maxuna_amd import ops
-from maxuna_amd.gguf import GgmlDType
+from maxuna_amd.gguf import ExpertStack, GgmlDType
 from maxuna_amd.synth import LayerSpec, build_layer, make_x, synth_stack, tensor_key
 
-from tests.gpu_util import check_ids, dev_f32, host, rel_l2, selection_margin
+from tests.gpu_util import assert_close, check_ids, dev_f32, dev_u32, host, rel_l2, selection_margin
 
 pytestmark = pytest.mark.gpu
 
@@ -133,3 +133,45 @@ def test_mul_mv_tokens_ranges(orc):
         bad[5, 700] = np.inf
         got = host(ops.mul_mv(st.buffer, dt, n_out, k, dev_f32(bad)))
         assert np.all(np.isfinite(got[:5])) and np.all(got[4] == 0) and not np.any(np.isfinite(got[5]))
+
+
+# (gate/up type, down type, hidden, ff): super-blocks of K at the ends of the wave
+# layouts of the stationary-activation matmuls (2 | 4 | 6 | 12 waves of one, 8 of two,
+# then three and four), each type on both projections
+GST = [
+    ("Q4_K", "Q4_K", 512, 768), ("Q4_K", "Q6_K", 1280, 1536), ("Q4_K", "Q6_K", 3072, 1792), ("Q4_K", "Q4_K", 3328, 1024),
+    ("Q4_K", "Q5_K", 4352, 512), ("Q4_K", "Q6_K", 6400, 512), ("Q5_K", "Q5_K", 1024, 2304), ("Q5_K", "Q6_K", 4096, 1280),
+    ("Q6_K", "Q6_K", 1536, 768), ("Q6_K", "Q5_K", 3840, 512), ("Q6_K", "Q4_K", 5120, 512), ("Q8_0", "Q8_0", 512, 1024),
+    ("Q8_0", "Q8_0", 2048, 1280), ("Q8_0", "Q8_0", 2560, 768), ("Q8_0", "Q8_0", 4096, 512), ("Q8_0", "Q8_0", 7168, 512),
+]
+
+
+@pytest.mark.parametrize("gate,down,hidden,ff", GST)
+def test_few_pairs_per_expert(orc, gate, down, hidden, ff):
+    """Layers of a few pairs per expert past the verify tiles, with runs of one and of
+    several tiles of pairs (a hot expert) and experts of none, against the oracle's own
+    routing.  f16 operands: the contract's bound."""
+    spec = LayerSpec(hidden, ff, 40, 4, GgmlDType[gate], GgmlDType[down], shared=hidden % 512 == 0, bias_sigma=0.3)
+    layer = build_layer(spec, seed=4600)
+    # past the verify tiles' pairs where the types have tiles, and under the 24 (K up to
+    # 4096) or 6 pairs per expert that these matmuls take
+    x = make_x(spec, 4601, 50 if hidden > 4096 else 210 if gate == "Q4_K" else 70)
+    out, ids, w = layer.block.forward(torch.from_numpy(x).cuda(), return_routing=True)
+    out, ids, w = host(out), host(ids), host(w)
+    want, _, _ = orc.moe_layer(spec, layer.keys, layer.router_t, layer.bias, x, ids=ids, w=w)
+    assert_close(out, want, what=f"{gate}/{down} {hidden}x{ff}")
+
+
+def test_few_pairs_per_expert_alignment_rule(orc):
+    """Q6_K stacks two bytes off 16-byte alignment take the other grouped kernel: same
+    outputs to f16-operand rounding."""
+    rng = np.random.default_rng(8)
+    t, top_k, e, n_out, k = 400, 4, 64, 512, 768
+    st = synth_stack(GgmlDType.Q6_K, e, n_out, k, tensor_key(4700, 0, 1))
+    raw = torch.zeros(st.nbytes + 2, dtype=torch.uint8, device="cuda")
+    raw[2:] = st.buffer
+    off = ExpertStack(raw, GgmlDType.Q6_K, e, n_out, k, 2)
+    ids = dev_u32(np.argsort(rng.random((t, e)), axis=1)[:, :top_k])
+    x = dev_f32(rng.standard_normal((t, 1, k)).astype(np.float32))
+    a, b = host(ops.mul_mm_id(st, x, ids)), host(ops.mul_mm_id(off, x, ids))
+    assert rel_l2(a, b) <= 1e-6  # (the same products in another order of summation)
