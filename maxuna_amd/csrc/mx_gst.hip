@@ -26,10 +26,10 @@
 //  * SwiGLU: a tile is 16 gate rows, then the same 16 up rows; the thread that
 //    sums a gate value keeps it until its up value is summed.
 //
-// Bound by instruction issue: about 180 (Q4_K) to 290 (Q6_K) VALU per wave and stage
+// Bound by instruction issue: about 180 (Q4_K) to 260 (Q6_K) VALU per wave and stage
 // of 16 x 256 weights, once per run of 32 pairs.  top-10 of 256 experts, hidden 4096,
 // ff 1536, Q4_K / Q6_K, grouped GEMM against these (gate, up and down with the
-// passes between them): t = 300 1180 / 892 us, 512 1279 / 1120, 700 1410 / 1300,
+// passes between them): t = 300 1180 / 892 us, 512 1267 / 1078, 700 1410 / 1300,
 // 1000 1548 / 1590.  Weight bytes fetched for the gate projection at t = 512: 1.46 ->
 // 1.19 GB (0.91 GB of weights, read once per run).  Also tried: reading a stage's
 // words one stage ahead (no change: latency of LDS is not what it waits on), and the
@@ -64,8 +64,8 @@ template <int PAR> __device__ __forceinline__ void gs_load(WB<kQ5_K> &w, const u
     w.q[0] = ld_w4(slot + 48 + 64 * PAR + 16 * kh);
     w.q[1] = ld_w4(slot + 80 + 64 * PAR + 16 * kh);
 }
-template <int PAR> __device__ __forceinline__ void gs_load(WB<kQ6_K> &w, const uint8_t *slot, int q, uint32_t ph) {
-    vm_load(w, slot, q >> 1, ph, PAR);
+template <int PAR> __device__ __forceinline__ void gs_load(VmQ6 &w, const uint8_t *slot, int q, uint32_t ph) {
+    w.template load<PAR>(slot, q, ph);
 }
 template <int PAR> __device__ __forceinline__ void gs_load(WB<kQ8_0> &w, const uint8_t *slot, int q, uint32_t ph) {
     w.load_lds(slot, q >> 1, ph + 136 * PAR, 0);
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__((64 * GsGeo<DT, SWIGLU, MT, NSB, WM>::WAVES))
     __attribute__((amdgpu_waves_per_eu(GsGeo<DT, SWIGLU, MT, NSB, WM>::WPE)))
 k_gst(GemmArgs a, int W) {
     using G = GsGeo<DT, SWIGLU, MT, NSB, WM>;
-    using WT = std::conditional_t<DT == kQ4_K, VmQ4, WB<DT>>;
+    using WT = std::conditional_t<DT == kQ4_K, VmQ4, std::conditional_t<DT == kQ6_K, VmQ6, WB<DT>>>;
     constexpr int NI = G::NI, POS = G::POS, CPR = G::CPR, BLK = G::BLK, RUN = 16 * MT, OUT = G::OUT;
     constexpr int NMAT = SWIGLU ? 2 : 1;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // the stage buffers, two per wave
@@ -295,16 +295,18 @@ k_gst(GemmArgs a, int W) {
                 issue(buf);
                 auto half = [&](auto parc, WT &w) MX_INLINE_LAMBDA {
                     constexpr int PAR = decltype(parc)::value;
-                    if constexpr (DT != kQ4_K) w.template prep<PAR>(kh);
-#pragma unroll
-                    for (int P = 0; P < 4; P++) {
+                    if constexpr (DT == kQ6_K) w.prep(kh);
+                    else if constexpr (DT != kQ4_K) w.template prep<PAR>(kh);
+static_for<0, 4>([&](auto pc) MX_INLINE_LAMBDA {
+                        constexpr int P = decltype(pc)::value;
                         half8_t bf;
                         if constexpr (DT == kQ4_K) bf = w.step(P);
+                        else if constexpr (DT == kQ6_K) bf = w.template step<P>();
                         else bf = w.step(P, hh);
 #pragma unroll
                         for (int mt = 0; mt < MT; mt++)
                             acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][mt][4 * PAR + P], bf, acc[mt], 0, 0, 0);
-                    }
+                    });
                 };
                 half(std::integral_constant<int, 0>{}, w0);
                 half(std::integral_constant<int, 1>{}, w1);

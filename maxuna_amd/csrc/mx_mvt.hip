@@ -35,6 +35,7 @@
 // against 64 bits 2.4e-7 before, 1.2e-7 here.  One stage buffer per wave took 91 us.
 #include "mx_launch.h"
 #include "mx_dma.h"
+#include "mx_wb.h"
 
 namespace mx {
 namespace {
@@ -51,13 +52,6 @@ template <> struct MtBlk<kQ5_K> { static constexpr int BLK = 176, CPR = 11; };
 template <> struct MtBlk<kQ6_K> { static constexpr int BLK = 210, CPR = 15; };
 template <> struct MtBlk<kQ8_0> { static constexpr int BLK = 272, CPR = 19; };
 
-// the 8 bytes at an even LDS address
-__device__ __forceinline__ uint2 lds8_a2(const uint8_t *slot, uint32_t off) {
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(slot + (off & ~3u));
-    const uint32_t sh = (off & 2u) * 8u;
-    const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
-    return make_uint2(__builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh));
-}
 // f16 (1024 + byte) of bytes 0..3 of a and b, minus off (both exact)
 __device__ __forceinline__ half8_t bytes_f16(uint32_t a, uint32_t b, float off) {
     const half2_t o = {(_Float16)off, (_Float16)off};

@@ -214,7 +214,7 @@ k_vmm(VmmArgs a, const int32_t *__restrict__ perm, const int32_t *__restrict__ r
     __shared__ __attribute__((aligned(16))) uint8_t sB[2][VM_WAVES][G::BUF];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = lane & 15, q = lane >> 4, kh = q >> 1, hh = q & 1;
+    const int n = lane & 15, q = lane >> 4, kh = q >> 1;
     const int gw = blockIdx.x * VM_WAVES + wave, NW = gridDim.x * VM_WAVES;
     const int CB = a.n_out / COLS;
     const int n_items = runs[0] * CB;
@@ -249,7 +249,7 @@ k_vmm(VmmArgs a, const int32_t *__restrict__ perm, const int32_t *__restrict__ r
         wait_vmcnt(8 + G::NI);
         auto half = [&](auto parc) {
             constexpr int PAR = decltype(parc)::value;
-            using W = std::conditional_t<DT == kQ4_K, VmQ4, WB<DT>>;
+            using W = std::conditional_t<DT == kQ4_K, VmQ4, VmQ6>;
             W wb[G::NBLK];
 #pragma unroll
             for (int nb = 0; nb < G::NBLK; nb++) {
@@ -257,12 +257,12 @@ k_vmm(VmmArgs a, const int32_t *__restrict__ perm, const int32_t *__restrict__ r
                 if constexpr (DT == kQ4_K) {
                     wb[nb].template load<PAR>(slot, q);
                 } else {
-                    vm_load(wb[nb], slot, kh, (cur.rowpos[nb] + (uint32_t)(ks * G::BLK)) & 15u, PAR);
-                    wb[nb].template prep<PAR>(kh);
+                    wb[nb].template load<PAR>(slot, q, (cur.rowpos[nb] + (uint32_t)(ks * G::BLK)) & 15u);
+                    wb[nb].prep(kh);
                 }
             }
-#pragma unroll
-            for (int P = 0; P < 4; P++) {
+            static_for<0, 4>([&](auto pc) MX_INLINE_LAMBDA {
+                constexpr int P = decltype(pc)::value;
                 // every column block's weight operand first, then the MFMAs: no MFMA
                 // waits on the instruction just before it (hazard nops 214 -> 85 in the
                 // gate/up loop; C2 278.9 -> 276.6 us)
@@ -270,12 +270,12 @@ k_vmm(VmmArgs a, const int32_t *__restrict__ perm, const int32_t *__restrict__ r
 #pragma unroll
                 for (int nb = 0; nb < G::NBLK; nb++) {
                     if constexpr (DT == kQ4_K) bf[nb] = wb[nb].step(P);
-                    else bf[nb] = wb[nb].step(P, hh);
+                    else bf[nb] = wb[nb].template step<P>();
                 }
 #pragma unroll
                 for (int nb = 0; nb < G::NBLK; nb++)
                     acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 * PAR + P], bf[nb], acc[nb], 0, 0, 0);
-            }
+            });
         };
         half(std::integral_constant<int, 0>{});
         half(std::integral_constant<int, 1>{});

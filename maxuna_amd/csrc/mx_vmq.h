@@ -9,21 +9,43 @@
 namespace mx {
 namespace {
 
-// Q6_K half super-block `par` of the lane's row from its stage slot (the whole
-// block, from the 16-byte-aligned address below it; m1 = the block's phase):
-// the registers WB<kQ6_K>::load_lds fills from the prefill GEMM's per-half slots.
-__device__ __forceinline__ void vm_load(WB<kQ6_K> &w, const uint8_t *slot, int kh, uint32_t m1, int par) {
-    w.lo = lds16_a2(slot, m1 + 64 * par + 16 * kh);       // ql[64 par + 16 kh, +16)
-    w.hi = lds16_a2(slot, m1 + 64 * par + 32 + 16 * kh);  // ql[64 par + 32 + 16 kh, +16)
-    w.qh = lds16_a2(slot, m1 + 128 + 32 * par + 16 * kh); // qh[32 par + 16 kh, +16)
-    const uint32_t so = m1 + 192 + 8 * par;               // scales[8 par, +8)
-    const uint32_t *p = reinterpret_cast<const uint32_t *>(slot + (so & ~3u));
-    const uint32_t sh = (so & 2u) * 8u;
-    const uint32_t a0 = p[0], a1 = p[1], a2 = p[2];
-    w.s0 = __builtin_amdgcn_alignbit(a1, a0, sh);
-    w.s1 = __builtin_amdgcn_alignbit(a2, a1, sh);
-    w.dbits = *reinterpret_cast<const uint16_t *>(slot + m1 + 208);
-}
+// Q6_K half super-block PAR of the lane's row from its slot (the block's span from
+// the 16-byte-aligned address below it; ph = the block's phase): 8 bytes of each
+// field, the lane's values 32 P + 8 q + [0, 8) of step P (part P of the half).  The
+// same weights as WB<kQ6_K>, whose lanes hold 16 bytes of a field for the 32 x 32
+// layout: here half of them would be read, shifted and selected away (the Q6_K
+// verify tiles 116 -> 108 us in a 16-token block of hidden 4096, ff 1536; mx_gst.hip at 512
+// tokens 478 -> 437).
+struct VmQ6 {
+    uint2 lo, hi, qh;   // ql[64 PAR + 8 q, +8), ql[64 PAR + 32 + 8 q, +8), qh[32 PAR + 8 q, +8)
+    uint2 sc;           // scales[8 PAR, +8)
+    uint32_t d;
+    float d1[4], c1[4]; // d * sc and -1056 * d * sc of the lane's 16-value group of each part
+    template <int PAR> __device__ __forceinline__ void load(const uint8_t *slot, int q, uint32_t ph) {
+        lo = lds8_a2(slot, ph + 64 * PAR + 8 * q);
+        hi = lds8_a2(slot, ph + 64 * PAR + 32 + 8 * q);
+        qh = lds8_a2(slot, ph + 128 + 32 * PAR + 8 * q);
+        sc = lds8_a2(slot, ph + 192 + 8 * PAR);
+        d = *reinterpret_cast<const uint16_t *>(slot + ph + 208);
+    }
+    __device__ __forceinline__ void prep(int kh) {
+        const float df = h2f((uint16_t)d);
+#pragma unroll
+        for (int p = 0; p < 4; p++) {  // scale 8 PAR + 2 p + kh
+            const uint32_t word = p < 2 ? sc.x : sc.y;
+            d1[p] = df * (float)(int)__builtin_amdgcn_sbfe((int)word, 16 * (p & 1) + 8 * kh, 8);
+            c1[p] = -1056.0f * d1[p];
+        }
+    }
+    template <int P> __device__ __forceinline__ half8_t step() const {
+        constexpr int S = 4 * (P >> 1);
+        const uint2 v = (P & 1) ? hi : lo;
+        auto top = [](uint32_t w) {
+            return P < 2 ? (w << (4 - 2 * P)) & 0x30303030u : P == 2 ? w & 0x30303030u : (w >> 2) & 0x30303030u;
+        };
+        return dq8_q6(((v.x >> S) & 0x0F0F0F0Fu) | top(qh.x), ((v.y >> S) & 0x0F0F0F0Fu) | top(qh.y), d1[P], c1[P]);
+    }
+};
 
 // Q4_K half super-block `PAR` of the lane's row for the sub-block-per-lane
 // order: sub-block j = 4 PAR + q (32 values, one 6-bit scale and min).  Word i of

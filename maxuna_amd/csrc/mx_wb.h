@@ -232,6 +232,14 @@ __device__ __forceinline__ uint4 lds16_a2(const uint8_t *slot, uint32_t off) {
                       __builtin_amdgcn_alignbit(d3, d2, sh), __builtin_amdgcn_alignbit(d4, d3, sh));
 }
 
+// the 8 bytes at an even LDS address
+__device__ __forceinline__ uint2 lds8_a2(const uint8_t *slot, uint32_t off) {
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(slot + (off & ~3u));
+    const uint32_t sh = (off & 2u) * 8u;
+    const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
+    return make_uint2(__builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh));
+}
+
 // Q6_K: stage = half n = par of super-block ks / 2 (128 values).  Lane half kh
 // holds ql[64n + 16kh, +16), ql[64n + 32 + 16kh, +16), qh[32n + 16kh, +16);
 // step p takes the 4-bit part from the low (p even) / high (p odd) ql piece,
