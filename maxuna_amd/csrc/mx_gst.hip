@@ -382,12 +382,24 @@ template <int DT, bool SWIGLU> void gs_launch(const GemmArgs &a, hipStream_t s) 
 }
 }  // namespace
 
-// Pairs per expert up to which they are the faster (µs, grouped GEMM against these):
-// hidden 3072, ff 1024 layers of 10 pairs per expert 499 / 391, 17: 522 / 472, 26: 613
-// / 602, 40: 697 / 788; Q8_0 hidden 3072, ff 2048 of 6: 359 / 270; Q6_K / Q4_K hidden
-// 6144, ff 2816 of 16: 968 / 812.  K above 4096 leaves registers for runs of 16 pairs
-// only: hidden 7168, ff 2048 of 1.3 pairs 813 / 572, 3: 851 / 715, 6: 976 / 980.
-constexpr int64_t GST_PAIRS = 24, GST_PAIRS_WIDE = 6;
+// Pairs per expert up to which they are taken.  Measured (µs, the other route -- the
+// grouped GEMM, or up to 2560 pairs of Q4_K / Q6_K the verify tiles -- against these;
+// 64 experts evenly used, top-4): plain [4096 x 1536] Q4_K of 24 pairs per expert 148 /
+// 107, 56: 160 / 162; Q5_K 12: 118 / 97, 24: 122 / 115, 36: 130 / 142; Q6_K 24: 173 /
+// 121, 56: 190 / 204; Q8_0 12: 139 / 125, 24: 146 / 147; layers (SwiGLU) of hidden 3072,
+// ff 1536 Q4_K 24: 290 / 239, 40: 299 / 304; Q5_K 24: 355 / 286, 40: 370 / 369; Q6_K 40:
+// 482 / 392; Q8_0 24: 418 / 355, 40: 440 / 463.  Unevenly used experts cut into more
+// runs (hidden 3072, ff 1024, 256 experts, a skewed router, Q4_K / Q6_K: 17 pairs 522 /
+// 472, 26: 613 / 605), so the lines lie below those crossings.  Beyond K = 4096 a run is
+// 16 pairs: half of them to 6144 (hidden 6144 Q4_K of 24: 530 / 469, Q6_K 12: 673 / 442,
+// Q8_0 12: 615 / 483), a quarter beyond (hidden 7168 Q4_K of 7: 535 / 344, skewed over
+// 256 experts of 6: 976 / 980; Q6_K 12: 729 / 529).
+int64_t gst_pairs(int dtype, bool swiglu, int k) {
+    int64_t p;
+    if (swiglu) p = dtype == kQ6_K ? 40 : 24;
+    else p = dtype == kQ4_K ? 30 : dtype == kQ6_K ? 36 : dtype == kQ5_K ? 18 : 16;
+    return k <= 4096 ? p : k <= 6144 ? p / 2 : p / 4;
+}
 bool gst_fits(int dtype, const GemmArgs &a, bool swiglu) {
     auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool sh = a.w_sh[0] != nullptr;
@@ -395,9 +407,7 @@ bool gst_fits(int dtype, const GemmArgs &a, bool swiglu) {
               a.row_bytes < (1 << 24) && (!sh || a.sh_row_bytes == a.row_bytes);
     for (int m = 0; m < (swiglu ? 2 : 1); m++)
         ok = ok && (a.n_expert == 0 || (al(a.w[m]) && a.expert_bytes % 16 == 0)) && (!sh || al(a.w_sh[m]));
-    (void)dtype;
-    const int64_t few = a.k / 256 <= 16 ? GST_PAIRS : GST_PAIRS_WIDE;
-    return ok && (int64_t)a.t * a.top_k < few * a.n_map_expert;
+    return ok && (int64_t)a.t * a.top_k < gst_pairs(dtype, swiglu, a.k) * a.n_map_expert;
 }
 
 mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s) {
