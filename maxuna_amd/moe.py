@@ -106,6 +106,8 @@ class MoeBlock:
         self.rms_eps = rms_eps
         self._ws = None
         self._c = self._layer_struct()
+        self._ref = C.byref(self._c)
+        self._need = {}  # workspace bytes by token count (a function of the struct)
 
     @property
     def hidden(self) -> int:
@@ -126,7 +128,9 @@ class MoeBlock:
             float(self.rms_eps), 0)
 
     def workspace(self, t: int, device) -> torch.Tensor:
-        need = lib().mx_moe_workspace_bytes(C.byref(self._c), t)
+        need = self._need.get(t)
+        if need is None:
+            need = self._need[t] = lib().mx_moe_workspace_bytes(self._ref, t)
         if self._ws is None or self._ws.numel() < need:
             # no state lives in the workspace between calls (every forward
             # initialises what it reads); zeroed only for tidiness
@@ -147,14 +151,17 @@ class MoeBlock:
         t = x.shape[0]
         if out is None:
             out = torch.empty_like(x)
-        ids = torch.empty((t, self.cfg.n_expert_used), dtype=torch.uint32, device=x.device)
-        w = torch.empty((t, self.cfg.n_expert_used), dtype=torch.float32, device=x.device)
+        ids, w = self._routing(t, x.device) if return_routing else (None, None)
         ws = self.workspace(t, x.device)
-        check(lib().mx_moe_forward(C.byref(self._c), x.data_ptr(), t,
-                                   residual.data_ptr() if residual is not None else None,
-                                   out.data_ptr(), ids.data_ptr(), w.data_ptr(), ws.data_ptr(),
-                                   ws.numel(), ops._stream()))
+        check(lib().mx_moe_forward(self._ref, x.data_ptr(), t, ops._ptr(residual), out.data_ptr(), ops._ptr(ids),
+                                   ops._ptr(w), ws.data_ptr(), ws.numel(), ops._stream()))
         return (out, ids, w) if return_routing else out
+
+    def _routing(self, t: int, device):
+        """Outputs for the routing decision (without them it stays in the workspace)."""
+        k = self.cfg.n_expert_used
+        return (torch.empty((t, k), dtype=torch.uint32, device=device),
+                torch.empty((t, k), dtype=torch.float32, device=device))
 
     def forward_noalloc(self, x: torch.Tensor, residual: torch.Tensor | None = None,
                         out: torch.Tensor | None = None, return_routing: bool = False):
@@ -167,9 +174,7 @@ class MoeBlock:
         t = x.shape[0]
         if out is None:
             out = torch.empty_like(x)
-        ids = torch.empty((t, self.cfg.n_expert_used), dtype=torch.uint32, device=x.device)
-        w = torch.empty((t, self.cfg.n_expert_used), dtype=torch.float32, device=x.device)
-        check(lib().mx_moe_forward_noalloc(C.byref(self._c), x.data_ptr(), t,
-                                           residual.data_ptr() if residual is not None else None,
-                                           out.data_ptr(), ids.data_ptr(), w.data_ptr(), ops._stream()))
+        ids, w = self._routing(t, x.device) if return_routing else (None, None)
+        check(lib().mx_moe_forward_noalloc(self._ref, x.data_ptr(), t, ops._ptr(residual), out.data_ptr(),
+                                           ops._ptr(ids), ops._ptr(w), ops._stream()))
         return (out, ids, w) if return_routing else out

@@ -43,8 +43,16 @@ def no_mm_id() -> bool:
     return "LAGUNA_NO_MM_ID" in os.environ
 
 
-def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# the current stream's handle without building a Stream object (a call of a small op
+# is bound by its host side); builds without a GPU have no such function
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream() -> int:
+    """Handle of the current device's current stream."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
