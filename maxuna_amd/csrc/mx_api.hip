@@ -229,7 +229,7 @@ mx_status pool_alloc(size_t bytes, hipStream_t s, void **out) {
 
 // bytes of x's f16 rows and their scales for the GEMM route
 size_t mm_x16_bytes(int64_t t, int64_t x_per_row, int64_t k) {
-    return (((size_t)(t * x_per_row * k) * 2 + 255) & ~size_t(255)) + (size_t)(t * x_per_row) * 4;
+    return (((size_t)(t * x_per_row * k) * 2 + 255) & ~size_t(255)) + (size_t)(t * x_per_row) * 4 + 4;
 }
 // the tiles route: the pair order (perm, then its runs: the tiles read 16 words
 // from a run's start, which stay inside the runs table), then x's f16 rows
@@ -248,7 +248,7 @@ GemmArgs mm_args(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64
     return a;
 }
 bool mm_on_gst(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64_t top_k) {
-    return gst_fits(st->dtype, mm_args(st, g, t, top_k), false);
+    return gst_fits(mm_args(st, g, t, top_k), false);
 }
 // A few pairs per expert: the 16-pair MFMA tiles of the verify blocks (each
 // touched expert's weights streamed once) instead of 128-pair GEMM m-tiles
@@ -313,12 +313,12 @@ mx_status mm_gemm(const mx_expert_stack *st, const StackGeom &g, const float *x,
     a.map = map;
     a.out = dst;
     const bool gst = mm_on_gst(st, g, t, top_k);
-    const bool perm = gst && st->dtype == kQ4_K;
+    a.done = gst ? reinterpret_cast<int32_t *>(x16s + t * x_per_row) : nullptr;  // (the last word of tmp)
     if (by_pair)
-        MX_TRY(launch_to_f16_rows(x, t * top_k, k, map + L.off + st->n_expert, x16, x16s, s, perm, map + L.list));
+        MX_TRY(launch_to_f16_rows(x, t * top_k, k, map + L.off + st->n_expert, x16, x16s, s, false, map + L.list));
     else
-        MX_TRY(launch_to_f16_rows(x, t, k, nullptr, x16, x16s, s, perm));
-    if (gst) return launch_gst(st->dtype, false, a, s);
+        MX_TRY(launch_to_f16_rows(x, t, k, nullptr, x16, x16s, s));
+    if (gst) MX_TRY(launch_gst(st->dtype, false, a, s));
     return launch_gemm(st->dtype, false, a, s);
 }
 }  // namespace
@@ -520,9 +520,9 @@ void plan_gst(const mx_moe_layer *L, int64_t t, Plan &p) {
     };
     set(L->up, L->shared_up, 1);
     set(L->gate, L->shared_gate, 0);
-    p.gst_gu = gst_fits(L->gate.dtype, a, true);
+    p.gst_gu = gst_fits(a, true);
     set(L->down, L->shared_down, 0);
-    p.gst_d = gst_fits(L->down.dtype, a, false);
+    p.gst_d = gst_fits(a, false);
 }
 
 // Chooses the kernels of a forward; every shape limit of the chosen kernels is
@@ -581,7 +581,7 @@ struct Layout {
     int32_t *runs = nullptr;  // their 16-pair runs (MFMA verify tiles)
     uint8_t *xstage = nullptr, *xstage_gm = nullptr;
     float *part = nullptr;
-    int32_t *map = nullptr, *map_sh = nullptr;
+    int32_t *map = nullptr, *map_sh = nullptr, *done = nullptr;
     _Float16 *x16 = nullptr, *act16 = nullptr;
     float *x16s = nullptr, *act16s = nullptr, *down = nullptr, *act_u = nullptr;
     float *sh_g = nullptr, *sh_u = nullptr, *sh_out = nullptr;
@@ -639,6 +639,7 @@ Layout carve(const mx_moe_layer *L, int64_t t, const Plan &p, void *base) {
         const int64_t EM = E + (p.shared_in_decode ? 1 : 0);
         const int64_t KM = K + (p.shared_in_decode ? 1 : 0);
         o.map = ws.take<int32_t>(map0_bytes((int)EM, (int)t, (int)KM) / 4);
+        o.done = ws.take<int32_t>(1);
         if (p.has_shared && !p.shared_in_decode) {
             o.map_sh = ws.take<int32_t>(map0_bytes(1, (int)t, 1) / 4);
             o.zero_ids = ws.take<uint32_t>(t);
@@ -934,9 +935,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         }
     }
     MX_STAGE();
-    // (the stationary-activation Q4_K matmuls read A in the verify tiles' K order)
-    const bool gst_gu = p.gst_gu, gst_d = p.gst_d;
-    MX_TRY(launch_to_f16_rows(xin, t, (int)H, nullptr, o.x16, o.x16s, s, gst_gu && L->gate.dtype == kQ4_K));
+    MX_TRY(launch_to_f16_rows(xin, t, (int)H, nullptr, o.x16, o.x16s, s));
     MX_STAGE();
     // one bucket map's gate+up (SwiGLU, act rows at its bucket positions from act_row0 on)
     // and down (rows token * KK + slot + out_add)
@@ -954,10 +953,12 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         ga.a = o.x16; ga.a_scale = o.x16s; ga.a_div = top_k;
         ga.t = (int)t; ga.top_k = top_k; ga.n_map_expert = n_map_expert; ga.map = map;
         ga.out = o.act + act_row0 * FF;
-        MX_TRY(gst_gu ? launch_gst(dt_gu, true, ga, s) : launch_gemm(dt_gu, true, ga, s));
+        ga.done = p.gst_gu ? o.done : nullptr;
+        if (p.gst_gu) MX_TRY(launch_gst(dt_gu, true, ga, s));
+        MX_TRY(launch_gemm(dt_gu, true, ga, s));
         MX_STAGE();
         MX_TRY(launch_to_f16_rows(ga.out, t * top_k, (int)FF, map + LM.off + n_map_expert,
-                                  o.act16 + act_row0 * FF, o.act16s + act_row0, s, gst_d && dt_d == kQ4_K));
+                                  o.act16 + act_row0 * FF, o.act16s + act_row0, s));
         MX_STAGE();
         GemmArgs da = ga;
         da.w[0] = wd; da.w[1] = nullptr;
@@ -966,7 +967,9 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         da.n_out = (int)H; da.k = (int)FF;
         da.a = o.act16 + act_row0 * FF; da.a_scale = o.act16s + act_row0; da.a_div = 0;
         da.out = o.down; da.out_stride = KK; da.out_add = out_add;
-        MX_TRY(gst_d ? launch_gst(dt_d, false, da, s) : launch_gemm(dt_d, false, da, s));
+        da.done = p.gst_d ? o.done : nullptr;
+        if (p.gst_d) MX_TRY(launch_gst(dt_d, false, da, s));
+        MX_TRY(launch_gemm(dt_d, false, da, s));
         MX_STAGE();
         return MX_OK;
     };

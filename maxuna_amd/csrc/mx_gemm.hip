@@ -180,6 +180,7 @@ __global__ void __launch_bounds__((64 * GemmNb<DT, SWIGLU>::waves))
     __shared__ int s_out[GM_BM];      // output row
     constexpr int NCOL = SWIGLU ? BROWS / 2 : BROWS;
     const int nt_count = (a.n_out + NCOL - 1) / NCOL;
+    if (a.done && *a.done) return;  // (k_gst took the launch)
     Tile tl;
     if (!tile_of(a, nt_count, tl)) return;
     const int tid = threadIdx.x, lane = tid & 63;

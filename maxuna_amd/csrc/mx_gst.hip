@@ -14,6 +14,9 @@
 // the grouped GEMM (the f16 rounding of the f32 value, mx_wb.h); A rows are f16
 // times a power of two per row; sums are f32.
 //
+//  * Which launches: those with few runs for their m-tiles of 128 pairs, decided from
+//    the map by every workgroup alike (gs_ratio); the grouped GEMM launched next reads
+//    the answer and leaves or does the work.
 //  * Work: the runs of all experts (each expert's bucket cut into 16 * MT pairs)
 //    times the row tiles, cut into one contiguous share per resident workgroup:
 //    a workgroup loads a run's activations once per share and run.  The map gives
@@ -71,6 +74,17 @@ template <int PAR> __device__ __forceinline__ void gs_load(WB<kQ8_0> &w, const u
     w.load_lds(slot, q >> 1, ph + 136 * PAR, 0);
 }
 
+// Ten times the most runs per m-tile of the map at which a launch is taken.  The
+// average of pairs per expert, all the host knows, does not tell: with a router that
+// uses a quarter of 256 experts (hidden 4096, ff 1536, Q4_K / Q6_K) 12 pairs on average
+// took 422 us in the grouped GEMM and 461 here, 20: 485 / 662; evenly used experts of 24
+// pairs 290 / 239, of 40 (1.9 runs per m-tile) 299 / 304.  By type, from even use: plain
+// [4096 x 1536] Q5_K of 24 pairs 122 / 115, 36: 130 / 142; Q6_K 36: 185 / 145; Q8_0 24:
+// 146 / 147; SwiGLU hidden 3072 Q6_K of 40: 482 / 392, Q8_0 440 / 463.
+__host__ __device__ constexpr int gs_ratio(int dtype, bool swiglu) {
+    return dtype == kQ6_K ? (swiglu ? 22 : 18) : dtype == kQ4_K ? 16 : swiglu ? 15 : 13;
+}
+
 template <int DT, bool SWIGLU, int MT, int NSB, int WM> struct GsGeo {
     static constexpr int CPR = GsBlk<DT>::CPR, BLK = GsBlk<DT>::BLK, SLOT = 16 * CPR;
     static constexpr int POS = 16 * CPR, NI = (POS + 63) / 64, STAGE = POS * 16;
@@ -117,8 +131,11 @@ k_gst(GemmArgs a, int W) {
     // ---- the runs of every expert: exclusive prefix ---------------------------------
     {
         const int per = (E + BT - 1) / BT, e0 = min(tid * per, E), e1 = min(e0 + per, E);
-        int sum = 0;
-        for (int e = e0; e < e1; e++) sum += (a.map[L.tpe + e] + RUN - 1) / RUN;
+        int sum = 0;  // runs, and m-tiles of 128 pairs in the upper half (both below 2^15: gst_fits)
+        for (int e = e0; e < e1; e++) {
+            const int v = a.map[L.tpe + e];
+            sum += (v + RUN - 1) / RUN + ((v + GM_BM - 1) / GM_BM << 16);
+        }
         int inc = sum;  // inclusive scan over the wave's lanes
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -127,17 +144,22 @@ k_gst(GemmArgs a, int W) {
         }
         if (lane == 63) sScan[gwave] = inc;
         __syncthreads();
-        int base = inc - sum;
-        for (int w = 0; w < gwave; w++) base += sScan[w];
+        int base0 = 0;
+        for (int w = 0; w < gwave; w++) base0 += sScan[w];
+        int base = base0 + inc - sum;
         for (int e = e0; e < e1; e++) {
-            sRuns[e] = base;
+            sRuns[e] = base & 0xFFFF;
             base += (a.map[L.tpe + e] + RUN - 1) / RUN;
         }
-        if (tid == BT - 1) sRuns[E] = base;
+        if (tid == BT - 1) sRuns[E] = (base & 0xFFFF) | (int)((uint32_t)(inc + base0) & 0xFFFF0000u);
         for (int i = tid; i < 2 * TEAMS * WM * OUT; i += BT) (&sRed[0][0][0][0])[i] = 0.f;
         __syncthreads();
     }
-    const int runs = __builtin_amdgcn_readfirstlane(sRuns[E]);
+    // many runs for their m-tiles: the grouped GEMM is the faster (block-uniform)
+    const int both = __builtin_amdgcn_readfirstlane(sRuns[E]), runs = both & 0xFFFF;
+    const bool mine = 10 * runs < gs_ratio(DT, SWIGLU) * (both >> 16);
+    if (blockIdx.x == 0 && tid == 0) *a.done = mine;
+    if (!mine) return;
     const int tiles = a.n_out / 16;
     // this workgroup's share [u0, u1) of the runs * tiles units; neighbouring shares on
     // one XCD (workgroups are dealt to the 8 XCDs round-robin)
@@ -245,7 +267,12 @@ k_gst(GemmArgs a, int W) {
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                for (int i = 0; i < 8; i++) asm volatile("" : "+v"(A[s][mt][i]));
+                for (int i = 0; i < 8; i++) {
+                    asm volatile("" : "+v"(A[s][mt][i]));
+                    // (VmQ4's weights come in the order 0, 2, 1, 3 of each four)
+                    if constexpr (DT == kQ4_K)
+                        A[s][mt][i] = __builtin_shufflevector(A[s][mt][i], A[s][mt][i], 0, 2, 1, 3, 4, 6, 5, 7);
+                }
         tab ^= 1;
         for (int m = tid; m < RUN; m += BT) {
             const int pos = pos0 + min(m, rows - 1);
@@ -382,32 +409,18 @@ template <int DT, bool SWIGLU> void gs_launch(const GemmArgs &a, hipStream_t s) 
 }
 }  // namespace
 
-// Pairs per expert up to which they are taken.  Measured (µs, the other route -- the
-// grouped GEMM, or up to 2560 pairs of Q4_K / Q6_K the verify tiles -- against these;
-// 64 experts evenly used, top-4): plain [4096 x 1536] Q4_K of 24 pairs per expert 148 /
-// 107, 56: 160 / 162; Q5_K 12: 118 / 97, 24: 122 / 115, 36: 130 / 142; Q6_K 24: 173 /
-// 121, 56: 190 / 204; Q8_0 12: 139 / 125, 24: 146 / 147; layers (SwiGLU) of hidden 3072,
-// ff 1536 Q4_K 24: 290 / 239, 40: 299 / 304; Q5_K 24: 355 / 286, 40: 370 / 369; Q6_K 40:
-// 482 / 392; Q8_0 24: 418 / 355, 40: 440 / 463.  Unevenly used experts cut into more
-// runs (hidden 3072, ff 1024, 256 experts, a skewed router, Q4_K / Q6_K: 17 pairs 522 /
-// 472, 26: 613 / 605), so the lines lie below those crossings.  Beyond K = 4096 a run is
-// 16 pairs: half of them to 6144 (hidden 6144 Q4_K of 24: 530 / 469, Q6_K 12: 673 / 442,
-// Q8_0 12: 615 / 483), a quarter beyond (hidden 7168 Q4_K of 7: 535 / 344, skewed over
-// 256 experts of 6: 976 / 980; Q6_K 12: 729 / 529).
-int64_t gst_pairs(int dtype, bool swiglu, int k) {
-    int64_t p;
-    if (swiglu) p = dtype == kQ6_K ? 40 : 24;
-    else p = dtype == kQ4_K ? 30 : dtype == kQ6_K ? 36 : dtype == kQ5_K ? 18 : 16;
-    return k <= 4096 ? p : k <= 6144 ? p / 2 : p / 4;
-}
-bool gst_fits(int dtype, const GemmArgs &a, bool swiglu) {
+bool gst_fits(const GemmArgs &a, bool swiglu) {
     auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool sh = a.w_sh[0] != nullptr;
     bool ok = a.k % 256 == 0 && a.k / 256 >= 2 && a.k / 256 <= 32 && a.n_out % 16 == 0 && a.n_map_expert < GS_MAX_E &&
               a.row_bytes < (1 << 24) && (!sh || a.sh_row_bytes == a.row_bytes);
     for (int m = 0; m < (swiglu ? 2 : 1); m++)
         ok = ok && (a.n_expert == 0 || (al(a.w[m]) && a.expert_bytes % 16 == 0)) && (!sh || al(a.w_sh[m]));
-    return ok && (int64_t)a.t * a.top_k < gst_pairs(dtype, swiglu, a.k) * a.n_map_expert;
+    // Less than one run (32 pairs, 16 beyond K = 4096) per expert on average: what the
+    // kernel then leaves to the grouped GEMM cost its launch, 3 to 4 us per matmul (2 to
+    // 3% of a layer of 64 to 256 experts under a skewed router); what it takes gained
+    // 1.08 (27 pairs) to 1.3x (12 pairs).
+    return ok && (int64_t)a.t * a.top_k < (a.k <= 4096 ? 32 : 16) * (int64_t)a.n_map_expert;
 }
 
 mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s) {

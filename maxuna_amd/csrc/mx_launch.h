@@ -252,6 +252,7 @@ struct GemmArgs {
     float *out;                 // SwiGLU: act [position, n_out]; plain: rows
                                 // (pair / top_k) * out_stride + pair % top_k + out_add
     int out_stride, out_add;
+    int32_t *done;              // NULL, or the word launch_gst set: not 0, the launch is done
 };
 bool gemm_supported(int dtype, int k);
 // the kernel's 32-bit operand offsets hold for t tokens of x [t, hidden] and
@@ -260,8 +261,9 @@ bool gemm_fits(int t, int hidden, int ff, int64_t gu_row_bytes, int64_t d_row_by
 // the same for one plain GEMM over a_rows A rows addressed by pair (a_div > 0)
 bool gemm_plain_fits(int64_t a_rows, int k, int n_out, int64_t row_bytes);
 // mx_gst.hip -- the same contraction for a few dozen pairs per expert (activations
-// stationary).  Q4_K: A rows in the verify tiles' K order (launch_to_f16_rows perm).
-bool gst_fits(int dtype, const GemmArgs &a, bool swiglu);
+// stationary).  It takes the launch only where the map's runs are few for its m-tiles
+// and says so in *a.done; launch_gemm with the same a follows and leaves when *a.done.
+bool gst_fits(const GemmArgs &a, bool swiglu);
 mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 mx_status launch_gemm(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 // rows of x (f32, [rows, k], k % 4 == 0) -> f16 times a per-row power of two;

@@ -153,8 +153,8 @@ def test_few_pairs_per_expert(orc, gate, down, hidden, ff):
     routing.  f16 operands: the contract's bound."""
     spec = LayerSpec(hidden, ff, 40, 4, GgmlDType[gate], GgmlDType[down], shared=hidden % 512 == 0, bias_sigma=0.3)
     layer = build_layer(spec, seed=4600)
-    # past the verify tiles' pairs where the types have tiles, and under the 24 (K up to
-    # 4096) or 6 pairs per expert that these matmuls take
+    # past the verify tiles' pairs where the types have tiles, and under the 32 (K up to
+    # 4096) or 16 pairs per expert up to which these matmuls are tried
     x = make_x(spec, 4601, 50 if hidden > 4096 else 210 if gate == "Q4_K" else 70)
     out, ids, w = layer.block.forward(torch.from_numpy(x).cuda(), return_routing=True)
     out, ids, w = host(out), host(ids), host(w)
@@ -175,3 +175,18 @@ def test_few_pairs_per_expert_alignment_rule(orc):
     x = dev_f32(rng.standard_normal((t, 1, k)).astype(np.float32))
     a, b = host(ops.mul_mm_id(st, x, ids)), host(ops.mul_mm_id(off, x, ids))
     assert rel_l2(a, b) <= 1e-6  # (the same products in another order of summation)
+
+
+@pytest.mark.parametrize("dt", ["Q4_K", "Q5_K", "Q6_K", "Q8_0"])
+def test_few_pairs_on_average_many_in_use(orc, dt):
+    """12 pairs per expert on average, but 400 on each of two experts: the grouped GEMM
+    does the work after the other kernel left it, with the same bits as at an expert count
+    whose average sends it there at once."""
+    rng = np.random.default_rng(9)
+    t, top_k, n_out, k = 400, 2, 512, 768
+    st = synth_stack(GgmlDType[dt], 64, n_out, k, tensor_key(4800, 0, 1))
+    few = ExpertStack(st.buffer, GgmlDType[dt], 3, n_out, k)
+    ids = dev_u32(np.argsort(rng.random((t, 2)), axis=1))
+    x = dev_f32(rng.standard_normal((t, 1, k)).astype(np.float32))
+    a, b = host(ops.mul_mm_id(st, x, ids)), host(ops.mul_mm_id(few, x, ids))
+    assert np.array_equal(a, b)
