@@ -393,13 +393,17 @@ template <int DT, bool SWIGLU, int MT, int NSB, int WM> void gs_go(const GemmArg
 template <int DT, bool SWIGLU> void gs_launch(const GemmArgs &a, hipStream_t s) {
     const int nsb = a.k / 256;
     if constexpr (DT == kQ8_0) {  // (its raw words spill at 168 registers next to two pair tiles)
-        if (nsb <= 2) return gs_go<DT, SWIGLU, 1, 1, 2>(a, s);
-        if (nsb <= 4) return gs_go<DT, SWIGLU, 1, 1, 4>(a, s);
+        if constexpr (!SWIGLU) {  // (gst_fits)
+            if (nsb <= 2) return gs_go<DT, SWIGLU, 1, 1, 2>(a, s);
+            if (nsb <= 4) return gs_go<DT, SWIGLU, 1, 1, 4>(a, s);
+        }
         if (nsb <= 8) return gs_go<DT, SWIGLU, 2, 2, 4>(a, s);
         if (nsb <= 12) return gs_go<DT, SWIGLU, 2, 2, 6>(a, s);
     } else {
-        if (nsb <= 2) return gs_go<DT, SWIGLU, 2, 1, 2>(a, s);
-        if (nsb <= 4) return gs_go<DT, SWIGLU, 2, 1, 4>(a, s);
+        if constexpr (!SWIGLU) {
+            if (nsb <= 2) return gs_go<DT, SWIGLU, 2, 1, 2>(a, s);
+            if (nsb <= 4) return gs_go<DT, SWIGLU, 2, 1, 4>(a, s);
+        }
         if (nsb <= 6) return gs_go<DT, SWIGLU, 2, 1, 6>(a, s);
         if (nsb <= 12) return gs_go<DT, SWIGLU, 2, 1, 12>(a, s);
     }
@@ -416,6 +420,9 @@ bool gst_fits(const GemmArgs &a, bool swiglu) {
               a.row_bytes < (1 << 24) && (!sh || a.sh_row_bytes == a.row_bytes);
     for (int m = 0; m < (swiglu ? 2 : 1); m++)
         ok = ok && (a.n_expert == 0 || (al(a.w[m]) && a.expert_bytes % 16 == 0)) && (!sh || al(a.w_sh[m]));
+    // Gate/up of K up to 1024 stay on the grouped GEMM: a layer of hidden 1024, ff 512, 64
+    // experts, Q6_K / Q4_K, took 92 us there, 101 with both projections here and 96 with the down alone (28 pairs).
+    ok = ok && (!swiglu || a.k > 1024);
     // Less than one run (32 pairs, 16 beyond K = 4096) per expert on average: what the
     // kernel then leaves to the grouped GEMM cost its launch, 3 to 4 us per matmul (2 to
     // 3% of a layer of 64 to 256 experts under a skewed router); what it takes gained

@@ -137,7 +137,8 @@ def test_mul_mv_tokens_ranges(orc):
 
 # (gate/up type, down type, hidden, ff): super-blocks of K at the ends of the wave
 # layouts of the stationary-activation matmuls (2 | 4 | 6 | 12 waves of one, 8 of two,
-# then three and four), each type on both projections
+# then three and four), each type on both projections; gate/up of up to four
+# super-blocks run the grouped GEMM
 GST = [
     ("Q4_K", "Q4_K", 512, 768), ("Q4_K", "Q6_K", 1280, 1536), ("Q4_K", "Q6_K", 3072, 1792), ("Q4_K", "Q4_K", 3328, 1024),
     ("Q4_K", "Q5_K", 4352, 512), ("Q4_K", "Q6_K", 6400, 512), ("Q5_K", "Q5_K", 1024, 2304), ("Q5_K", "Q6_K", 4096, 1280),
