@@ -758,18 +758,26 @@ static mx_status launch_mv_q6(const MvArgs &a, int ng, int p, hipStream_t s) {
 }
 
 // ---- shape fits of the LDS-ring kernels (host) --------------------------------------
-// Each kernel holds NG <= NG_MAX activation groups per lane, copies a batch of rows
-// with at most DMA_MAX_INSTS wave instructions per matrix set, and needs its LDS.
+// Each kernel holds at most G_MAX groups per row, copies a row (a gate and an up row)
+// with at most DMA_MAX_INSTS wave instructions, and needs its LDS.
 template <int DT> static int64_t row_bytes_of(int k) { return (int64_t)(k / block_size(DT)) * type_size(DT); }
-template <int DT> static bool mv_fits_dt(int k) {
+// Down rows: the act row and one batch of every wave in LDS.  Q4_K / Q5_K rows whose
+// group count is seven times a power of two (k = 1792, 3584, 7168, 14336) stay on the
+// f32 mat-vec, which holds every activation in f32 (Q4_K [50000 x 3584] against 64
+// bits: 1.5e-7; the block grid 2.7e-7, and without bound where a block's largest value
+// meets small weights); it has always had them, and so have the layers built on it.
+template <int DT> static bool row_fits(int k) {
     const int G = groups<DT>(k);
     if (k <= 0 || k % block_size(DT) || G > G_MAX) return false;
-    // Q4_K / Q5_K rows of 28 and 56 groups (k = 1792, 3584) keep the f32 mat-vec: it
-    // is what they have always had, and its error is the smaller (Q4_K [50000 x
-    // 3584]: 1.5e-7 against 2.7e-7 with the activation grid)
-    if ((DT == kQ4_K || DT == kQ5_K) && (G == 28 || G == 56)) return false;
+    if ((DT == kQ4_K || DT == kQ5_K) && G / (G & -G) == 7) return false;
     return dma_insts(1, 1, row_bytes_of<DT>(k)) <= DMA_MAX_INSTS &&
            align16(xstage_bytes(k)) + (size_t)WAVES * batch_area(1, row_bytes_of<DT>(k)) <= 160 * 1024;
+}
+// mul_mv_id rows: two rows of every wave in whole copy instructions; wider ones stay on
+// the f32 mat-vec as well (k from 20224 Q4_K, 17920 Q5_K, 16384 Q6_K, 13504 Q8_0)
+template <int DT> static bool mv_fits_dt(int k) {
+    return row_fits<DT>(k) && align16(xstage_bytes(k)) + (size_t)WAVES * 2 * 1024 * dma_insts(1, 1, row_bytes_of<DT>(k)) <=
+                                  160 * 1024;
 }
 // gate/up rows: a gate and an up row of at most DMA_MAX_INSTS copies together
 template <int DT> static bool gu_fits_dt(int hidden, int64_t row_bytes) {
@@ -777,7 +785,7 @@ template <int DT> static bool gu_fits_dt(int hidden, int64_t row_bytes) {
            dma_insts(2, 1, row_bytes) <= DMA_MAX_INSTS;
 }
 template <int DT> static bool dn_fits_dt(int ff, int64_t row_bytes) {
-    return mv_fits_dt<DT>(ff) && row_bytes == row_bytes_of<DT>(ff);
+    return row_fits<DT>(ff) && row_bytes == row_bytes_of<DT>(ff);
 }
 #define MX_DT_SWITCH(dtype, EXPR)                       \
     switch (dtype) {                                    \

@@ -86,6 +86,52 @@ def test_mul_mv_row_widths(orc, dt, k):
         assert r <= F32_CLASS
 
 
+# rows the f32 mat-vec holds: seven groups times a power of two, and rows too wide for
+# the mat-vec's two copies in LDS (the narrowest of each type whose scale group is 128 values)
+F32_ROWS = [
+    (GgmlDType.Q4_K, 1792), (GgmlDType.Q4_K, 7168), (GgmlDType.Q4_K, 14336), (GgmlDType.Q4_K, 20224),
+    (GgmlDType.Q5_K, 3584), (GgmlDType.Q5_K, 7168), (GgmlDType.Q5_K, 14336), (GgmlDType.Q5_K, 17920),
+    (GgmlDType.Q6_K, 16384), (GgmlDType.Q8_0, 13568),
+]
+
+
+@pytest.mark.parametrize("dt,k", F32_ROWS, ids=lambda v: str(getattr(v, "name", v)))
+def test_f32_rows_keep_their_precision(orc, dt, k):
+    """Activations held in f32: a value of 2^20 that meets only zero weights takes nothing
+    from the 127 others of its scale group (the 24-bit block grid would hold those to
+    2^-4).  Bound: f32 products and sums, as the precision tests hold the mat-vec to."""
+    rng = np.random.default_rng(k)
+    e, n_out, t, top_k = 4, 70, 2, 2
+    st = synth_stack(dt, e, n_out, k, tensor_key(4450, 0, k))
+    raw = st.buffer.reshape(-1, dt.type_size)
+    if dt in (GgmlDType.Q4_K, GgmlDType.Q5_K):  # the first sub-block's 6-bit scale and minimum
+        raw[:, 4] &= 0xC0
+        raw[:, 8] &= 0xC0
+    elif dt == GgmlDType.Q6_K:  # the first two 16-value groups' scales
+        raw[:, 192:194] = 0
+    else:  # every fourth block's scale
+        raw[::4, 0:2] = 0
+    x = rng.standard_normal((t, 1, k)).astype(np.float32)
+    x[..., :: 256 if dt.block_size == 256 else 128] = np.float32(2.0**20)
+    ids = np.stack([rng.permutation(e)[:top_k] for _ in range(t)])
+    got = host(ops.mul_mv_id(st, dev_f32(x), dev_u32(ids)))
+    w = orc.dequantize(int(dt), host(st.buffer), e * n_out * k).reshape(e, n_out, k).astype(np.float64)
+    want = np.einsum("tsnk,tk->tsn", w[ids], x[:, 0].astype(np.float64))
+    r = rel_l2(got, want)
+    print(f"{dt.name} k={k}: rel-L2 {r:.2e}", flush=True)
+    assert r <= 2e-6
+
+
+@pytest.mark.parametrize("dt,ff", [(GgmlDType.Q4_K, 1792), (GgmlDType.Q4_K, 7168), (GgmlDType.Q4_K, 14336),
+                                   (GgmlDType.Q5_K, 7168)], ids=lambda v: str(getattr(v, "name", v)))
+def test_f32_down_rows_keep_the_layer_in_f32(orc, dt, ff):
+    """Layers with such down rows run the f32 mat-vecs below 32 tokens, also at the
+    token counts whose experts elsewhere take f16 operands (an error near 5e-4)."""
+    spec = LayerSpec(512, ff, 8, 2, GgmlDType.Q4_K, dt, shared=False)
+    for t in (1, 5, 20):
+        layer_against_oracle(orc, spec, t, 4470 + t, F32_CLASS)
+
+
 def _mul_mv_errors(orc, dt, n_out, k, x, off=0):
     """Relative error of each token's row of mul_mv against float64."""
     st = synth_stack(dt, 1, n_out, k, tensor_key(4500, 0, n_out))
