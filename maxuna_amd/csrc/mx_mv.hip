@@ -35,6 +35,8 @@
 //
 // Reference kernels replaced: kernel_mul_mv_id_*_f32_v (mv.metal:680-731, dispatch
 // geometry dispatch.rs:409-462), silu_mul.metal:57-72, combine.metal:70-97.
+#include <algorithm>
+
 #include "mx_launch.h"
 #include "mx_stage.h"
 #include "mx_dma.h"
@@ -404,9 +406,10 @@ template <int DT, int LPR, int AUX> struct RowWalk {
 };
 
 // The compiled (LPR, NG) pairs: the fewest padded groups, and of equal ones the
-// most rows per pass (fewer exchange steps per row).  Q4_K / Q5_K groups are 64
-// weights and 52 registers of activation digits, the others 32 weights and up to
-// 36, so the former stop at two groups a lane where they can.
+// most rows per pass (fewer exchange steps per row).  Three groups a lane fill all
+// lanes at 48, 96 and 192 groups, where two or four leave a quarter of them idle
+// (mul_mv, us: Q4_K [100352 x 3072] 35.0 -> 31.4, Q5_K [16384 x 6144] 23.5 -> 19.8;
+// Q6_K [100352 x 6144] 131 -> 108 with the grid below), six at 384.
 // f(integral_constant LPR, integral_constant NG)
 template <int DT, class F> static auto with_lanes(int G, F &&f) {
 #define MX_LN(L, N) return f(std::integral_constant<int, L>{}, std::integral_constant<int, N>{})
@@ -414,7 +417,9 @@ template <int DT, class F> static auto with_lanes(int G, F &&f) {
         if (G <= 8) MX_LN(8, 1);
         if (G <= 16) MX_LN(16, 1);
         if (G <= 32) MX_LN(16, 2);
+        if (G <= 48) MX_LN(16, 3);
         if (G <= 64) MX_LN(32, 2);
+        if (G <= 96) MX_LN(32, 3);
     } else {
         if (G <= 16) MX_LN(16, 1);
         if (G <= 24) MX_LN(8, 3);
@@ -426,7 +431,9 @@ template <int DT, class F> static auto with_lanes(int G, F &&f) {
         if (G <= 96) MX_LN(32, 3);
     }
     if (G <= 128) MX_LN(64, 2);
+    if (G <= 192) MX_LN(64, 3);
     if (G <= 256) MX_LN(64, 4);
+    if (G <= 384) MX_LN(64, 6);
     MX_LN(64, 8);
 #undef MX_LN
 }
@@ -434,7 +441,7 @@ constexpr int G_MAX = 512;  // groups of the widest compiled row
 template <int DT> __host__ __device__ constexpr int groups(int k) { return k / block_size(DT) * Q<DT>::GPB; }
 // waves per SIMD the registers of NG activation groups allow without spilling
 template <int DT, int NG> constexpr int rows_wpe() {
-    if (DT == kQ4_K || DT == kQ5_K) return NG == 1 ? 4 : NG == 2 ? 3 : 1;
+    if (DT == kQ4_K || DT == kQ5_K) return NG == 1 ? 4 : NG == 2 ? 3 : NG == 3 ? 2 : 1;
     return NG == 1 ? 4 : NG <= 3 ? 3 : NG == 4 ? 2 : 1;
 }
 // rows per batch: passes of rpi rows up to about 5 KB, a power of two of them
@@ -550,24 +557,49 @@ k_mul_mv_id(MvArgs a, int br, int nb, int area, int two) {
     rw.run(xs, groups<DT>(a.k), [&](int row, float v) { dst[row] = v; });
 }
 
-// waves a launch aims at (8 per CU), at least two batches each
-#ifndef MX_MV_WAVES
-#define MX_MV_WAVES 4096
-#endif
+// Workgroups per pair of a mul_mv_id launch of `batches` batches a pair: one batch a wave
+// where all of them are resident at once, else whole rounds of the `resident` workgroups,
+// as few as fill their wave slots to nine tenths (every workgroup stages its activation
+// row, and a last round that is nearly empty costs as much as a full one).
+static int64_t mv_grid(int64_t batches, int64_t pairs, int64_t resident) {
+    auto wgs = [&](int64_t nb) { return (batches + nb * WAVES - 1) / (nb * WAVES); };
+    if (wgs(1) * pairs <= resident) return wgs(1);
+    int64_t best = 1;
+    double fill = 0;
+    for (int64_t r = 1; r <= 8; r++) {
+        const int64_t gx = std::min(wgs(2), std::max<int64_t>(1, r * resident / pairs));
+        const int64_t nb = (batches + gx * WAVES - 1) / (gx * WAVES), rounds = (gx * pairs + resident - 1) / resident;
+        const double f = (double)(batches * pairs) / (double)(rounds * resident * WAVES * nb);
+        if (f > fill + 0.02) best = wgs(nb), fill = f;
+        if (gx == wgs(2) || f >= 0.9) break;
+    }
+    return best;
+}
+// LDS and registers: workgroups of k_mul_mv_id a CU holds
+template <int DT, int NG> static int mv_per_cu(size_t lds) {
+    const int by_lds = (int)(160 * 1024 / lds), by_regs = rows_wpe<DT, NG>();
+    return by_lds < by_regs ? by_lds : by_regs;
+}
 template <int DT> static mx_status launch_mv_dt(const MvArgs &a, hipStream_t s) {
     return with_lanes<DT>(groups<DT>(a.k), [&](auto lpr, auto ng) -> mx_status {
         constexpr int LPR = decltype(lpr)::value, NG = decltype(ng)::value;
-        const int br = batch_rows(64 / LPR, a.row_bytes, 16), area = batch_area(br, a.row_bytes);
-        const int64_t pairs = (int64_t)a.t * a.top_k, batches = (a.n_out + br - 1) / br;
-        int64_t nb = batches * pairs / MX_MV_WAVES;
-        nb = nb < 2 ? 2 : nb;
-        const unsigned gx = (unsigned)((batches + nb * WAVES - 1) / (nb * WAVES));
-        // (the waves' batches interleave over the launched grid: round nb up to cover it)
-        nb = (batches + (int64_t)gx * WAVES - 1) / ((int64_t)gx * WAVES);
+        const int64_t pairs = (int64_t)a.t * a.top_k;
         const size_t stg = align16(xstage_bytes(a.k));
+        // a batch grows into LDS that would stay idle, while every resident wave still has
+        // two (wide rows, one workgroup per CU: Q8_0 [1024 x 7168] for 16 pairs 28.5 -> 26.4)
+        int br = batch_rows(64 / LPR, a.row_bytes, 16);
+        auto need = [&](int b) { return stg + (size_t)WAVES * 2 * batch_area(b, a.row_bytes); };
+        while (br < 16 && need(2 * br) <= 160 * 1024 && mv_per_cu<DT, NG>(need(2 * br)) == mv_per_cu<DT, NG>(need(br)) &&
+               (int64_t)a.n_out * pairs >= (int64_t)4 * br * WAVES * mv_per_cu<DT, NG>(need(br)) * device_cus())
+            br *= 2;
+        const int area = batch_area(br, a.row_bytes);
+        const int64_t batches = (a.n_out + br - 1) / br;
         const int two = stg + (size_t)WAVES * 2 * area <= 160 * 1024;
         const size_t lds = stg + (size_t)WAVES * (two ? 2 : 1) * area;
-        hipLaunchKernelGGL((k_mul_mv_id<DT, NG, LPR>), dim3(gx, (unsigned)pairs), dim3(64 * WAVES), lds, s, a, br,
+        const int64_t gx = mv_grid(batches, pairs, (int64_t)mv_per_cu<DT, NG>(lds) * device_cus());
+        // (the waves' batches interleave over the launched grid)
+        const int64_t nb = (batches + gx * WAVES - 1) / (gx * WAVES);
+        hipLaunchKernelGGL((k_mul_mv_id<DT, NG, LPR>), dim3((unsigned)gx, (unsigned)pairs), dim3(64 * WAVES), lds, s, a, br,
                            (int)nb, area, two);
         return MX_OK;
     });

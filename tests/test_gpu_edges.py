@@ -86,6 +86,41 @@ def test_mul_mv_row_widths(orc, dt, k):
         assert r <= F32_CLASS
 
 
+# rows at and just past the ends of the lane layouts of three and six groups
+THREES = [
+    (GgmlDType.Q4_K, 3072), (GgmlDType.Q4_K, 3328), (GgmlDType.Q4_K, 6144), (GgmlDType.Q5_K, 4352),
+    (GgmlDType.Q5_K, 6144), (GgmlDType.Q5_K, 12288), (GgmlDType.Q6_K, 4352), (GgmlDType.Q6_K, 6144),
+    (GgmlDType.Q6_K, 8448), (GgmlDType.Q6_K, 12288), (GgmlDType.Q8_0, 4128), (GgmlDType.Q8_0, 6144),
+    (GgmlDType.Q8_0, 12288), (GgmlDType.Q8_0, 12320),
+]
+
+
+@pytest.mark.parametrize("dt,k", THREES, ids=lambda v: str(getattr(v, "name", v)))
+def test_mul_mv_id_grids(orc, dt, k):
+    """One batch a wave, whole rounds of workgroups and rounds that share a wave's batches
+    unevenly: 2, 26 and 330 pairs of a row count that no batch divides."""
+    rng = np.random.default_rng(k)
+    e, n_out, top_k = 3, 197, 2
+    st = synth_stack(dt, e, n_out, k, tensor_key(4460, 0, k))
+    w = orc.dequantize(int(dt), host(st.buffer), e * n_out * k).reshape(e, n_out, k).astype(np.float64)
+    for t in (1, 13, 165):
+        x = rng.standard_normal((t, 1, k)).astype(np.float32)
+        ids = np.stack([rng.permutation(e)[:top_k] for _ in range(t)])
+        got = host(ops.mul_mv_id(st, dev_f32(x), dev_u32(ids)))
+        y = x[:, 0].astype(np.float64) @ w.reshape(e * n_out, k).T
+        want = y.reshape(t, e, n_out)[np.arange(t)[:, None], ids]
+        r = rel_l2(got, want)
+        print(f"{dt.name} k={k} t={t}: rel-L2 {r:.2e}", flush=True)
+        assert r <= F32_CLASS
+
+
+@pytest.mark.parametrize("dt,ff", [THREES[i] for i in (0, 2, 4, 7, 12)], ids=lambda v: str(getattr(v, "name", v)))
+def test_decode_down_rows_of_three(orc, dt, ff):
+    for t in (1, 2, 5):
+        spec = LayerSpec(288, ff, 12, 3, GgmlDType.Q8_0, dt, shared=True)
+        layer_against_oracle(orc, spec, t, 4310 + t, F32_CLASS)
+
+
 # rows the f32 mat-vec holds: seven groups times a power of two, and rows too wide for
 # the mat-vec's two copies in LDS (the narrowest of each type whose scale group is 128 values)
 F32_ROWS = [
