@@ -1406,13 +1406,8 @@ k_decode_down(DecodeDownArgs a, int rpw, int br, int area, int two) {
 // its own LDS area and streams the slot's `rows` down rows; the partial rows meet in
 // LDS and threads 0 .. rows - 1 combine them in slot order, with the arithmetic of
 // k_decode_down's combine (combine.metal:70-97).  No partial rows in global
-// memory, no arrival counters, no cross-block tail.
-// above this, more and smaller blocks (k_decode_down) keep the CUs fuller (Q5_K /
-// Q6_K hidden 5120 at t = 4: layer 151 -> 136 us; Q6_K / Q4_K hidden 6144, ff 2816
-// at t = 3: 183 -> 139; hidden 4096 at t = 3: the same)
-#ifndef MX_DN_SLOTS_MAX_T
-#define MX_DN_SLOTS_MAX_T 2
-#endif
+// memory, no arrival counters, no cross-block tail.  Taken where its few large
+// workgroups fill the CUs (dn_slots_fit).
 constexpr int DN_SLOTS_MAX = 12;  // 3 waves per SIMD: 168 VGPRs
 constexpr int XPRE_W = 4;  // act quarters per lane held in registers before the weight copies
 template <int DT, int NG, int LPR, int AUX>
@@ -1583,7 +1578,7 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDow
     a.out[o] = vv;
 }
 
-// Verify-block form of the compile-time Q6_K down rows (t > 4, the grid of
+// Verify-block form of the compile-time Q6_K down rows (t > 2, the grid of
 // k_decode_down: one workgroup per (row tile, slot, token), DQ6V_RPW rows per
 // wave, the pair's act row staged once per workgroup): the field offsets of
 // k_decode_down_q6r, hoisted out of the row loop, and its two-buffer ring of
@@ -1722,7 +1717,15 @@ struct DnSlots {
 };
 // true when the slot-per-wave kernel takes this launch
 template <int DT> static bool dn_slots_fit(const DecodeDownArgs &a) {
-    if (a.t > MX_DN_SLOTS_MAX_T || a.top_k + (a.sh_down ? 1 : 0) > DN_SLOTS_MAX) return false;
+    if (a.top_k + (a.sh_down ? 1 : 0) > DN_SLOTS_MAX) return false;
+    // One workgroup holds every slot of 16 rows: at most one of them per CU, or two full
+    // rounds.  A partly filled second round waits for whole workgroups, where the more and
+    // smaller ones of k_decode_down keep the CUs fuller (layers, us, this kernel / that one:
+    // Q5_K hidden 5120, ff 1536 at t = 1 (320 tiles) 52.7 / 43.5; Q6_K hidden 6144, ff 2816 at
+    // t = 1 (384) 68 / 50; hidden 7168 at t = 2 109 / 100; Q4_K hidden 1024 at t = 4 (256)
+    // 20.2 / 21.9, hidden 2048, ff 768 at t = 2 (256) 27.3 / 29.8, at t = 4 (512) 35 / 39)
+    const int64_t n = (int64_t)((a.hidden + RW_DN - 1) / RW_DN) * a.t, cus = device_cus();
+    if (DT == kQ6_K && dn_q6_ok(a) ? a.t > 2 : n > cus && (n > 2 * cus || 20 * n < 39 * cus)) return false;
     return with_lanes<DT>(groups<DT>(a.ff), [&](auto lpr, auto ng) {
         return decltype(ng)::value <= dn_slots_max_ng<DT>() &&
                DnSlots(a, 64 / decltype(lpr)::value).lds <= 160 * 1024 - sizeof(float) * DN_SLOTS_MAX * RW_DN;

@@ -121,6 +121,15 @@ def test_decode_down_rows_of_three(orc, dt, ff):
         layer_against_oracle(orc, spec, t, 4310 + t, F32_CLASS)
 
 
+@pytest.mark.parametrize("hidden,ts", [(1024, (3, 4, 5)), (2048, (2, 3, 4)), (5120, (1, 2))])
+def test_decode_down_slots_line(orc, hidden, ts):
+    """Both sides of the slot-per-wave down kernel's line: up to 256 tiles of 16 rows, a
+    partly filled second round, two full rounds."""
+    for t in ts:
+        spec = LayerSpec(hidden, 512, 12, 3, GgmlDType.Q8_0, GgmlDType.Q6_K, shared=True)
+        layer_against_oracle(orc, spec, t, 4320 + t, F32_CLASS)
+
+
 # rows the f32 mat-vec holds: seven groups times a power of two, and rows too wide for
 # the mat-vec's two copies in LDS (the narrowest of each type whose scale group is 128 values)
 F32_ROWS = [
