@@ -32,9 +32,10 @@ bool mv_ring_fits(int dtype, int k);
 // compute units of the current device (mx_vmm.hip)
 int device_cus();
 
-// mx_mvt.hip -- plain mat-vec for several tokens (2 and more): one matrix w
-// [n_out, k], x [t, k] -> dst [t, n_out]
-bool mv_tokens_fits(int t, int k);
+// mx_mvt.hip -- plain mat-vec of one matrix w [n_out, k] for several tokens at once, x
+// [t, k] -> dst [t, n_out]; k a multiple of 256.  Taken where it is faster than a mat-vec
+// per token (from 2 tokens on, or one where the ring kernel does not take the rows).
+bool mv_tokens_takes(int dtype, int t, int n_out, int k, int64_t row_bytes);
 mx_status launch_mv_tokens(int dtype, const uint8_t *w, int64_t row_bytes, int n_out, int k, const float *x, int t,
                            float *dst, hipStream_t s);
 

@@ -834,11 +834,8 @@ bool decode_down_fits(int dtype, int ff, int64_t row_bytes) { MX_DT_SWITCH(dtype
 
 mx_status launch_mul_mv_id(int dtype, const MvArgs &a, hipStream_t s) {
     if (a.n_out == 0 || (int64_t)a.t * a.top_k == 0) return MX_OK;
-    // one matrix, several tokens: the weights read once for up to 16 of them (lm_head
-    // [100352 x 3072] Q6_K, us, per-token mat-vecs against this: t = 2 84 / 78, 4 133 /
-    // 77, 8 255 / 78, 16 503 / 82), and the one-token rows the ring kernel does not
-    // take (Q4_K [50000 x 3584] 94 / 48; both forms' errors are below theirs)
-    if (!a.ids && a.top_k == 1 && mv_tokens_fits(a.t, a.k) && (a.t > 1 || !mv_ring_fits(dtype, a.k)))
+    // one matrix, several tokens: the weights read once for up to 16 of them
+    if (!a.ids && a.top_k == 1 && mv_tokens_takes(dtype, a.t, a.n_out, a.k, a.row_bytes))
         return launch_mv_tokens(dtype, a.w, a.row_bytes, a.n_out, a.k, a.x, a.t, a.dst, s);
     if (!mv_ring_fits(dtype, a.k)) {  // any other row width: the f32 mat-vec
         const MvfArgs f{a.w, a.expert_bytes, a.row_bytes, a.n_expert, a.n_out, a.k, a.x, a.x_per_row,

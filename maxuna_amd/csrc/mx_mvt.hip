@@ -1,6 +1,7 @@
-// Plain quantised mat-vec for several tokens at once (mul_mv from two tokens on:
-// the vocabulary projection of a verified block or of a small batch; replaces
-// ops::mv_id::mul_mv, mv_id.rs:54-56, for those).
+// Plain quantised mat-vec for several tokens at once (the vocabulary projection of a
+// verified block or of a small batch; replaces ops::mv_id::mul_mv, mv_id.rs:54-56, for
+// those), and for one token of rows that the ring kernel does not take
+// (mv_tokens_takes).
 //
 // The per-token mat-vecs read and unpack the matrix once per token.  Here the
 // activations stay put and the weights stream past them once: every wave of a
@@ -420,7 +421,32 @@ template <int DT> void mt_launch(MtArgs a, hipStream_t s) {
 }
 }  // namespace
 
-bool mv_tokens_fits(int t, int k) { return t <= 65535 * MT_TOK && k > 0 && k % 256 == 0; }
+// Whether this form is the faster one, from the estimated us of both.  Its launches have a
+// latency of their own, one per 12 super-blocks of K, so few rows stay on the per-token
+// mat-vecs: Q6_K [512 x 4096], us, per token / here: t = 2 12 / 19, 16 13 / 27; [8192 x
+// 4096] t = 2 13 / 24, 8 33 / 27, 16 59 / 32; [100352 x 3072] t = 2 76 / 73, 16 505 / 78;
+// Q4_K [8192 x 6144] t = 2 14 / 20, 4 21 / 21, 16 68 / 25.  Rows that the ring kernel does
+// not take cost the f32 mat-vec far more per byte: Q4_K at one token [32000 x 7168] 117 /
+// 59, [2048 x 14336] 18 / 38.  Of 1370 calls (64 to 100352 rows, K 512 to 28672, 2 to 24
+// tokens, replayed in a graph) taking every one here left 292 more than 4% slower than the
+// per-token form of before; the line leaves 18, the worst 16% (Q6_K, K 14336).
+bool mv_tokens_takes(int dtype, int t, int n_out, int k, int64_t row_bytes) {
+    if (t > 65535 * MT_TOK || k <= 0 || k % 256) return false;
+    if (t > 65535) return true;  // (the per-token grid's limit)
+    const bool ring = mv_ring_fits(dtype, k);
+    if (t == 1 && ring) return false;
+    // bytes per us and token of the per-token form, bytes per us and pass of this one, us per launch
+    struct Rates { double per_token, pass, launch; };
+    const Rates r = dtype == kQ4_K   ? Rates{4.0e6, 3.5e6, 8}
+                    : dtype == kQ5_K ? Rates{3.5e6, 2.5e6, 8}
+                    : dtype == kQ6_K ? Rates{5.5e6, 3.0e6, 10}
+                                     : Rates{3.0e6, 2.5e6, 10};
+    const double bytes = (double)n_out * (double)row_bytes;
+    const int launches = (k / 256 + MT_WAVES - 1) / MT_WAVES, passes = (t + MT_TOK - 1) / MT_TOK;
+    const double per_token = 4.0 + t * bytes / (ring ? r.per_token : 1.1e6);
+    const double here = launches * r.launch * (1.0 + 0.02 * (t < MT_TOK ? t : MT_TOK)) + passes * bytes / r.pass;
+    return here < per_token;
+}
 
 mx_status launch_mv_tokens(int dtype, const uint8_t *w, int64_t row_bytes, int n_out, int k, const float *x, int t,
                            float *dst, hipStream_t s) {

@@ -139,6 +139,18 @@ F32_ROWS = [
 ]
 
 
+def _no_weight_in_first_group(buffer, dt):
+    """Zeroes the weights of the first 32 values of every 256 (of every 128 for Q8_0)."""
+    raw = buffer.reshape(-1, dt.type_size)
+    if dt in (GgmlDType.Q4_K, GgmlDType.Q5_K):  # the first sub-block's 6-bit scale and minimum
+        raw[:, 4] &= 0xC0
+        raw[:, 8] &= 0xC0
+    elif dt == GgmlDType.Q6_K:  # the first two 16-value groups' scales
+        raw[:, 192:194] = 0
+    else:  # every fourth block's scale
+        raw[::4, 0:2] = 0
+
+
 @pytest.mark.parametrize("dt,k", F32_ROWS, ids=lambda v: str(getattr(v, "name", v)))
 def test_f32_rows_keep_their_precision(orc, dt, k):
     """Activations held in f32: a value of 2^20 that meets only zero weights takes nothing
@@ -147,14 +159,7 @@ def test_f32_rows_keep_their_precision(orc, dt, k):
     rng = np.random.default_rng(k)
     e, n_out, t, top_k = 4, 70, 2, 2
     st = synth_stack(dt, e, n_out, k, tensor_key(4450, 0, k))
-    raw = st.buffer.reshape(-1, dt.type_size)
-    if dt in (GgmlDType.Q4_K, GgmlDType.Q5_K):  # the first sub-block's 6-bit scale and minimum
-        raw[:, 4] &= 0xC0
-        raw[:, 8] &= 0xC0
-    elif dt == GgmlDType.Q6_K:  # the first two 16-value groups' scales
-        raw[:, 192:194] = 0
-    else:  # every fourth block's scale
-        raw[::4, 0:2] = 0
+    _no_weight_in_first_group(st.buffer, dt)
     x = rng.standard_normal((t, 1, k)).astype(np.float32)
     x[..., :: 256 if dt.block_size == 256 else 128] = np.float32(2.0**20)
     ids = np.stack([rng.permutation(e)[:top_k] for _ in range(t)])
@@ -203,6 +208,27 @@ def test_mul_mv_tokens(orc, dt, k):
         err = _mul_mv_errors(orc, dt, n_out, k, rng.standard_normal((t, k)).astype(np.float32), off)
         print(f"{dt.name} [{n_out} x {k}] t={t}: {err.max():.2e}", flush=True)
         assert err.max() <= (TOKENS if n_out > 16 else F32_CLASS)
+
+
+@pytest.mark.parametrize("dt", [GgmlDType.Q4_K, GgmlDType.Q5_K, GgmlDType.Q6_K, GgmlDType.Q8_0], ids=lambda v: v.name)
+@pytest.mark.parametrize("k", [256, 1024, 3072, 3328, 6400])
+def test_mul_mv_tokens_taken(orc, dt, k):
+    """Calls past the line between a mat-vec per token and the several-token kernel: partial
+    row tiles and token groups, 1 to 12 waves, K in up to three launches.  A value of 2^20
+    that meets zero weights tells the two apart: the several-token kernel holds its
+    neighbours to 2^-40 of it (an error near 1e-6), the block grid to 2^-23 (4e-2)."""
+    rng = np.random.default_rng(k)
+    for n_out in (17, 333, 4201):
+        st = synth_stack(dt, 1, n_out, k, tensor_key(4520, 0, n_out))
+        t = int(1e8) * (k // 3073 + 2) // st.nbytes | 1  # (by bytes: the line's measure)
+        _no_weight_in_first_group(st.buffer, dt)
+        x = rng.standard_normal((t, k)).astype(np.float32)
+        x[:, ::256] = np.float32(2.0**20)
+        got = host(ops.mul_mv(st.buffer, dt, n_out, k, dev_f32(x)))
+        w = orc.dequantize(int(dt), host(st.buffer), n_out * k).reshape(n_out, k).astype(np.float64)
+        r = rel_l2(got, x.astype(np.float64) @ w.T)
+        print(f"{dt.name} [{n_out} x {k}] t={t}: rel-L2 {r:.2e}", flush=True)
+        assert r <= F32_CLASS
 
 
 def test_mul_mv_tokens_ranges(orc):
