@@ -374,7 +374,8 @@ __global__ void __launch_bounds__(64 * MT_WAVES) k_mv_tokens(MtArgs a) {
         });
         float f = 1.0f;
         if constexpr (DT == kQ6_K) f = h2f((uint16_t)w.d);
-        const float4_t acc = {f * ts.x * sum[0], f * ts.y * sum[1], f * ts.z * sum[2], f * ts.w * sum[3]};
+        // (the token's power of two last: f times it may be subnormal, Q6_K with |x| below 2^-113)
+        const float4_t acc = {f * sum[0] * ts.x, f * sum[1] * ts.y, f * sum[2] * ts.z, f * sum[3] * ts.w};
         // the waves' partial sums, added in wave order; one barrier a tile (the other
         // parity's buffer is rewritten only after the next tile's barrier)
         *reinterpret_cast<float4_t *>(&sRed[par][wave][4 * lane]) = acc;

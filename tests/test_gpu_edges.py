@@ -231,6 +231,25 @@ def test_mul_mv_tokens_taken(orc, dt, k):
         assert r <= F32_CLASS
 
 
+@pytest.mark.parametrize("exponent", [-124, -114, 100])
+def test_mul_mv_tokens_magnitudes(orc, exponent):
+    """Whole calls of very small and very large activations through the several-token kernel,
+    with the block scales of centred weights (2e-5): no product of a block's scale and the
+    token's power of two may lose bits."""
+    rng = np.random.default_rng(5)
+    n_out, k, t = 4201, 1024, 143
+    st = synth_stack(GgmlDType.Q6_K, 1, n_out, k, tensor_key(4530, 0, 0))
+    d = (2e-5 * (0.5 + rng.random(n_out * k // 256))).astype(np.float16)
+    st.buffer.reshape(-1, 210)[:, 208:210] = torch.from_numpy(d.view(np.uint8).reshape(-1, 2)).cuda()
+    x = (rng.standard_normal((t, k)) * 2.0**exponent).astype(np.float32)
+    got = host(ops.mul_mv(st.buffer, GgmlDType.Q6_K, n_out, k, dev_f32(x)))
+    w = orc.dequantize(int(GgmlDType.Q6_K), host(st.buffer), n_out * k).reshape(n_out, k).astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    r = rel_l2(got.astype(np.float64) * 2.0**-exponent, want * 2.0**-exponent)
+    print(f"2^{exponent}: {r:.2e}", flush=True)
+    assert r <= TOKENS
+
+
 def test_mul_mv_tokens_ranges(orc):
     """Tokens of very different magnitudes, super-blocks 2^40 apart, an all-zero token,
     and a token with an Inf: only that token's outputs are not finite."""
