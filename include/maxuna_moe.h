@@ -149,11 +149,12 @@ mx_status mx_prepare_map0(int64_t n_expert, const uint32_t *ids, int64_t t, int6
  * Shapes as mx_mul_mv_id; `map` must come from mx_prepare_map0 with the same
  * ids, and its geometry must match (n_expert, t, top_k), else MX_ERR_SCRATCH
  * (dispatch.rs:886-896).  Supported: Q4_K, Q5_K, Q6_K, Q8_0.
- * Up to 1024 (token, slot) pairs (Q4_K / Q6_K, K a multiple of 512, n_out of
+ * Up to 1280 (token, slot) pairs (Q4_K / Q6_K, K a multiple of 512, n_out of
  * 32) the projection runs the 16-pair MFMA tiles of the MoE forward's verify
  * blocks; beyond that, when K is a multiple of 256, the MFMA matmuls of the
- * prefill path (of a few pairs per expert, or the grouped GEMM; the tiles go on to
- * 2560 pairs where the former do not take the shape); all over x rounded to f16 (one power-of-two scale per x row).  Their
+ * prefill path (for few pairs per expert, or the grouped GEMM; the tiles go on to
+ * 2560 pairs where the former do not take the stack: matrices of less than 256 MB
+ * in all among others); all over x rounded to f16 (one power-of-two scale per x row).  Their
  * temporaries (the f16 rows, t * x_per_row * (2k + 4) bytes, and the tiles'
  * pair order) are stream-ordered memory from a library pool per device, which
  * keeps its peak size reserved.  Other K run the fallback tiles with no
@@ -214,7 +215,7 @@ mx_status mx_route_from_logits(const float *logits, const float *bias, int64_t t
  *   out = FusedExperts(x, route(x)) + SharedExpert(x)
  * Fewer than 16 tokens run the f32-class fused decode kernels.  From 16 tokens
  * on, the expert matmuls take f16 operands (the reference's grouped-matmul
- * precision class): 16-pair MFMA tiles while t * (top_k + shared) <= 1024 (2560
+ * precision class): 16-pair MFMA tiles while t * (top_k + shared) <= 1280 (2560
  * where the matmuls for few pairs per expert do not take the shape), the grouped
  * matmuls beyond that for t >= mm_min_seq (moe.rs:236-240; mm_min_seq == 0
  * selects the default 32, ops/mod.rs:31), else the decode kernels.

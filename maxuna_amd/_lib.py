@@ -130,11 +130,12 @@ SIGNATURES = {
     "mx_synth_blocks": (I32, [I32, U64, P, I64, P]),
 }
 
-# bench-only instrumentation (maxuna_amd/csrc/mx_instrument.h): exported by the
+# bench and test instrumentation (maxuna_amd/csrc/mx_instrument.h): exported by the
 # library, not part of the boundary header
 INSTRUMENT_SIGNATURES = {
     "mx_moe_forward_profiled": (I32, [C.POINTER(MoeLayerC), P, I64, P, P, P, P, P, SZ, P, P, I32, P]),
     "mx_moe_forward_repeat": (I32, [C.POINTER(MoeLayerC), P, I64, P, P, P, P, P, SZ, P, I32, I32]),
+    "mx_moe_few_pairs_words": (None, [C.POINTER(MoeLayerC), I64, C.POINTER(I64), C.POINTER(I64)]),
     "mx_probe_read": (I32, [P, I64, P, P]),
 }
 

@@ -41,11 +41,13 @@ mx_status hip_check(hipError_t e, const char *what) {
 #endif
 constexpr int64_t kVmmMaxPairs = MX_VMM_MAX_PAIRS;
 static_assert(kVmmMaxPairs <= PAIR_ORDER_MAX, "the pair order covers the tiles' range");
-// ... and where the stationary-activation matmuls (mx_gst.hip) take the shape: C1-shaped
-// layers (11 slots), µs, tiles vs those: t = 32: 324 vs 371, 64: 414 vs 438, 128:
-// 541 vs 501, 200: 671 vs 581, 232: 730 vs 610; hidden 3072, ff 1024: t = 64: 251 vs
-// 256, 128: 328 vs 301, 200: 378 vs 339
-constexpr int64_t kVmmGstPairs = 1024;
+// ... and where the stationary-activation matmuls (mx_gst.hip) are tried.  Even routers, µs,
+// tiles vs those: C1-shaped layers (11 slots) t = 94: 468 vs 482, 116: 518 vs 494, 128: 526
+// vs 503, 230: 713 vs 632; with Q4_K down rows t = 94: 416 vs 434, 116: 460 vs 452; hidden
+// 3072, ff 1024, Q4_K t = 94: 245 vs 268, 108: 260 vs 272, 116: 289 vs 274.  Skewed routers,
+// where those leave most launches to the grouped GEMM behind them: C1 with 29 experts in use
+// t = 116: 312 vs 229, 230: 498 vs 273; hidden 3072 with 34 t = 108: 169 vs 181, 116: 201 vs 181
+constexpr int64_t kVmmGstPairs = 1280;
 
 static bool supported(int dt) { return dt == kQ4_K || dt == kQ5_K || dt == kQ6_K || dt == kQ8_0; }
 static bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
@@ -248,7 +250,7 @@ GemmArgs mm_args(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64
     return a;
 }
 bool mm_on_gst(const mx_expert_stack *st, const StackGeom &g, int64_t t, int64_t top_k) {
-    return gst_fits(mm_args(st, g, t, top_k), false);
+    return gst_fits(st->dtype, mm_args(st, g, t, top_k), false);
 }
 // A few pairs per expert: the 16-pair MFMA tiles of the verify blocks (each
 // touched expert's weights streamed once) instead of 128-pair GEMM m-tiles
@@ -520,9 +522,9 @@ void plan_gst(const mx_moe_layer *L, int64_t t, Plan &p) {
     };
     set(L->up, L->shared_up, 1);
     set(L->gate, L->shared_gate, 0);
-    p.gst_gu = gst_fits(a, true);
+    p.gst_gu = gst_fits(L->gate.dtype, a, true);
     set(L->down, L->shared_down, 0);
-    p.gst_d = gst_fits(a, false);
+    p.gst_d = gst_fits(L->down.dtype, a, false);
 }
 
 // Chooses the kernels of a forward; every shape limit of the chosen kernels is
@@ -639,7 +641,7 @@ Layout carve(const mx_moe_layer *L, int64_t t, const Plan &p, void *base) {
         const int64_t EM = E + (p.shared_in_decode ? 1 : 0);
         const int64_t KM = K + (p.shared_in_decode ? 1 : 0);
         o.map = ws.take<int32_t>(map0_bytes((int)EM, (int)t, (int)KM) / 4);
-        o.done = ws.take<int32_t>(1);
+        o.done = ws.take<int32_t>(2);  // gate/up, down
         if (p.has_shared && !p.shared_in_decode) {
             o.map_sh = ws.take<int32_t>(map0_bytes(1, (int)t, 1) / 4);
             o.zero_ids = ws.take<uint32_t>(t);
@@ -967,7 +969,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
         da.n_out = (int)H; da.k = (int)FF;
         da.a = o.act16 + act_row0 * FF; da.a_scale = o.act16s + act_row0; da.a_div = 0;
         da.out = o.down; da.out_stride = KK; da.out_add = out_add;
-        da.done = p.gst_d ? o.done : nullptr;
+        da.done = p.gst_d ? o.done + 1 : nullptr;
         if (p.gst_d) MX_TRY(launch_gst(dt_d, false, da, s));
         MX_TRY(launch_gemm(dt_d, false, da, s));
         MX_STAGE();
@@ -1016,6 +1018,17 @@ mx_status mx_moe_forward_profiled(const mx_moe_layer *L, const float *x, int64_t
         MX_HIP(hipEventElapsedTime(&stage_ms[k], tm.ev[i - 1], tm.ev[i]));
     *n_stages = k;
     return MX_OK;
+}
+
+void mx_moe_few_pairs_words(const mx_moe_layer *L, int64_t t, int64_t *gate_up, int64_t *down) {
+    *gate_up = *down = -1;
+    if (!L || t <= 0) return;
+    const Plan p = plan_for(L, t);
+    if (!p.mm) return;
+    uint8_t *const base = reinterpret_cast<uint8_t *>(256);  // (only offsets are taken from it)
+    const int64_t at = reinterpret_cast<uint8_t *>(carve(L, t, p, base).done) - base;
+    if (p.gst_gu) *gate_up = at;
+    if (p.gst_d) *down = at + 4;
 }
 
 mx_status mx_probe_read(const void *src, int64_t nbytes, uint32_t *sink, mx_stream_t stream) {

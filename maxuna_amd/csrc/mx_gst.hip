@@ -77,7 +77,7 @@ template <int PAR> __device__ __forceinline__ void gs_load(WB<kQ8_0> &w, const u
 // Ten times the most runs per m-tile of the map at which a launch is taken.  The
 // average of pairs per expert, all the host knows, does not tell: with a router that
 // uses a quarter of 256 experts (hidden 4096, ff 1536, Q4_K / Q6_K) 12 pairs on average
-// took 422 us in the grouped GEMM and 461 here, 20: 485 / 662; evenly used experts of 24
+// took 414 us in the grouped GEMM and 461 here, 20: 485 / 662; evenly used experts of 24
 // pairs 290 / 239, of 40 (1.9 runs per m-tile) 299 / 304.  By type, from even use: plain
 // [4096 x 1536] Q5_K of 24 pairs 122 / 115, 36: 130 / 142; Q6_K 36: 185 / 145; Q8_0 24:
 // 146 / 147; SwiGLU hidden 3072 Q6_K of 40: 482 / 392, Q8_0 440 / 463.
@@ -129,6 +129,7 @@ k_gst(GemmArgs a, int W) {
     const MapLayout L(E, a.t, a.top_k);
 
     // ---- the runs of every expert: exclusive prefix ---------------------------------
+    int runs;
     {
         const int per = (E + BT - 1) / BT, e0 = min(tid * per, E), e1 = min(e0 + per, E);
         int sum = 0;  // runs, and m-tiles of 128 pairs in the upper half (both below 2^15: gst_fits)
@@ -144,22 +145,27 @@ k_gst(GemmArgs a, int W) {
         }
         if (lane == 63) sScan[gwave] = inc;
         __syncthreads();
-        int base0 = 0;
-        for (int w = 0; w < gwave; w++) base0 += sScan[w];
-        int base = base0 + inc - sum;
+        int base = inc - sum, both = 0;
+        for (int w = 0; w < W * teams; w++) {
+            const int v = sScan[w];
+            both += v;
+            if (w < gwave) base += v;
+        }
+        both = __builtin_amdgcn_readfirstlane(both);
+        // many runs for their m-tiles: the grouped GEMM is the faster (block-uniform; nothing
+        // else is done before this: a launch left behind costs 2 to 2.5 us)
+        runs = both & 0xFFFF;
+        const bool mine = 10 * runs < gs_ratio(DT, SWIGLU) * (both >> 16);
+        if (blockIdx.x == 0 && tid == 0) *a.done = mine;
+        if (!mine) return;
         for (int e = e0; e < e1; e++) {
             sRuns[e] = base & 0xFFFF;
             base += (a.map[L.tpe + e] + RUN - 1) / RUN;
         }
-        if (tid == BT - 1) sRuns[E] = (base & 0xFFFF) | (int)((uint32_t)(inc + base0) & 0xFFFF0000u);
+        if (tid == 0) sRuns[E] = runs;
         for (int i = tid; i < 2 * TEAMS * WM * OUT; i += BT) (&sRed[0][0][0][0])[i] = 0.f;
         __syncthreads();
     }
-    // many runs for their m-tiles: the grouped GEMM is the faster (block-uniform)
-    const int both = __builtin_amdgcn_readfirstlane(sRuns[E]), runs = both & 0xFFFF;
-    const bool mine = 10 * runs < gs_ratio(DT, SWIGLU) * (both >> 16);
-    if (blockIdx.x == 0 && tid == 0) *a.done = mine;
-    if (!mine) return;
     const int tiles = a.n_out / 16;
     // this workgroup's share [u0, u1) of the runs * tiles units; neighbouring shares on
     // one XCD (workgroups are dealt to the 8 XCDs round-robin)
@@ -324,7 +330,7 @@ k_gst(GemmArgs a, int W) {
                     constexpr int PAR = decltype(parc)::value;
                     if constexpr (DT == kQ6_K) w.prep(kh);
                     else if constexpr (DT != kQ4_K) w.template prep<PAR>(kh);
-static_for<0, 4>([&](auto pc) MX_INLINE_LAMBDA {
+                    static_for<0, 4>([&](auto pc) MX_INLINE_LAMBDA {
                         constexpr int P = decltype(pc)::value;
                         half8_t bf;
                         if constexpr (DT == kQ4_K) bf = w.step(P);
@@ -349,7 +355,6 @@ static_for<0, 4>([&](auto pc) MX_INLINE_LAMBDA {
             const int o = ttid + NT * j;
             if (o < OUT) {
                 float v = 0.f;
-                
 #pragma unroll
                 for (int w = 0; w < WM; w++) v += sRed[par][team][w][o];
                 const int m = 16 * (o >> 8) + 4 * ((o >> 6) & 3) + (o & 3);
@@ -388,6 +393,8 @@ template <int DT, bool SWIGLU, int MT, int NSB, int WM> void gs_go(const GemmArg
     const unsigned grid = (unsigned)(device_cus() & ~7);
     hipLaunchKernelGGL((k_gst<DT, SWIGLU, MT, NSB, WM>), dim3(grid), dim3(64 * W * teams), W * teams * 2 * G::STAGE, s, a, W);
 }
+// pairs per run of the instantiation gs_launch takes
+int gs_run(int dtype, bool swiglu, int nsb) { return nsb > 16 || (dtype == kQ8_0 && !swiglu && nsb <= 4) ? 16 : 32; }
 // W waves of NSB super-blocks: all the super-blocks of a run's pairs fit the CU's
 // registers (12 waves of one, 8 of more), in several teams where K is short
 template <int DT, bool SWIGLU> void gs_launch(const GemmArgs &a, hipStream_t s) {
@@ -413,7 +420,7 @@ template <int DT, bool SWIGLU> void gs_launch(const GemmArgs &a, hipStream_t s) 
 }
 }  // namespace
 
-bool gst_fits(const GemmArgs &a, bool swiglu) {
+bool gst_fits(int dtype, const GemmArgs &a, bool swiglu) {
     auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool sh = a.w_sh[0] != nullptr;
     bool ok = a.k % 256 == 0 && a.k / 256 >= 2 && a.k / 256 <= 32 && a.n_out % 16 == 0 && a.n_map_expert < GS_MAX_E &&
@@ -423,11 +430,16 @@ bool gst_fits(const GemmArgs &a, bool swiglu) {
     // Gate/up of K up to 1024 stay on the grouped GEMM: a layer of hidden 1024, ff 512, 64
     // experts, Q6_K / Q4_K, took 92 us there, 101 with both projections here and 96 with the down alone (28 pairs).
     ok = ok && (!swiglu || a.k > 1024);
-    // Less than one run (32 pairs, 16 beyond K = 4096) per expert on average: what the
-    // kernel then leaves to the grouped GEMM cost its launch, 3 to 4 us per matmul (2 to
-    // 3% of a layer of 64 to 256 experts under a skewed router); what it takes gained
-    // 1.08 (27 pairs) to 1.3x (12 pairs).
-    return ok && (int64_t)a.t * a.top_k < (a.k <= 4096 ? 32 : 16) * (int64_t)a.n_map_expert;
+    // Matrices of at least 256 MB in all (what the Infinity Cache holds): below, the grouped
+    // GEMM's repeated reads are cheap, and the launch left behind under a skewed router is a
+    // larger share of the layer (layers, us, the GEMM alone / here: hidden 1024, ff 512, 64
+    // experts Q5_K 62 / 71; hidden 2048, ff 768, 128 experts Q4_K / Q6_K at 200 tokens, even
+    // router 206 / 180, skewed 115 / 122).
+    ok = ok && (int64_t)a.n_map_expert * a.n_out * a.row_bytes * (swiglu ? 2 : 1) >= (int64_t)256 << 20;
+    // Less than one run per expert on average: beyond, even an evenly used map has two runs
+    // per m-tile, which no gs_ratio takes where runs are of 16 pairs and few do at 32; what it
+    // takes gained 1.08 (27 pairs) to 1.3x (12 pairs).
+    return ok && (int64_t)a.t * a.top_k < gs_run(dtype, swiglu, a.k / 256) * (int64_t)a.n_map_expert;
 }
 
 mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s) {

@@ -5,7 +5,7 @@
  * reference's MoE interface (src/moe.rs:19-21, src/ops/ files) has no
  * counterpart, and a host binding for the reference never calls them.  They
  * exist so bench.py can time the decode stages inside a replayed graph and
- * read per-stage event times.  mx_moe_forward_repeat with times != 1 gives
+ * read per-stage event times, and the tests see which kernel took a launch.  mx_moe_forward_repeat with times != 1 gives
  * wrong outputs by design (it skips or repeats a stage).
  */
 #ifndef MX_INSTRUMENT_H
@@ -49,6 +49,11 @@ mx_status mx_moe_forward_repeat(const mx_moe_layer *layer, const float *x, int64
                                 const float *residual, float *out, uint32_t *ids_out, float *w_out,
                                 void *workspace, size_t workspace_bytes, mx_stream_t stream,
                                 int32_t stage, int32_t times);
+
+/* Byte offsets in the workspace of the words in which a grouped forward of t tokens says
+ * whether the matmuls for few pairs per expert took gate/up and down (1) or left them to the
+ * grouped GEMM launched behind (0); -1 where they are not tried.  For the tests. */
+void mx_moe_few_pairs_words(const mx_moe_layer *layer, int64_t t, int64_t *gate_up, int64_t *down);
 
 /* A plain streaming read of nbytes (multiple of 16) from src (16-byte aligned),
  * 512 x 256 threads with four 16-byte loads in flight each: the achievable HBM

@@ -264,7 +264,7 @@ bool gemm_plain_fits(int64_t a_rows, int k, int n_out, int64_t row_bytes);
 // mx_gst.hip -- the same contraction for a few dozen pairs per expert (activations
 // stationary).  It takes the launch only where the map's runs are few for its m-tiles
 // and says so in *a.done; launch_gemm with the same a follows and leaves when *a.done.
-bool gst_fits(const GemmArgs &a, bool swiglu);
+bool gst_fits(int dtype, const GemmArgs &a, bool swiglu);
 mx_status launch_gst(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 mx_status launch_gemm(int dtype, bool swiglu, const GemmArgs &a, hipStream_t s);
 // rows of x (f32, [rows, k], k % 4 == 0) -> f16 times a per-row power of two;

@@ -3,11 +3,14 @@ lane layouts, partial tiles, the smallest and largest row counts), against the
 oracle."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from maxuna_amd import ops
+from maxuna_amd._lib import lib
 from maxuna_amd.gguf import ExpertStack, GgmlDType
 from maxuna_amd.synth import LayerSpec, build_layer, make_x, synth_stack, tensor_key
 
@@ -270,39 +273,114 @@ def test_mul_mv_tokens_ranges(orc):
         assert np.all(np.isfinite(got[:5])) and np.all(got[4] == 0) and not np.any(np.isfinite(got[5]))
 
 
-# (gate/up type, down type, hidden, ff): super-blocks of K at the ends of the wave
-# layouts of the stationary-activation matmuls (2 | 4 | 6 | 12 waves of one, 8 of two,
-# then three and four), each type on both projections; gate/up of up to four
-# super-blocks run the grouped GEMM
-GST = [
+# (gate/up type, down type, hidden, ff): every type on both projections, an odd and an even
+# number of super-blocks
+SMALL_GROUPED = [
     ("Q4_K", "Q4_K", 512, 768), ("Q4_K", "Q6_K", 1280, 1536), ("Q4_K", "Q6_K", 3072, 1792), ("Q4_K", "Q4_K", 3328, 1024),
-    ("Q4_K", "Q5_K", 4352, 512), ("Q4_K", "Q6_K", 6400, 512), ("Q5_K", "Q5_K", 1024, 2304), ("Q5_K", "Q6_K", 4096, 1280),
+    ("Q4_K", "Q5_K", 4352, 512), ("Q4_K", "Q6_K", 6400, 512), ("Q5_K", "Q5_K", 1024, 2304), ("Q5_K", "Q6_K", 3584, 1280),
     ("Q6_K", "Q6_K", 1536, 768), ("Q6_K", "Q5_K", 3840, 512), ("Q6_K", "Q4_K", 5120, 512), ("Q8_0", "Q8_0", 512, 1024),
-    ("Q8_0", "Q8_0", 2048, 1280), ("Q8_0", "Q8_0", 2560, 768), ("Q8_0", "Q8_0", 4096, 512), ("Q8_0", "Q8_0", 7168, 512),
+    ("Q8_0", "Q8_0", 2048, 1280), ("Q8_0", "Q8_0", 2560, 768), ("Q8_0", "Q8_0", 4096, 512), ("Q8_0", "Q8_0", 5632, 512),
 ]
 
 
-@pytest.mark.parametrize("gate,down,hidden,ff", GST)
-def test_few_pairs_per_expert(orc, gate, down, hidden, ff):
-    """Layers of a few pairs per expert past the verify tiles, with runs of one and of
-    several tiles of pairs (a hot expert) and experts of none, against the oracle's own
-    routing.  f16 operands: the contract's bound."""
+@pytest.mark.parametrize("gate,down,hidden,ff", SMALL_GROUPED)
+def test_few_pairs_small_matrices(orc, gate, down, hidden, ff):
+    """Layers of a few pairs per expert, skewed, past the verify tiles, whose matrices are too
+    small for the matmuls of few pairs: the grouped GEMM, against the oracle's own routing.
+    f16 operands: the contract's bound."""
     spec = LayerSpec(hidden, ff, 40, 4, GgmlDType[gate], GgmlDType[down], shared=hidden % 512 == 0, bias_sigma=0.3)
     layer = build_layer(spec, seed=4600)
-    # past the verify tiles' pairs where the types have tiles, and under the 32 (K up to
-    # 4096) or 16 pairs per expert up to which these matmuls are tried
-    x = make_x(spec, 4601, 50 if hidden > 4096 else 210 if gate == "Q4_K" else 70)
+    t = 50 if hidden > 4096 else 210 if gate == "Q4_K" else 70
+    assert few_pairs_words(layer.block, t) == (-1, -1)
+    x = make_x(spec, 4601, t)
     out, ids, w = layer.block.forward(torch.from_numpy(x).cuda(), return_routing=True)
     out, ids, w = host(out), host(ids), host(w)
     want, _, _ = orc.moe_layer(spec, layer.keys, layer.router_t, layer.bias, x, ids=ids, w=w)
     assert_close(out, want, what=f"{gate}/{down} {hidden}x{ff}")
 
 
+def few_pairs_words(block, t):
+    """Workspace offsets of the words that say whether the matmuls for few pairs per expert
+    took gate/up and down (-1: not tried)."""
+    gu, dn = C.c_int64(), C.c_int64()
+    lib().mx_moe_few_pairs_words(C.byref(block._c), t, C.byref(gu), C.byref(dn))
+    return gu.value, dn.value
+
+
+def moe_f64(block, x, ids, w):
+    """The layer in 64-bit torch from the dequantised stacks and the given routing."""
+    def weights(st, e):
+        step = st.n_out * st.k // st.dtype.block_size * st.dtype.type_size
+        return ops.dequantize(st.buffer[e * step:(e + 1) * step], st.dtype, st.n_out * st.k).double().reshape(st.n_out, st.k)
+
+    def expert(x, gate, up, down, e):
+        g, u = x @ weights(gate, e).T, x @ weights(up, e).T
+        return (g / (1.0 + torch.exp(-g)) * u) @ weights(down, e).T
+
+    x, ids, w = x.double(), ids.view(torch.int32).long(), w.double()
+    out = torch.zeros_like(x)
+    b = block.experts
+    for e in torch.unique(ids).tolist():
+        tok, slot = torch.nonzero(ids == e, as_tuple=True)
+        out.index_add_(0, tok, expert(x[tok], b.gate, b.up, b.down, e) * w[tok, slot][:, None])
+    if block.shared is not None:
+        out += expert(x, block.shared.gate, block.shared.up, block.shared.down, 0)
+    return out
+
+
+# (gate/up type, down type, hidden, ff): the K of both projections through every wave
+# layout of the stationary-activation matmuls (2, 4, 6 and 12 waves of one super-block, 8 of
+# two, of three and of four; Q8_0 4 and 6 of two in place of 6 and 12 of one), at the ends of
+# each: full and partly filled teams and last waves, several teams
+GST = [
+    ("Q4_K", "Q4_K", 1280, 512), ("Q4_K", "Q6_K", 1536, 1536), ("Q4_K", "Q5_K", 1792, 768), ("Q4_K", "Q4_K", 3072, 1024),
+    ("Q4_K", "Q6_K", 3328, 512), ("Q4_K", "Q4_K", 4096, 1280), ("Q4_K", "Q5_K", 4352, 1536), ("Q4_K", "Q6_K", 6144, 1024),
+    ("Q4_K", "Q4_K", 6400, 2304), ("Q4_K", "Q6_K", 8192, 3072),
+    ("Q5_K", "Q5_K", 1280, 512), ("Q5_K", "Q6_K", 1792, 768), ("Q5_K", "Q5_K", 3072, 1024), ("Q5_K", "Q6_K", 4096, 3328),
+    ("Q5_K", "Q5_K", 6144, 2304), ("Q5_K", "Q4_K", 6400, 3328), ("Q5_K", "Q5_K", 4352, 4096), ("Q5_K", "Q4_K", 2048, 4352),
+    ("Q6_K", "Q6_K", 1536, 4352), ("Q6_K", "Q4_K", 1792, 8192), ("Q6_K", "Q6_K", 3840, 6400), ("Q6_K", "Q5_K", 5120, 6144),
+    ("Q6_K", "Q6_K", 7168, 512), ("Q6_K", "Q5_K", 3072, 6400),
+    ("Q8_0", "Q8_0", 1280, 512), ("Q8_0", "Q8_0", 2048, 1024), ("Q8_0", "Q8_0", 2304, 1280), ("Q8_0", "Q8_0", 3072, 2048),
+    ("Q8_0", "Q8_0", 3328, 2304), ("Q8_0", "Q8_0", 4096, 3072), ("Q8_0", "Q8_0", 4352, 4096), ("Q8_0", "Q8_0", 6400, 4352),
+    ("Q8_0", "Q8_0", 1536, 6400),
+]
+
+
+@pytest.mark.parametrize("gate,down,hidden,ff", GST)
+def test_few_pairs_per_expert(gate, down, hidden, ff):
+    """Layers whose gate/up and down both run the stationary-activation matmuls (read back from
+    the words they write): an expert of every token (several runs), experts of none, the rest
+    evenly used with under a run each.  Against 64 bits, all outputs; f16 operands: the
+    contract's bound."""
+    top_k = 4
+    gdt, ddt = GgmlDType[gate], GgmlDType[down]
+    # both projections' matrices past the 256 MB from which they are tried
+    row = lambda dt, k: k // dt.block_size * dt.type_size  # noqa: E731
+    e = max(128, -(-(264 << 20) // min(2 * ff * row(gdt, hidden), hidden * row(ddt, ff))))
+    spec = LayerSpec(hidden, ff, e, top_k, gdt, ddt, shared=hidden % 512 == 0, bias_sigma=0.0)
+    layer = build_layer(spec, seed=4600)
+    bias = torch.zeros(e)
+    bias[1], bias[2:6] = 10.0, -10.0
+    layer.block.exp_probs_b.copy_(bias)
+    # past the tiles' 1280 pairs where the shape has tiles, about 4 pairs per expert (plus the hot one's)
+    t = max(40 if (hidden // 256) % 2 or (ff // 256) % 2 or "Q5_K" in (gate, down) or gate != "Q4_K" else 325, e)
+    words = few_pairs_words(layer.block, t)
+    assert min(words) >= 0, words
+    x = torch.from_numpy(make_x(spec, 4601, t)).cuda()
+    out, ids, w = layer.block.forward(x, return_routing=True)
+    ws = layer.block._ws.cpu()
+    assert [int(ws[o:o + 4].view(torch.int32)) for o in words] == [1, 1]
+    got = ids.view(torch.int32).cpu()
+    assert int((got == 1).sum()) == t and not torch.any((got >= 2) & (got < 6))
+    want = moe_f64(layer.block, x, ids, w)
+    assert_close(host(out), host(want), what=f"{gate}/{down} {hidden}x{ff} E{e} t{t}")
+
+
 def test_few_pairs_per_expert_alignment_rule(orc):
     """Q6_K stacks two bytes off 16-byte alignment take the other grouped kernel: same
     outputs to f16-operand rounding."""
     rng = np.random.default_rng(8)
-    t, top_k, e, n_out, k = 400, 4, 64, 512, 768
+    t, top_k, e, n_out, k = 400, 4, 224, 2048, 768  # (matrices of 289 MB)
     st = synth_stack(GgmlDType.Q6_K, e, n_out, k, tensor_key(4700, 0, 1))
     raw = torch.zeros(st.nbytes + 2, dtype=torch.uint8, device="cuda")
     raw[2:] = st.buffer
@@ -315,12 +393,12 @@ def test_few_pairs_per_expert_alignment_rule(orc):
 
 @pytest.mark.parametrize("dt", ["Q4_K", "Q5_K", "Q6_K", "Q8_0"])
 def test_few_pairs_on_average_many_in_use(orc, dt):
-    """12 pairs per expert on average, but 400 on each of two experts: the grouped GEMM
+    """3 pairs per expert on average, but 400 on each of two experts: the grouped GEMM
     does the work after the other kernel left it, with the same bits as at an expert count
     whose average sends it there at once."""
     rng = np.random.default_rng(9)
-    t, top_k, n_out, k = 400, 2, 512, 768
-    st = synth_stack(GgmlDType[dt], 64, n_out, k, tensor_key(4800, 0, 1))
+    t, top_k, n_out, k = 400, 2, 2560, 768
+    st = synth_stack(GgmlDType[dt], 256, n_out, k, tensor_key(4800, 0, 1))
     few = ExpertStack(st.buffer, GgmlDType[dt], 3, n_out, k)
     ids = dev_u32(np.argsort(rng.random((t, 2)), axis=1))
     x = dev_f32(rng.standard_normal((t, 1, k)).astype(np.float32))

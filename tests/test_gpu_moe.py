@@ -140,8 +140,8 @@ def test_verify_block_no_shared(dev, orc):
 
 
 def test_prefill_grouped_gemm_small(dev, orc):
-    """C3 layer at t = 96 (16-pair MFMA tiles) and t = 240 (the grouped GEMM, past
-    the tiles' 2560 pairs) against the oracle."""
+    """C3 layer at t = 96 (16-pair MFMA tiles) and t = 240 (the matmuls for few pairs per
+    expert, past the tiles' 1280 pairs) against the oracle."""
     cfg = CONFIGS["C3"]
     layer = build_layer(cfg["spec"], seed=1003)
     for t in (96, 240):
@@ -308,7 +308,7 @@ def test_laguna_geometry(dev, orc):
     Q4_K groups per gate/up row and 4 Q6_K blocks per down row, so decode takes the
     generic slot kernels (not the ff = 1536 compile-time forms); t = 6 is a
     verify block on them, t = 16 and 64 run the MFMA verify tiles and t = 240
-    the grouped GEMM."""
+    the matmuls for few pairs per expert."""
     spec = LayerSpec(3072, 1024, 256, 10, GgmlDType.Q4_K, GgmlDType.Q6_K, shared=True, weights_scale=2.5)
     layer = build_layer(spec, seed=1051)
     for t in (1, 6, 16, 64, 240):

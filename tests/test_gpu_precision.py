@@ -107,8 +107,8 @@ def test_mv_id_wide_rows(dev, orc, dt, k):
 
 
 def test_workspace_reuse_across_t(dev, orc):
-    """One block's workspace serves calls of any t in any order: a grouped-GEMM
-    call (t = 240), MFMA verify tiles (t = 64) and then verify blocks on the
+    """One block's workspace serves calls of any t in any order: a grouped
+    call (t = 240, the matmuls for few pairs per expert), MFMA verify tiles (t = 64) and then verify blocks on the
     decode kernels (t = 12, 3) must each match the oracle."""
     spec = CONFIGS["C2"]["spec"]
     layer = build_layer(spec, seed=1102)
