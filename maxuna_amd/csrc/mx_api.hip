@@ -529,8 +529,9 @@ void plan_gst(const mx_moe_layer *L, int64_t t, Plan &p) {
 
 // Chooses the kernels of a forward; every shape limit of the chosen kernels is
 // checked here, so a validated call never fails after its first launch.
-// small_ws: of two plans the one with the smaller workspace (the no-alloc forward)
-Plan plan_for(const mx_moe_layer *L, int64_t t, bool small_ws = false) {
+// few_pairs: past kVmmGstPairs the matmuls for few pairs per expert where they fit,
+// else the tiles up to kVmmMaxPairs.
+Plan plan_of(const mx_moe_layer *L, int64_t t, bool few_pairs) {
     Plan p;
     p.min_seq = L->mm_min_seq > 0 ? L->mm_min_seq : kDefaultMmMinSeq;
     // < 0: never (LAGUNA_NO_MM_ID).  The MFMA GEMM needs K % 256 == 0 for every
@@ -558,7 +559,8 @@ Plan plan_for(const mx_moe_layer *L, int64_t t, bool small_ws = false) {
     // LAGUNA_NO_MM_ID (mm_min_seq < 0) keeps every t on the mat-vec kernels
     const bool vmm_ok =
         L->mm_min_seq >= 0 && decode_fits && t >= kVmmMinT && (!p.has_shared || p.shared_in_decode) &&
-        t * slots <= (p.gst_gu && p.gst_d && shapes && t >= p.min_seq && !small_ws ? kVmmGstPairs : kVmmMaxPairs) && L->gate.n_expert <= 1024 &&
+        t * slots <= (p.gst_gu && p.gst_d && shapes && t >= p.min_seq && few_pairs ? kVmmGstPairs : kVmmMaxPairs) &&
+        L->gate.n_expert <= 1024 &&
         vmm_supported(L->gate.dtype, L->down.dtype, (int)L->hidden, (int)L->expert_ff, gu_rb, d_rb) &&
         L->expert_ff * gu_rb < ((int64_t)1 << 31) && L->hidden * d_rb < ((int64_t)1 << 31) &&
         (!p.has_shared || (stack_row_bytes(L->shared_gate) == gu_rb && stack_row_bytes(L->shared_down) == d_rb));
@@ -657,6 +659,20 @@ Layout carve(const mx_moe_layer *L, int64_t t, const Plan &p, void *base) {
     return o;
 }
 
+// The plan of a call.  Where only the tiles' workspace (the bucket map and the padding are
+// what differs) fits the no-alloc forward's array, every forward takes the tiles, so that the
+// two forwards run the same kernels and the array holds what it held before the matmuls for
+// few pairs took over from 1280 pairs on.
+Plan plan_for(const mx_moe_layer *L, int64_t t) {
+    const Plan p = plan_of(L, t, true);
+    if (!p.mm || !p.gst_gu || !p.gst_d) return p;
+    const Plan tiles = plan_of(L, t, false);
+    return tiles.vmm && carve(L, t, p, nullptr).bytes > MX_NOALLOC_SCRATCH_BYTES &&
+                   carve(L, t, tiles, nullptr).bytes <= MX_NOALLOC_SCRATCH_BYTES
+               ? tiles
+               : p;
+}
+
 __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -743,7 +759,7 @@ struct Repeat {
 
 mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, const float *residual, float *out,
                            uint32_t *ids_out, float *w_out, void *workspace, size_t workspace_bytes,
-                           hipStream_t s, StageTimer *tm, Repeat rep = Repeat(), bool small_ws = false) {
+                           hipStream_t s, StageTimer *tm, Repeat rep = Repeat()) {
     StackGeom gg, gu, gd, sg{}, su{}, sd{};
     MX_TRY(check_layer(L, t, gg, gu, gd, sg, su, sd));
     if (t == 0) return MX_OK;
@@ -751,7 +767,7 @@ mx_status moe_forward_impl(const mx_moe_layer *L, const float *x, int64_t t, con
     MX_TRY(check_f32(out, "out"));
     if (residual) MX_TRY(check_f32(residual, "residual"));
     if (!workspace) return fail(MX_ERR_NULL, "moe: workspace is NULL");
-    const Plan p = plan_for(L, t, small_ws);
+    const Plan p = plan_for(L, t);
     const Layout o = carve(L, t, p, workspace);
     if (workspace_bytes < o.bytes)
         return fail(MX_ERR_SCRATCH, "moe: workspace of %zu bytes, need %zu", workspace_bytes, o.bytes);
@@ -1090,11 +1106,7 @@ mx_status mx_moe_forward_noalloc(const mx_moe_layer *L, const float *x, int64_t 
                                  uint32_t *ids_out, float *w_out, mx_stream_t stream) {
     StackGeom gg, gu, gd, sg{}, su{}, sd{};
     MX_TRY(check_layer(L, t, gg, gu, gd, sg, su, sd));
-    size_t need = mx_moe_workspace_bytes(L, t);
-    // (the verify tiles' workspace is the smaller one: they keep the sizes whose grouped
-    // path does not fit)
-    const bool small_ws = need > kNoAllocScratchBytes;
-    if (small_ws) need = carve(L, t, plan_for(L, t, true), nullptr).bytes;
+    const size_t need = mx_moe_workspace_bytes(L, t);
     if (need > kNoAllocScratchBytes)
         return fail(MX_ERR_SCRATCH,
                     "no-alloc forward: t = %lld needs %zu bytes of workspace, its scratch holds %zu "
@@ -1104,7 +1116,7 @@ mx_status mx_moe_forward_noalloc(const mx_moe_layer *L, const float *x, int64_t 
     void *ws = nullptr;
     MX_TRY(scratch_for_current_device(&ws));
     return moe_forward_impl(L, x, t, residual, out, ids_out, w_out, ws, kNoAllocScratchBytes, (hipStream_t)stream,
-                            nullptr, Repeat(), small_ws);
+                            nullptr);
 }
 
 uint64_t mx_tensor_key(uint64_t seed, uint32_t layer, uint32_t tensor_id) {

@@ -83,3 +83,21 @@ def test_noalloc_grouped_path_and_limit(dev):
         with pytest.raises(ops.MaxunaError) as ei:
             blk.forward_noalloc(x)
         assert ei.value.code == MX_ERR_SCRATCH, ei.value
+
+
+def test_noalloc_limit_is_the_workspace_limit(dev):
+    """A layer whose last token counts below 16 MiB are past the verify tiles' 1280 pairs
+    (hidden 1536, ff 512, 512 experts, top-4): at t = 379 (the matmuls for few pairs per
+    expert) and 380 (the largest t the array holds: the tiles) both forwards run the same
+    kernels, and 381 is rejected."""
+    spec = LayerSpec(1536, 512, 512, 4, GgmlDType.Q4_K, GgmlDType.Q6_K, shared=False)
+    blk = build_layer(spec, seed=1309).block
+    assert _largest_fitting_t(blk, lib().mx_moe_forward_noalloc_max_bytes()) == 380
+    for t in (379, 380):
+        x = dev_f32(make_x(spec, 950 + t, t))
+        want = host(blk.forward(x))
+        got = host(blk.forward_noalloc(x))
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"t={t}: out"
+    with pytest.raises(ops.MaxunaError) as ei:
+        blk.forward_noalloc(dev_f32(make_x(spec, 960, 381)))
+    assert ei.value.code == MX_ERR_SCRATCH, ei.value
