@@ -106,8 +106,7 @@ class MoeBlock:
         self.rms_eps = rms_eps
         self._ws = None
         self._c = self._layer_struct()
-        self._ref = C.byref(self._c)
-        self._need = {}  # workspace bytes by token count (a function of the struct)
+        self._need = (None, 0)  # the last (token count, struct) and its workspace bytes
 
     @property
     def hidden(self) -> int:
@@ -128,9 +127,12 @@ class MoeBlock:
             float(self.rms_eps), 0)
 
     def workspace(self, t: int, device) -> torch.Tensor:
-        need = self._need.get(t)
-        if need is None:
-            need = self._need[t] = lib().mx_moe_workspace_bytes(self._ref, t)
+        # a function of the struct's bytes and t: asked again when either differs
+        key = (t, bytes(self._c))
+        last, need = self._need
+        if key != last:
+            need = lib().mx_moe_workspace_bytes(C.byref(self._c), t)
+            self._need = (key, need)
         if self._ws is None or self._ws.numel() < need:
             # no state lives in the workspace between calls (every forward
             # initialises what it reads); zeroed only for tidiness
@@ -153,7 +155,7 @@ class MoeBlock:
             out = torch.empty_like(x)
         ids, w = self._routing(t, x.device) if return_routing else (None, None)
         ws = self.workspace(t, x.device)
-        check(lib().mx_moe_forward(self._ref, x.data_ptr(), t, ops._ptr(residual), out.data_ptr(), ops._ptr(ids),
+        check(lib().mx_moe_forward(C.byref(self._c), x.data_ptr(), t, ops._ptr(residual), out.data_ptr(), ops._ptr(ids),
                                    ops._ptr(w), ws.data_ptr(), ws.numel(), ops._stream()))
         return (out, ids, w) if return_routing else out
 
@@ -175,6 +177,6 @@ class MoeBlock:
         if out is None:
             out = torch.empty_like(x)
         ids, w = self._routing(t, x.device) if return_routing else (None, None)
-        check(lib().mx_moe_forward_noalloc(self._ref, x.data_ptr(), t, ops._ptr(residual), out.data_ptr(),
+        check(lib().mx_moe_forward_noalloc(C.byref(self._c), x.data_ptr(), t, ops._ptr(residual), out.data_ptr(),
                                            ops._ptr(ids), ops._ptr(w), ops._stream()))
         return (out, ids, w) if return_routing else out

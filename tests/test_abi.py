@@ -160,3 +160,28 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "nope.so")
     with pytest.raises(RuntimeError, match="no non-native fallback"):
         _lib.lib()
+
+
+def test_workspace_follows_the_layer_struct():
+    """The block's workspace is sized for the layer as it is at the call: a limit changed
+    after a first call (16 tokens from the verify tiles to the mat-vec kernels, whose workspace
+    is the larger) is not answered from the earlier one."""
+    import torch
+
+    from maxuna_amd.gguf import ExpertStack, GgmlDType
+    from maxuna_amd.moe import MoeBlock, MoeConfig
+
+    e, hidden, ff = 8, 512, 512
+
+    def stack(dt, n_out, k):
+        return ExpertStack(torch.zeros(e * n_out * k // 256 * dt.type_size, dtype=torch.uint8), dt, e, n_out, k)
+
+    block = MoeBlock(torch.zeros(e, hidden), torch.zeros(e), stack(GgmlDType.Q4_K, ff, hidden),
+                     stack(GgmlDType.Q4_K, ff, hidden), stack(GgmlDType.Q6_K, hidden, ff), MoeConfig(2))
+    sizes = []
+    for min_seq in (32, -1, 32):
+        block._c.mm_min_seq = min_seq
+        need = _lib.lib().mx_moe_workspace_bytes(C.byref(block._c), 16)
+        assert block.workspace(16, "cpu").numel() >= need
+        sizes.append(need)
+    assert sizes[1] > sizes[0] == sizes[2]
