@@ -309,12 +309,12 @@ template <> struct Q<kQ8_0> {
     }
 };
 
-// the sum over aligned groups of P lanes (a power of two >= 8), in every lane
+// the sum over aligned groups of P lanes (a power of two >= 4), in every lane
 template <int P> __device__ __forceinline__ float lane_sum(float v) {
     if constexpr (P >= 64) v += lane_partner<32>(v);
     if constexpr (P >= 32) v += lane_partner<16>(v);
     if constexpr (P >= 16) v += lane_partner<8>(v);
-    v += lane_partner<4>(v);
+    if constexpr (P >= 8) v += lane_partner<4>(v);
     v += lane_partner<2>(v);
     v += lane_partner<1>(v);
     return v;
@@ -409,11 +409,15 @@ template <int DT, int LPR, int AUX> struct RowWalk {
 // most rows per pass (fewer exchange steps per row).  Three groups a lane fill all
 // lanes at 48, 96 and 192 groups, where two or four leave a quarter of them idle
 // (mul_mv, us: Q4_K [100352 x 3072] 35.0 -> 31.4, Q5_K [16384 x 6144] 23.5 -> 19.8;
-// Q6_K [100352 x 6144] 131 -> 108 with the grid below), six at 384.
+// Q6_K [100352 x 6144] 131 -> 108 with the grid below), six at 384.  Rows of 256 values
+// fill 4 (8) lanes; on twice as many, half of them idle, mul_mv_id [2048 x 256] of Q6_K
+// took 16.3 us for 96 pairs (11.5 now, 13.1 in the form before the row walk), [3072 x 256]
+// of Q5_K for 192 pairs 32.5 (21.5, 28.7), layers of ff 256 up to 1.18 times as long.
 // f(integral_constant LPR, integral_constant NG)
 template <int DT, class F> static auto with_lanes(int G, F &&f) {
 #define MX_LN(L, N) return f(std::integral_constant<int, L>{}, std::integral_constant<int, N>{})
     if constexpr (DT == kQ4_K || DT == kQ5_K) {
+        if (G <= 4) MX_LN(4, 1);
         if (G <= 8) MX_LN(8, 1);
         if (G <= 16) MX_LN(16, 1);
         if (G <= 32) MX_LN(16, 2);
@@ -421,6 +425,7 @@ template <int DT, class F> static auto with_lanes(int G, F &&f) {
         if (G <= 64) MX_LN(32, 2);
         if (G <= 96) MX_LN(32, 3);
     } else {
+        if (G <= 8) MX_LN(8, 1);
         if (G <= 16) MX_LN(16, 1);
         if (G <= 24) MX_LN(8, 3);
         // (16 lanes of two: 113 registers, one workgroup of 11 slot waves per CU

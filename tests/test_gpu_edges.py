@@ -58,6 +58,7 @@ def test_decode_gate_up_row_widths(orc, dt, hidden):
 
 # k / ff: groups per row at the lane layouts' ends and just past them
 DOWN_ROWS = [
+    (GgmlDType.Q4_K, 256), (GgmlDType.Q5_K, 256), (GgmlDType.Q6_K, 256), (GgmlDType.Q8_0, 256), (GgmlDType.Q8_0, 288),
     (GgmlDType.Q4_K, 512), (GgmlDType.Q4_K, 768), (GgmlDType.Q4_K, 1280), (GgmlDType.Q4_K, 2304),
     (GgmlDType.Q4_K, 4352), (GgmlDType.Q4_K, 8448), (GgmlDType.Q5_K, 1024), (GgmlDType.Q5_K, 2048),
     (GgmlDType.Q5_K, 4096), (GgmlDType.Q6_K, 512), (GgmlDType.Q6_K, 768), (GgmlDType.Q6_K, 1024),
