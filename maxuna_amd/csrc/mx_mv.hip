@@ -888,17 +888,27 @@ static_assert(64 * WAVES == SEL_THREADS, "the in-block top-k needs SEL_THREADS t
 // 159 us; Q5_K hidden 5120 at t = 4: 177 -> 150 us.
 // What bounds it: the copies' latency and the VALU work of the dots (about 200
 // instructions per 64 groups of a row, the third digit plane among them).
-template <int DT, int NG> constexpr int gu_wpe() {
+// Rows whose words, all at once next to the activations, would take a wave per SIMD (or the
+// only second one): contracted group by group, the next copy behind the row's last read.
+// Layers, us, all words at once / group by group (and the form before the row passes): Q6_K
+// hidden 7168, ff 768, 2 slots at t = 8 96 / 65 (70), hidden 8192, ff 1024, top-6 at t = 2
+// 103 / 75 (76); Q5_K hidden 9216, ff 768 at t = 2 90 / 68 (68), hidden 7168, ff 768, top-3
+// at t = 4 62 / 55 (55).  Up to 96 groups (32 lanes)
+// the words fit and the copies overlap the dots.
+template <int DT, int NG, int LPR> constexpr bool gu_group_by_group() {
+    return LPR == 64 && (DT == kQ5_K ? NG >= 2 : DT == kQ6_K ? NG >= 3 : DT != kQ8_0 && NG >= 4);
+}
+template <int DT, int NG, int LPR> constexpr int gu_wpe() {
     // waves per SIMD the registers allow without spilling (the three digit planes
     // of a group are 48 VGPRs for Q4_K / Q5_K, 24 for the others)
     if (NG == 1) return DT == kQ5_K ? 4 : MX_GU_WPE;
-    if (DT == kQ4_K) return NG == 2 ? 3 : NG == 3 ? 2 : 1;
-    if (DT == kQ5_K) return NG == 2 ? 2 : 1;
-    if (DT == kQ6_K) return NG == 2 ? 3 : NG == 3 ? 2 : 1;
+    if (DT == kQ4_K) return NG == 2 ? 3 : 2;
+    if (DT == kQ5_K) return NG == 2 ? 3 : 2;
+    if (DT == kQ6_K) return NG <= (LPR == 64 ? 4 : 2) ? 3 : 2;
     return NG == 2 ? 4 : NG == 3 ? 3 : 2;
 }
 template <int DT, int NG, int LPR, int AUX>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(gu_wpe<DT, NG>())))
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(gu_wpe<DT, NG, LPR>())))
 k_decode_gate_up(DecodeGateUpArgs a, int slot0, int nr, int area) {
     constexpr int PP = LPR == 64 ? 1 : 32 / LPR;   // row pairs per pass
     constexpr int NMP = LPR == 64 ? 2 : 1;         // rows a lane contracts per pass
@@ -974,23 +984,35 @@ k_decode_gate_up(DecodeGateUpArgs a, int slot0, int nr, int area) {
             const uint8_t *wm = mat ? w[1] : w[0];
             const int off = (int)(reinterpret_cast<uintptr_t>(wm + (int64_t)p0 * rb) & 15);
             const uint8_t *rl = buf + mat * area + off + pair * (int)rb;
-            typename Q<DT>::Raw raw[NG];
-#pragma unroll
-            for (int jg = 0; jg < NG; jg++) {
-                const int g = sub + LPR * jg;
-                raw[jg] = Q<DT>::load(rl, g < G ? g : 0);
-            }
-            wait_lgkmcnt0();  // the words are in registers: their bytes may be overwritten
-            if (more) {
-                issue(NMP == 2 ? m : 0, i + 1);
-                if (NMP == 1) issue(1, i + 1);
-            }
+            auto next = [&] {
+                wait_lgkmcnt0();  // the words are in registers: their bytes may be overwritten
+                if (more) {
+                    issue(NMP == 2 ? m : 0, i + 1);
+                    if (NMP == 1) issue(1, i + 1);
+                }
+            };
             v[m] = 0.f;
+            if constexpr (gu_group_by_group<DT, NG, LPR>()) {
 #pragma unroll
-            for (int jg = 0; jg < NG; jg++) {
-                const int g = sub + LPR * jg;
-                const float d = Q<DT>::dot(raw[jg], g, xs[jg]);
-                v[m] += g < G ? d : 0.f;
+                for (int jg = 0; jg < NG; jg++) {
+                    const int g = sub + LPR * jg;
+                    if (g < G) v[m] += Q<DT>::dot(Q<DT>::load(rl, g), g, xs[jg]);
+                }
+                next();
+            } else {
+                typename Q<DT>::Raw raw[NG];
+#pragma unroll
+                for (int jg = 0; jg < NG; jg++) {
+                    const int g = sub + LPR * jg;
+                    raw[jg] = Q<DT>::load(rl, g < G ? g : 0);
+                }
+                next();
+#pragma unroll
+                for (int jg = 0; jg < NG; jg++) {
+                    const int g = sub + LPR * jg;
+                    const float d = Q<DT>::dot(raw[jg], g, xs[jg]);
+                    v[m] += g < G ? d : 0.f;
+                }
             }
         }
         // the rows' sums over their lanes; a pair's gate sum ends in the lower half of

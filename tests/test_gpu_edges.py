@@ -56,6 +56,15 @@ def test_decode_gate_up_row_widths(orc, dt, hidden):
         layer_against_oracle(orc, spec, t, 4200 + t, F32_CLASS)
 
 
+@pytest.mark.parametrize("dt,hidden", [GU_ROWS[i] for i in (6, 10, 13, 14, 15)], ids=lambda v: str(getattr(v, "name", v)))
+def test_decode_gate_up_wide_rows_passes(orc, dt, hidden):
+    """Rows contracted group by group, four and eight passes a wave: each row's copy follows
+    the last read of the row before it in the same buffer."""
+    for t, ff in ((1, 4160), (3, 2112)):
+        spec = LayerSpec(hidden, ff, 12, 3, dt, GgmlDType.Q8_0, shared=True)
+        layer_against_oracle(orc, spec, t, 4220 + t, F32_CLASS)
+
+
 # k / ff: groups per row at the lane layouts' ends and just past them
 DOWN_ROWS = [
     (GgmlDType.Q4_K, 256), (GgmlDType.Q5_K, 256), (GgmlDType.Q6_K, 256), (GgmlDType.Q8_0, 256), (GgmlDType.Q8_0, 288),
