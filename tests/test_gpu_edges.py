@@ -67,7 +67,6 @@ def test_decode_gate_up_wide_rows_passes(orc, dt, hidden):
 
 # k / ff: groups per row at the lane layouts' ends and just past them
 DOWN_ROWS = [
-    (GgmlDType.Q4_K, 256), (GgmlDType.Q5_K, 256), (GgmlDType.Q6_K, 256), (GgmlDType.Q8_0, 256), (GgmlDType.Q8_0, 288),
     (GgmlDType.Q4_K, 512), (GgmlDType.Q4_K, 768), (GgmlDType.Q4_K, 1280), (GgmlDType.Q4_K, 2304),
     (GgmlDType.Q4_K, 4352), (GgmlDType.Q4_K, 8448), (GgmlDType.Q5_K, 1024), (GgmlDType.Q5_K, 2048),
     (GgmlDType.Q5_K, 4096), (GgmlDType.Q6_K, 512), (GgmlDType.Q6_K, 768), (GgmlDType.Q6_K, 1024),
@@ -192,6 +191,38 @@ def test_f32_down_rows_keep_the_layer_in_f32(orc, dt, ff):
     spec = LayerSpec(512, ff, 8, 2, GgmlDType.Q4_K, dt, shared=False)
     for t in (1, 5, 20):
         layer_against_oracle(orc, spec, t, 4470 + t, F32_CLASS)
+
+
+SHORT_ROWS = [(GgmlDType.Q4_K, 256), (GgmlDType.Q5_K, 256), (GgmlDType.Q6_K, 256), (GgmlDType.Q8_0, 256), (GgmlDType.Q8_0, 288)]
+
+
+@pytest.mark.parametrize("dt,ff", SHORT_ROWS, ids=lambda v: str(getattr(v, "name", v)))
+def test_decode_down_short_rows(orc, dt, ff):
+    for t in (1, 2, 3, 7):
+        spec = LayerSpec(288, ff, 12, 3, GgmlDType.Q8_0, dt, shared=True)
+        layer_against_oracle(orc, spec, t, 4340 + t, F32_CLASS)
+
+
+@pytest.mark.parametrize("dt,k", SHORT_ROWS, ids=lambda v: str(getattr(v, "name", v)))
+def test_mul_mv_id_short_rows(orc, dt, k):
+    """Few to many batches a wave, row counts that no batch divides.  Bound per output (a short
+    dot may cancel to nothing): the activation grid's 2^-23 (1 + 2^-8) of a scale group's largest
+    value on every weight of it, and two f32 roundings of the sum of magnitudes."""
+    rng = np.random.default_rng(k)
+    e, top_k, group = 3, 2, 128 if k % 128 == 0 else 32
+    for n_out, t in ((1, 1), (5, 2), (333, 9), (2049, 40)):
+        st = synth_stack(dt, e, n_out, k, tensor_key(4480, 0, n_out))
+        w = orc.dequantize(int(dt), host(st.buffer), e * n_out * k).reshape(e, n_out, k).astype(np.float64)
+        x = rng.standard_normal((t, 1, k)).astype(np.float32)
+        ids = np.stack([rng.permutation(e)[:top_k] for _ in range(t)])
+        got = host(ops.mul_mv_id(st, dev_f32(x), dev_u32(ids)))
+        xd, aw = x[:, 0].astype(np.float64), np.abs(w)
+        top = np.repeat(np.abs(xd).reshape(t, -1, group).max(-1), group, axis=1)
+        pick = lambda y: y.reshape(t, e, n_out)[np.arange(t)[:, None], ids]  # noqa: E731
+        err = np.abs(got - pick(xd @ w.reshape(-1, k).T))
+        bound = pick((2.0**-23 * (1 + 2.0**-8) * top + 2.0**-23 * np.abs(xd)) @ aw.reshape(-1, k).T)
+        print(f"{dt.name} [{n_out} x {k}] t={t}: {np.max(err / bound):.3f} of the bound", flush=True)
+        assert np.all(err <= bound)
 
 
 def _mul_mv_errors(orc, dt, n_out, k, x, off=0):
