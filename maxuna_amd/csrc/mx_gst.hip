@@ -85,6 +85,15 @@ __host__ __device__ constexpr int gs_ratio(int dtype, bool swiglu) {
     return dtype == kQ6_K ? (swiglu ? 22 : 18) : dtype == kQ4_K ? 16 : swiglu ? 15 : 13;
 }
 
+// Gate/up of the cheaply unpacked types are taken below 40 * fill - 14 pairs per m-tile, fill:
+// the share of the CU's waves and super-blocks that K fills (9 at K = 1792, 26 where all are).
+// A stage costs a run the same whatever its pairs, and few waves make every stage slower,
+// while the GEMM gains with the pairs.  Layers, time here over the GEMM's (or the tiles'),
+// even routers, at 8 / 16 / 24 pairs per expert: Q4_K K = 1536 0.91 / 0.98 / 1.02, 1792 0.99 /
+// 1.06 / 1.13, 2048 at 16 / 24 1.04 / 1.10, 3072 0.96 / 0.88 / 0.97; Q5_K 1792 0.97 / 1.05 / 1.07,
+// 3584 1.00 / 1.03 / 1.08; Q6_K 1792 0.85 / 0.86 / 0.94 (no line).
+__host__ __device__ constexpr bool gs_by_fill(int dtype, bool swiglu) { return swiglu && dtype != kQ6_K; }
+
 template <int DT, bool SWIGLU, int MT, int NSB, int WM> struct GsGeo {
     static constexpr int CPR = GsBlk<DT>::CPR, BLK = GsBlk<DT>::BLK, SLOT = 16 * CPR;
     static constexpr int POS = 16 * CPR, NI = (POS + 63) / 64, STAGE = POS * 16;
@@ -155,7 +164,9 @@ k_gst(GemmArgs a, int W) {
         // many runs for their m-tiles: the grouped GEMM is the faster (block-uniform; nothing
         // else is done before this: a launch left behind costs 2 to 2.5 us)
         runs = both & 0xFFFF;
-        const bool mine = 10 * runs < gs_ratio(DT, SWIGLU) * (both >> 16);
+        const int mtiles = both >> 16, fill = 40 * (a.k / 256) * teams / (G::WAVES * NSB) - 14;
+        const bool mine = 10 * runs < gs_ratio(DT, SWIGLU) * mtiles &&
+                          (!gs_by_fill(DT, SWIGLU) || a.t * a.top_k < fill * mtiles);
         if (blockIdx.x == 0 && tid == 0) *a.done = mine;
         if (!mine) return;
         for (int e = e0; e < e1; e++) {

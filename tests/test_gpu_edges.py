@@ -417,6 +417,25 @@ def test_few_pairs_per_expert(gate, down, hidden, ff):
     assert_close(host(out), host(want), what=f"{gate}/{down} {hidden}x{ff} E{e} t{t}")
 
 
+@pytest.mark.parametrize("gate,hidden", [("Q4_K", 1792), ("Q5_K", 2304), ("Q8_0", 1792)])
+def test_few_pairs_gate_up_line(gate, hidden):
+    """Gate/up whose K fills part of a CU's waves: taken at 4 pairs per expert, left to the
+    grouped GEMM at 30 (read back from the word it writes); both against 64 bits."""
+    ff, top_k = 512, 4
+    gdt = GgmlDType[gate]
+    e = -(-(264 << 20) // (2 * ff * (hidden // gdt.block_size * gdt.type_size)))
+    spec = LayerSpec(hidden, ff, e, top_k, gdt, gdt, shared=False, bias_sigma=0.0)
+    layer = build_layer(spec, seed=4900)
+    for per, taken in ((4, 1), (30, 0)):
+        t = per * e // top_k
+        x = torch.from_numpy(make_x(spec, 4901, t)).cuda()
+        at, _ = few_pairs_words(layer.block, t)
+        assert at >= 0
+        out, ids, w = layer.block.forward(x, return_routing=True)
+        assert int(layer.block._ws[at:at + 4].cpu().view(torch.int32)) == taken
+        assert_close(host(out), host(moe_f64(layer.block, x, ids, w)), what=f"{gate} {hidden} t{t}")
+
+
 def test_few_pairs_per_expert_alignment_rule(orc):
     """Q6_K stacks two bytes off 16-byte alignment take the other grouped kernel: same
     outputs to f16-operand rounding."""
