@@ -1602,7 +1602,7 @@ __global__ void __launch_bounds__(64 * DN_SLOTS_MAX) k_decode_down_q6r(DecodeDow
     a.out[o] = vv;
 }
 
-// Verify-block form of the compile-time Q6_K down rows (t > 2, the grid of
+// Verify-block form of the compile-time Q6_K down rows (t > 2 past two rounds of tiles, the grid of
 // k_decode_down: one workgroup per (row tile, slot, token), DQ6V_RPW rows per
 // wave, the pair's act row staged once per workgroup): the field offsets of
 // k_decode_down_q6r, hoisted out of the row loop, and its two-buffer ring of
@@ -1747,12 +1747,27 @@ template <int DT> static bool dn_slots_fit(const DecodeDownArgs &a) {
     // smaller ones of k_decode_down keep the CUs fuller (layers, us, this kernel / that one:
     // Q5_K hidden 5120, ff 1536 at t = 1 (320 tiles) 52.7 / 43.5; Q6_K hidden 6144, ff 2816 at
     // t = 1 (384) 68 / 50; hidden 7168 at t = 2 109 / 100; Q4_K hidden 1024 at t = 4 (256)
-    // 20.2 / 21.9, hidden 2048, ff 768 at t = 2 (256) 27.3 / 29.8, at t = 4 (512) 35 / 39)
+    // 20.2 / 21.9, hidden 2048, ff 768 at t = 2 (256) 27.3 / 29.8, at t = 4 (512) 35 / 39).
+    // Up to four slots of short rows (two batches a wave) and four tokens a CU holds several
+    // workgroups, and rounds are counted by those (Q6_K hidden 6144, ff 768, 4 slots at t = 2 36.5
+    // / 39.3, Q8_0 hidden 6144, ff 768, 2 slots at t = 3 28.9 / 33.1; rows of more batches the
+    // other way: Q6_K hidden 2560, ff 2304, 2 slots at t = 3 42.2 / 39.5).
     const int64_t n = (int64_t)((a.hidden + RW_DN - 1) / RW_DN) * a.t, cus = device_cus();
-    if (DT == kQ6_K && dn_q6_ok(a) ? a.t > 2 : n > cus && (n > 2 * cus || 20 * n < 39 * cus)) return false;
+    const int slots = a.top_k + (a.sh_down ? 1 : 0);
+    // Q6_K rows of ff 1536: up to two tokens, and past them two rounds of tiles; the few
+    // workgroups of 256 rows of k_decode_down_q6v take longer there, and less time beyond
+    // (layers, us, k_decode_down_q6r / q6v: hidden 2048 at t = 3 (384 tiles) 1 slot 27.1 / 33.8,
+    // 4 slots 34.4 / 40.6, 8 slots 46.0 / 46.6; hidden 4096 at t = 4 (1024) 56.9 / 49.8 at 4 slots,
+    // 83.4 / 78.6 at 8; hidden 3072 at t = 3 (576) 58.1 / 50.3 at 6).
+    if (DT == kQ6_K && dn_q6_ok(a) && a.t > 2 && n > 2 * cus) return false;
     return with_lanes<DT>(groups<DT>(a.ff), [&](auto lpr, auto ng) {
+        const DnSlots d(a, 64 / decltype(lpr)::value);
+        int64_t most = cus;
+        if (slots <= 4 && a.t <= 4 && 2 * d.br >= d.rows)
+            most *= std::min<int64_t>(DN_SLOTS_MAX / slots, 160 * 1024 / d.lds);
+        if (!(DT == kQ6_K && dn_q6_ok(a)) && n > most && (n > 2 * most || 20 * n < 39 * most)) return false;
         return decltype(ng)::value <= dn_slots_max_ng<DT>() &&
-               DnSlots(a, 64 / decltype(lpr)::value).lds <= 160 * 1024 - sizeof(float) * DN_SLOTS_MAX * RW_DN;
+               d.lds <= 160 * 1024 - sizeof(float) * DN_SLOTS_MAX * RW_DN;
     });
 }
 template <int DT>

@@ -133,12 +133,15 @@ def test_decode_down_rows_of_three(orc, dt, ff):
         layer_against_oracle(orc, spec, t, 4310 + t, F32_CLASS)
 
 
-@pytest.mark.parametrize("hidden,ts", [(1024, (3, 4, 5)), (2048, (2, 3, 4)), (5120, (1, 2))])
-def test_decode_down_slots_line(orc, hidden, ts):
-    """Both sides of the slot-per-wave down kernel's line: up to 256 tiles of 16 rows, a
-    partly filled second round, two full rounds."""
+@pytest.mark.parametrize("hidden,ff,top_k,ts", [
+    (1024, 512, 3, (3, 4, 5)), (2048, 512, 3, (2, 3, 4)), (5120, 512, 3, (1, 2)), (8192, 512, 3, (1, 2)),
+    (4128, 256, 1, (3, 4)), (5120, 512, 5, (1, 2)), (2048, 512, 11, (1, 2, 3, 4)), (1024, 1536, 3, (3, 4, 5))])
+def test_decode_down_slots_line(orc, hidden, ff, top_k, ts):
+    """Both sides of the slot-per-wave down kernel's lines: one round of its tiles of 16 rows,
+    a partly filled second round, two full rounds; few slots (several workgroups per CU), many,
+    and Q6_K rows of 1536."""
     for t in ts:
-        spec = LayerSpec(hidden, 512, 12, 3, GgmlDType.Q8_0, GgmlDType.Q6_K, shared=True)
+        spec = LayerSpec(hidden, ff, 12, top_k, GgmlDType.Q8_0, GgmlDType.Q6_K, shared=top_k < 11)
         layer_against_oracle(orc, spec, t, 4320 + t, F32_CLASS)
 
 
