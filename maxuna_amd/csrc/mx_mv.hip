@@ -893,10 +893,10 @@ static_assert(64 * WAVES == SEL_THREADS, "the in-block top-k needs SEL_THREADS t
 // Layers, us, all words at once / group by group (and the form before the row passes): Q6_K
 // hidden 7168, ff 768, 2 slots at t = 8 96 / 65 (70), hidden 8192, ff 1024, top-6 at t = 2
 // 103 / 75 (76); Q5_K hidden 9216, ff 768 at t = 2 90 / 68 (68), hidden 7168, ff 768, top-3
-// at t = 4 62 / 55 (55).  Up to 96 groups (32 lanes)
-// the words fit and the copies overlap the dots.
+// at t = 4 62 / 55 (55); Q6_K of 65 to 96 groups (hidden 2304 to 3072, 32 lanes of three) over
+// 220 layers 0.94 times the time.  Q5_K and Q4_K on 32 lanes gain no wave by it.
 template <int DT, int NG, int LPR> constexpr bool gu_group_by_group() {
-    return LPR == 64 && (DT == kQ5_K ? NG >= 2 : DT == kQ6_K ? NG >= 3 : DT != kQ8_0 && NG >= 4);
+    return (LPR == 64 || DT == kQ6_K) && (DT == kQ5_K ? NG >= 2 : DT == kQ6_K ? NG >= 3 : DT != kQ8_0 && NG >= 4);
 }
 template <int DT, int NG, int LPR> constexpr int gu_wpe() {
     // waves per SIMD the registers allow without spilling (the three digit planes
@@ -904,7 +904,7 @@ template <int DT, int NG, int LPR> constexpr int gu_wpe() {
     if (NG == 1) return DT == kQ5_K ? 4 : MX_GU_WPE;
     if (DT == kQ4_K) return NG == 2 ? 3 : 2;
     if (DT == kQ5_K) return NG == 2 ? 3 : 2;
-    if (DT == kQ6_K) return NG <= (LPR == 64 ? 4 : 2) ? 3 : 2;
+    if (DT == kQ6_K) return NG <= 4 ? 3 : 2;
     return NG == 2 ? 4 : NG == 3 ? 3 : 2;
 }
 template <int DT, int NG, int LPR, int AUX>
