@@ -392,8 +392,8 @@ def bench_lm_head(args):
 def t_sweep(ts, replays=20):
     """C1-shaped layers (C2's routing spread) at other block sizes: 4 distinct
     layers replayed as one graph per t, µs per layer forward.  Which kernels run
-    depends on t: the 16-pair MFMA tiles up to 2560 (token, slot) pairs, the
-    grouped GEMM beyond."""
+    depends on t: the 16-pair MFMA tiles up to 1280 (token, slot) pairs, the matmuls
+    for few pairs per expert or the grouped GEMM beyond."""
     import torch
     from maxuna_amd.synth import CONFIGS, build_layer, make_x
 
@@ -405,7 +405,7 @@ def t_sweep(ts, replays=20):
         ys = [torch.empty_like(x) for x in xs]
         us = graph_us(lambda: [layers[i].block.forward(xs[i], out=ys[i]) for i in range(4)], replays) / 4
         slots = spec.top_k + 1
-        path = "tiles" if t >= 16 and t * slots <= 2560 else ("grouped GEMM" if t >= 32 else "decode")
+        path = "tiles" if t >= 16 and t * slots <= 1280 else ("grouped" if t >= 32 else "decode")
         log(f"t-sweep t={t}: {us:.1f} us/layer ({path})")
         out[t] = round(us, 1)
     return out

@@ -29,8 +29,9 @@
 //  * SwiGLU: a tile is 16 gate rows, then the same 16 up rows; the thread that
 //    sums a gate value keeps it until its up value is summed.
 //
-// Bound by instruction issue: about 180 (Q4_K) to 260 (Q6_K) VALU per wave and stage
-// of 16 x 256 weights, once per run of 32 pairs.  top-10 of 256 experts, hidden 4096,
+// Bound by instruction issue and the waits between: about 170 (Q4_K) to 250 (Q6_K) VALU per
+// wave and stage of 16 x 256 weights, once per run of 32 pairs; VALU and MFMA instructions
+// execute in 64 to 70% of the SIMD cycles.  top-10 of 256 experts, hidden 4096,
 // ff 1536, Q4_K / Q6_K, grouped GEMM against these (gate, up and down with the
 // passes between them): t = 300 1180 / 892 us, 512 1267 / 1078, 700 1410 / 1300,
 // 1000 1548 / 1590.  Weight bytes fetched for the gate projection at t = 512: 1.46 ->
