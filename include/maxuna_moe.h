@@ -153,7 +153,7 @@ mx_status mx_prepare_map0(int64_t n_expert, const uint32_t *ids, int64_t t, int6
  * 32) the projection runs the 16-pair MFMA tiles of the MoE forward's verify
  * blocks; beyond that, when K is a multiple of 256, the MFMA matmuls of the
  * prefill path (for few pairs per expert, or the grouped GEMM; the tiles go on to
- * 2560 pairs where the former do not take the stack: matrices of less than 256 MB
+ * 2560 pairs where the former do not take the stack: most matrices of less than 256 MB
  * in all among others); all over x rounded to f16 (one power-of-two scale per x row).  Their
  * temporaries (the f16 rows, t * x_per_row * (2k + 4) bytes, and the tiles'
  * pair order) are stream-ordered memory from a library pool per device, which

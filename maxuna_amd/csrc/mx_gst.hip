@@ -446,8 +446,15 @@ bool gst_fits(int dtype, const GemmArgs &a, bool swiglu) {
     // GEMM's repeated reads are cheap, and the launch left behind under a skewed router is a
     // larger share of the layer (layers, us, the GEMM alone / here: hidden 1024, ff 512, 64
     // experts Q5_K 62 / 71; hidden 2048, ff 768, 128 experts Q4_K / Q6_K at 200 tokens, even
-    // router 206 / 180, skewed 115 / 122).
-    ok = ok && (int64_t)a.n_map_expert * a.n_out * a.row_bytes * (swiglu ? 2 : 1) >= (int64_t)256 << 20;
+    // router 206 / 180, skewed 115 / 122).  Smaller ones where the GEMM has too little to run
+    // on, up to 12 pairs per expert and half a workgroup per CU (60 random layers 0.90 of its
+    // time, 7 more than 4% slower), and Q6_K gate/up, which the GEMM unpacks slowest (73 layers
+    // 0.90, 2 slower; hidden 3584, ff 256, 16 experts at 40 tokens 110 / 60).
+    const int64_t bytes = (int64_t)a.n_map_expert * a.n_out * a.row_bytes * (swiglu ? 2 : 1);
+    const int rows = swiglu ? 2 * a.n_out : a.n_out, wg = !swiglu && (dtype == kQ6_K || dtype == kQ8_0) ? 256 : 512;
+    const bool idle = 2 * (int64_t)a.n_map_expert * ((rows + wg - 1) / wg) <= device_cus() &&
+                      (int64_t)a.t * a.top_k < 12 * (int64_t)a.n_map_expert;
+    ok = ok && (bytes >= (int64_t)256 << 20 || idle || (swiglu && dtype == kQ6_K));
     // Less than one run per expert on average: beyond, even an evenly used map has two runs
     // per m-tile, which no gs_ratio takes where runs are of 16 pairs and few do at 32; what it
     // takes gained 1.08 (27 pairs) to 1.3x (12 pairs).

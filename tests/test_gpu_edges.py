@@ -329,13 +329,16 @@ SMALL_GROUPED = [
 
 @pytest.mark.parametrize("gate,down,hidden,ff", SMALL_GROUPED)
 def test_few_pairs_small_matrices(orc, gate, down, hidden, ff):
-    """Layers of a few pairs per expert, skewed, past the verify tiles, whose matrices are too
-    small for the matmuls of few pairs: the grouped GEMM, against the oracle's own routing.
-    f16 operands: the contract's bound."""
+    """Layers of a few pairs per expert, skewed, past the verify tiles, whose matrices are
+    small: the grouped GEMM, or the matmuls of few pairs for Q6_K gate/up and where the GEMM
+    would have few workgroups, against the oracle's own routing.  f16 operands: the contract's
+    bound."""
     spec = LayerSpec(hidden, ff, 40, 4, GgmlDType[gate], GgmlDType[down], shared=hidden % 512 == 0, bias_sigma=0.3)
     layer = build_layer(spec, seed=4600)
     t = 50 if hidden > 4096 else 210 if gate == "Q4_K" else 70
-    assert few_pairs_words(layer.block, t) == (-1, -1)
+    tried = [w >= 0 for w in few_pairs_words(layer.block, t)]
+    assert tried[0] or gate != "Q6_K"
+    assert not any(tried) or gate == "Q6_K" or 12 * 40 > 4 * t
     x = make_x(spec, 4601, t)
     out, ids, w = layer.block.forward(torch.from_numpy(x).cuda(), return_routing=True)
     out, ids, w = host(out), host(ids), host(w)
